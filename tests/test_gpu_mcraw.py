@@ -76,3 +76,38 @@ def test_decode_equals_oracle_and_the_coded_frame(hip, owd, oht, ox, oy, single,
     ref = mc.oracle_decode(bits, off, refs, data, ox, oy, owd, oht, wd, ht)
     assert np.array_equal(out_gpu, ref)
     assert np.array_equal(out_gpu, mc.unorm_store(coded[oy:oy + ht, ox:ox + wd]))
+
+
+@pytest.mark.parametrize("owd,oht,dshift,cut", [(192, 4, 0, 0), (320, 4, 0, 0), (192, 12, 4, 0), (320, 8, 1, 0), (320, 8, 0, 60)],
+                         ids=["12-blocks", "20-blocks", "data-4-off", "data-1-off", "data-cut"])
+def test_decode_partial_waves_and_unaligned_data(hip, owd, oht, dshift, cut):
+    """block counts that leave a wave partly empty, data off the 8-byte
+    alignment, and data that ends inside a block (zeros past its end): equal
+    to the oracle on the bytes there are"""
+    rng = np.random.default_rng(owd * oht + dshift + cut)
+    nb = owd * oht // 64
+    cnt = rng.integers(0, 16, size=-(-nb // 64) * 64).astype(np.uint8)
+    cnt[nb:] = 0
+    bits = (cnt[0::2] | (cnt[1::2] << 4)).astype(np.uint8)
+    refs = rng.integers(0, 65536, size=cnt.size).astype(np.uint16)
+    off = mc.oracle_prefix(bits, nb)
+    data = rng.integers(0, 256, size=int(off[-1]), dtype=np.uint8)
+    n = data.size - cut
+    padded = np.concatenate([data[:n], np.zeros(cut, np.uint8)])
+    bufs = [hip.DeviceBuffer(w, 1, 1, f) for w, f in ((bits.size, H.FMT_UI8), (refs.size, H.FMT_UI16), (dshift + n, H.FMT_UI8),
+                                                      (cnt.size, H.FMT_UI32), (16, H.FMT_UI32))]
+    out = hip.DeviceBuffer(owd, oht, 1, H.FMT_UI16)
+    try:
+        for b, a in zip(bufs, (bits, refs, np.concatenate([np.zeros(dshift, np.uint8), data[:n]]))):
+            b.upload(a)
+        b_bits, b_ref, b_dat, b_off, b_scr = bufs
+        dat = H.Buf(b_dat.ptr + dshift, n, 1, n, 1, H.FMT_UI8, 1, n)
+        hip.launch("i-mcraw", "prefix", None, None, [b_bits, b_off, b_scr], (nb + 511) // 512 * 8, 1)
+        hip.launch("i-mcraw", "decode", np.array([0, 0, owd, oht], np.int32), None, [out, b_bits, b_off, b_ref, dat], nb * 8, 1)
+        hip.sync()
+        assert np.array_equal(b_off.download()[0][:nb], off)
+        ref = mc.oracle_decode(bits, off, refs, padded, 0, 0, owd, oht, owd, oht)
+        assert np.array_equal(out.download(), ref)
+    finally:
+        for b in bufs + [out]:
+            b.free()
