@@ -93,6 +93,23 @@ def test_pitch(hip):
     assert gpu_jpg(hip, img, 95, 1, 1, pad=37) == oracle_jpg(img, 95, 1, 1)
 
 
+# extents round the 32-MCU strips, the last MCU and the 256-block groups; one
+# strip and many; noise at quality 100 (groups larger than their LDS words)
+EDGES = [(1, 1, 95, 1, 1, None), (8, 8, 85, 2, 2, None), (255, 9, 95, 1, 1, None), (256, 8, 95, 1, 1, 1), (257, 24, 97, 1, 1, 2),
+         (511, 17, 91, 2, 1, None), (513, 16, 92, 2, 1, 2), (512, 33, 85, 2, 2, 1), (529, 31, 60, 2, 2, None),
+         (1033, 40, 100, 2, 2, 2), (264, 8800, 90, 1, 1, None)]
+
+
+@pytest.mark.parametrize("W,Hh,q,hs,vs,dct", EDGES)
+def test_strip_and_group_edges(hip, W, Hh, q, hs, vs, dct):
+    rng = np.random.default_rng(W * 31 + Hh)
+    x = np.arange(W)[None, :, None] * np.array([1, 2, 3]) + np.arange(Hh)[:, None, None] * np.array([3, 1, 2])
+    img = np.clip(128 + 90 * np.sin(x / 17.0) + rng.normal(0, 60 if q == 100 else 4, (Hh, W, 3)), 0, 255).astype(np.uint8)
+    print(f"[gpu_jpg] {W}x{Hh} q{q} {hs}x{vs} dct {dct}", flush=True)
+    ex = {} if dct is None else dict(dct=dct)
+    assert gpu_jpg(hip, img, q, hs, vs, **ex) == oracle_jpg(img, q, hs, vs, dct or 0, 0)
+
+
 def test_24mp_timing(hip):
     rng = np.random.default_rng(5)
     W, Hh = 6000, 4000

@@ -3,19 +3,21 @@
 // optimised Huffman coding).  The steps are libjpeg's published ones (ITU-T
 // T.81 baseline with IJG's choices), so the file's tables and entropy-coded
 // data are those libjpeg writes for the same image and settings:
-//   k_jpg_coef    one lane per 8x8 block in MCU order: fixed-point YCbCr,
-//                 2:1 chroma boxes with the alternating bias (or libjpeg's
-//                 smoothing filter), samples past the edges replicated,
-//                 the islow, ifast or float DCT and its quantisation, all
-//                 in registers; stored zigzag ordered, so the passes below
-//                 load a block in 8 vectors
-//   k_jpg_dummy   blocks of the last MCUs past a component's own extent:
-//                 zero, with the DC of the block to the left / above
-//   k_jpg_stats   symbol counts of the four tables (LDS, then global)
+//   k_jpg_front   a strip of MCUs per work group: fixed-point YCbCr, 2:1 chroma
+//                 boxes with the alternating bias, samples past the edges
+//                 replicated, the islow, ifast or float DCT (rows in
+//                 registers, columns through LDS) and its quantisation, the
+//                 blocks of the last MCUs past a component's own extent
+//                 (zero, with the DC of the block to the left / above), and
+//                 the symbol counts of the four tables; coefficients stored
+//                 in zigzag order
+//   k_jpg_dc0     the DC symbols of the strips' first MCUs
+//   k_jpg_coef, k_jpg_dummy, k_jpg_stats   the same one lane a block, for
+//                 libjpeg's smoothing filter, which reads past its block
 //   (host)        optimal code lengths per table (T.81 K.2, K.3)
-//   k_jpg_len     bits per block; k_scan_* their offsets
-//   k_jpg_emit    each block writes its codes at its bit offset (atomic OR
-//                 into zeroed words, most significant bit first)
+//   k_jpg_code<0> bits per 256 blocks; k_jpg_scan their offsets
+//   k_jpg_code<1> each work group's codes into LDS at their bit offsets, then
+//                 to memory in whole words (most significant bit first)
 //   k_stuff_*     a zero byte after every 0xFF: counts per chunk, offsets,
 //                 scatter
 #include "launch.h"
@@ -23,6 +25,7 @@
 #include <algorithm>
 #include <stdlib.h>
 #include <string.h>
+#include <type_traits>
 #include <vector>
 
 namespace {
@@ -202,7 +205,93 @@ DEV int jpg_quant(int32_t v, int q8)
   return v >= q8 ? v / q8 : 0;
 }
 
-// coefficients in natural order; q8: the divisors, luma then chroma: 8 x
+// a pixel's luma and chroma as jpg_ycc
+DEV void jpg_ycc_px(uint32_t p, int &Y, int &cb, int &cr)
+{
+  const int r = p & 255, g = (p >> 8) & 255, b = (p >> 16) & 255;
+  Y  = (19595 * r + 38470 * g + 7471 * b + 32768) >> 16;
+  cb = (-11059 * r - 21709 * g + 32768 * b + (128 << 16) + 32767) >> 16;
+  cr = (32768 * r - 27439 * g - 5329 * b + (128 << 16) + 32767) >> 16;
+}
+
+// the row transform of eight samples (level shifted); islow's and ifast's
+// results stay below 2^13 (samples below 2^7, at most 8 of them times 4, or
+// the scaled basis' 8 x 1.39), so LDS holds them in 16 bits
+template<int DCT, typename T>
+DEV void jpg_rows(int32_t *l, T *d)
+{
+  if(DCT == 2)
+  {
+    float f[8];
+#pragma unroll
+    for(int k = 0; k < 8; k++) f[k] = (float)l[k];
+    jpg_fdct8_float<1>(f);
+#pragma unroll
+    for(int k = 0; k < 8; k++) d[k] = (T)f[k];
+    return;
+  }
+  if(DCT == 1) jpg_fdct8_ifast<1>(l);
+  else jpg_fdct8<0, 1>(l);
+#pragma unroll
+  for(int k = 0; k < 8; k++) d[k] = (T)l[k];
+}
+
+// eight row values into LDS in 16-byte stores
+DEV void jpg_put8(int16_t __attribute__((may_alias)) *p, const int16_t __attribute__((may_alias)) *d)
+{
+  uint32_t w[4];
+#pragma unroll
+  for(int k = 0; k < 4; k++) w[k] = (uint32_t)(uint16_t)d[2 * k] | ((uint32_t)(uint16_t)d[2 * k + 1] << 16);
+  typedef uint4 __attribute__((may_alias)) u4;
+  *(u4 *)p = make_uint4(w[0], w[1], w[2], w[3]);
+}
+DEV void jpg_put8(float *p, const float *d)
+{
+  ((float4 *)p)[0] = make_float4(d[0], d[1], d[2], d[3]);
+  ((float4 *)p)[1] = make_float4(d[4], d[5], d[6], d[7]);
+}
+
+// v / q rounded half away from zero, as jpg_quant, by the reciprocal
+// m = ceil(2^32 / q): floor(x m / 2^32) = floor(x / q) while x (m q - 2^32)
+// stays below 2^32, and here x < 2^19, q < 2^12; q = 1 has m = 0
+DEV int32_t jpg_quant_m(int32_t v, int32_t q, uint32_t m)
+{
+  const uint32_t x = (uint32_t)(v < 0 ? -v : v) + ((uint32_t)q >> 1);
+  const uint32_t d = m ? __umulhi(x, m) : x;
+  return v < 0 ? -(int32_t)d : (int32_t)d;
+}
+
+// a block's column (elements 8 apart) transformed and quantised; q: the
+// divisors of the column, their reciprocals 128 further
+template<int DCT, typename T>
+DEV void jpg_cols(const T *p, int32_t o[8], const int32_t *q)
+{
+  if(DCT == 2)
+  {
+    float f[8];
+#pragma unroll
+    for(int r = 0; r < 8; r++) f[r] = (float)p[8 * r];
+    jpg_fdct8_float<1>(f);
+#pragma unroll
+    for(int r = 0; r < 8; r++) o[r] = (int32_t)rintf(f[r] * __int_as_float(q[8 * r]));
+    return;
+  }
+  int32_t d[8];
+#pragma unroll
+  for(int r = 0; r < 8; r++) d[r] = (int32_t)p[8 * r];
+  if(DCT == 1) jpg_fdct8_ifast<1>(d);
+  else jpg_fdct8<1, 1>(d);
+#pragma unroll
+  for(int r = 0; r < 8; r++) o[r] = jpg_quant_m(d[r], q[8 * r], (uint32_t)q[128 + 8 * r]);
+}
+
+constexpr uint8_t jz_dev[64] = {
+  0, 1, 8, 16, 9, 2, 3, 10, 17, 24, 32, 25, 18, 11, 4, 5, 12, 19, 26, 33, 40, 48, 41, 34, 27, 20, 13, 6, 7, 14, 21,
+  28, 35, 42, 49, 56, 57, 50, 43, 36, 29, 22, 15, 23, 30, 37, 44, 51, 58, 59, 52, 45, 38, 31, 39, 46, 53, 60, 61, 54,
+  47, 55, 62, 63 };
+
+// One lane a block, for the smoothing filter only (its 3x3 and 4x4 windows
+// reach past the block).  q8: the divisors, luma then chroma: 8 x
 // quantiser (DCT 0, islow), 8 x quantiser x the AAN factors in integer
 // (1, ifast), or the float reciprocal of that (2, float; its bits)
 template<int DCT>
@@ -251,15 +340,11 @@ __global__ void __launch_bounds__(64) k_jpg_coef(jpg_geom g, const int32_t *q8, 
     for(int k = 0; k < 8; k++) jpg_fdct8<1, 8>(d + k);
   }
   // stored in zigzag order, the order the entropy coder walks them
-  constexpr uint8_t zz[64] = {
-    0, 1, 8, 16, 9, 2, 3, 10, 17, 24, 32, 25, 18, 11, 4, 5, 12, 19, 26, 33, 40, 48, 41, 34, 27, 20, 13, 6, 7, 14, 21,
-    28, 35, 42, 49, 56, 57, 50, 43, 36, 29, 22, 15, 23, 30, 37, 44, 51, 58, 59, 52, 45, 38, 31, 39, 46, 53, 60, 61, 54,
-    47, 55, 62, 63 };
 #pragma unroll
   for(int k = 0; k < 64; k += 2)
   {
-    const int a = DCT == 2 ? d[zz[k]] : jpg_quant(d[zz[k]], q[zz[k]]);
-    const int e = DCT == 2 ? d[zz[k + 1]] : jpg_quant(d[zz[k + 1]], q[zz[k + 1]]);
+    const int a = DCT == 2 ? d[jz_dev[k]] : jpg_quant(d[jz_dev[k]], q[jz_dev[k]]);
+    const int e = DCT == 2 ? d[jz_dev[k + 1]] : jpg_quant(d[jz_dev[k + 1]], q[jz_dev[k + 1]]);
     *(uint32_t *)(o + k) = (uint32_t)(uint16_t)a | ((uint32_t)(uint16_t)e << 16);
   }
 }
@@ -344,154 +429,439 @@ __global__ void __launch_bounds__(256) k_jpg_stats(jpg_geom g, const int16_t *co
     if(h[k]) atomicAdd(freq + k, h[k]);
 }
 
-struct jpg_codes { uint16_t code[4][256]; uint8_t len[4][256]; };
-
-// bits per block (mode 0) or the block's codes at its offset (mode 1)
-template<int EMIT>
-__global__ void __launch_bounds__(256) k_jpg_code(jpg_geom g, const int16_t *coef, const jpg_codes *hc,
-                                                  uint64_t *bits, uint32_t *words)
+// nonzero flags of the eight coefficients of a 16-byte chunk, one bit each
+DEV uint32_t jpg_nz8(uint4 u)
 {
-  const int b = blockIdx.x * 256 + threadIdx.x;
-  if(b >= g.nb) return;
-  int c, bx, by, i;
-  jpg_block(g, b, c, bx, by, i);
-  const int t = c ? 1 : 0;
-  const uint16_t *dcc = hc->code[2 * t], *acc_c = hc->code[2 * t + 1];
-  const uint8_t *dcl = hc->len[2 * t], *acl = hc->len[2 * t + 1];
-  jpg_blk z;
-  jpg_load(z, coef, b);
-  const int p = jpg_prev(g, b);
-  const int last = p < 0 ? 0 : coef[(long)p * 64];
-  // writer: acc holds the bits from word w on, `used` of them taken
-  uint64_t total = 0, acc = 0;
-  long w = 0;
-  int used = 0;
-  if(EMIT) { const uint64_t off = bits[b]; w = (long)(off >> 5); used = (int)(off & 31); }
+  const uint32_t w[4] = { u.x, u.y, u.z, u.w };
+  uint32_t m = 0;
+#pragma unroll
+  for(int k = 0; k < 4; k++) m |= ((w[k] & 0xffffu) ? 1u << (2 * k) : 0u) | ((w[k] >> 16) ? 2u << (2 * k) : 0u);
+  return m;
+}
+
+// ---- samples, DCT, quantisation and symbol counts ------------------------------
+//
+// A work group takes 32 MCUs of one MCU row.  Thread (r, i) loads the pixels
+// of chroma row r of MCU i (8 HS x VS pixels, 16-byte loads where the image
+// allows), forms the component samples in registers and transforms their rows;
+// the columns go through LDS (8 lanes a block: its columns; the block stride of
+// 72 keeps both directions free of bank conflicts), where the quantised
+// coefficients land in zigzag order and leave in 16-byte stores.  One lane a
+// block with its 64 samples in registers converted every pixel once per
+// component and touched 64 cache lines an instruction: 707 us for 24 MP 4:4:4,
+// and 101 us more to read the coefficients again for the counts; this takes
+// 123 us.  The 144 MB written and 96 MB read take 48 us at 5 TB/s.
+#define JF_N 32                       // MCUs a strip
+#define JF_S 72                       // elements a block in LDS
+#define JF_COPIES 4                   // LDS histograms, by lane
+#define JF_FREQ 8                     // global histograms, by work group
+#define JF_HIST (2 * 256 + 2 * 16)    // AC luma, AC chroma, DC luma, DC chroma
+typedef int16_t __attribute__((may_alias)) jpg_i16;
+typedef uint4 __attribute__((may_alias)) jpg_u4;
+
+template<int DCT, int HS, int VS>
+__global__ void __launch_bounds__(256) k_jpg_front(jpg_geom g, const int32_t *q8, const uint8_t *zinv, int16_t *coef,
+                                                   uint32_t *freq, int ntx, int ntiles, int vec)
+{
+  constexpr int NL = HS * VS, BPM = NL + 2;
+  typedef typename std::conditional<DCT == 2, float, jpg_i16>::type T;
+  __shared__ __align__(16) T tmp[BPM * JF_N * JF_S];
+  __shared__ __align__(8) uint8_t nz[BPM * JF_N * 8];
+  __shared__ uint32_t hist[JF_COPIES][JF_HIST];
+  constexpr int ZS = JF_S * sizeof(T) / 2;   // int16 elements a block
+  jpg_i16 *zt = (jpg_i16 *)tmp;
+  const int t = threadIdx.x, col = t % 8;
+  for(int k = t; k < JF_COPIES * JF_HIST; k += 256) (&hist[0][0])[k] = 0;
+  uint32_t zp[8];   // zigzag positions of this lane's column
+#pragma unroll
+  for(int r = 0; r < 8; r++) zp[r] = zinv[8 * r + col];
+#pragma unroll 1
+  for(int tile = blockIdx.x; tile < ntiles; tile += gridDim.x)
+  {
+    const int uy = tile / ntx, u0 = (tile - uy * ntx) * JF_N, nu = min(JF_N, g.mx - u0);
+    {
+      const int i = t % JF_N, r = t / JF_N, ux = min(u0 + i, g.mx - 1);
+      int cb[8], cr[8];
+#pragma unroll
+      for(int k = 0; k < 8; k++) cb[k] = cr[k] = 0;
+#pragma unroll
+      for(int v = 0; v < VS; v++)
+#pragma unroll
+        for(int h = 0; h < HS; h++)
+        {
+          const int yy = VS * r + v, x0 = (ux * HS + h) * 8, y = min(uy * 8 * VS + yy, g.H - 1);
+          const uint8_t *row = g.rgba + 4 * (long)y * g.pitch;
+          uint32_t px[8];
+          if(vec && x0 + 8 <= g.W)
+          {
+            const uint4 a = *(const uint4 *)(row + 4 * x0), b = *(const uint4 *)(row + 4 * x0 + 16);
+            px[0] = a.x; px[1] = a.y; px[2] = a.z; px[3] = a.w;
+            px[4] = b.x; px[5] = b.y; px[6] = b.z; px[7] = b.w;
+          }
+          else
+#pragma unroll
+            for(int k = 0; k < 8; k++) px[k] = *(const uint32_t *)(row + 4 * min(x0 + k, g.W - 1));
+          T d[8];
+          int32_t l[8];
+#pragma unroll
+          for(int k = 0; k < 8; k++)
+          {
+            int Y, b, c;
+            jpg_ycc_px(px[k], Y, b, c);
+            l[k] = Y - 128;
+            cb[(h * 8 + k) / HS] += b;
+            cr[(h * 8 + k) / HS] += c;
+          }
+          jpg_rows<DCT>(l, d);
+          const int j = (yy / 8) * HS + h;
+          jpg_put8(tmp + (j * JF_N + i) * JF_S + (yy % 8) * 8, d);
+        }
+#pragma unroll
+      for(int c = 0; c < 2; c++)
+      {
+        int32_t l[8];
+        T d[8];
+#pragma unroll
+        for(int k = 0; k < 8; k++)
+        {
+          const int sum = c ? cr[k] : cb[k];
+          l[k] = (NL == 1 ? sum : VS == 2 ? (sum + ((k & 1) ? 2 : 1)) >> 2 : (sum + (k & 1)) >> 1) - 128;
+        }
+        jpg_rows<DCT>(l, d);
+        jpg_put8(tmp + ((NL + c) * JF_N + i) * JF_S + r * 8, d);
+      }
+    }
+    __syncthreads();
+    const bool edge = (u0 + nu) * HS > g.wib[0] || (uy + 1) * VS > g.hib[0];
+#pragma unroll
+    for(int j = 0; j < BPM; j++)
+    { // the columns of block j of 32 MCUs, 8 lanes a block; a block's lanes are
+      // of one wave, so its coefficients may take the place of its rows
+      const int i = t / 8;
+      T *p = tmp + (j * JF_N + i) * JF_S + col;
+      int32_t o[8];
+      jpg_cols<DCT>(p, o, q8 + (j < NL ? 0 : 64) + col);
+      if(edge && j < NL && ((u0 + i) * HS + j % HS >= g.wib[0] || uy * VS + j / HS >= g.hib[0]))
+#pragma unroll
+        for(int r = 0; r < 8; r++) o[r] = 0;
+      __builtin_amdgcn_wave_barrier();
+      jpg_i16 *z = zt + (j * JF_N + i) * ZS;
+#pragma unroll
+      for(int r = 0; r < 8; r++) z[zp[r]] = (int16_t)o[r];
+    }
+    __syncthreads();
+    if(NL > 1 && edge)
+    { // blocks past the extent take the DC of the block to the left or, in the
+      // rows below, of the last block of the row above in the MCU
+      if(t < nu)
+        for(int j = 1; j < NL; j++)
+        {
+          const bool below = uy * VS + j / HS >= g.hib[0], right = (u0 + t) * HS + j % HS >= g.wib[0];
+          if(below || right) zt[(j * JF_N + t) * ZS] = zt[((below ? j - j % HS - 1 : j - 1) * JF_N + t) * ZS];
+        }
+      __syncthreads();
+    }
+    int16_t *co = coef + ((long)uy * g.mx + u0) * BPM * 64;
+    for(int e = t; e < nu * BPM * 8; e += 256)
+    {
+      const int b = e / 8, c = e % 8, i = b / BPM, j = b - i * BPM;
+      const uint4 u = *(const jpg_u4 *)(zt + (j * JF_N + i) * ZS + 8 * c);
+      *(uint4 *)(co + (long)e * 8) = u;
+      nz[(j * JF_N + i) * 8 + c] = (uint8_t)jpg_nz8(u);
+    }
+    __syncthreads();
+    if(t < BPM * JF_N && t % JF_N < nu)
+    { // a thread a block: its symbols
+      const int j = t / JF_N, i = t % JF_N, c = j < NL ? 0 : 1;
+      const jpg_i16 *z = zt + t * ZS;
+      uint32_t *h = hist[t % JF_COPIES];
+      const bool first = j == 0 || j >= NL;     // its predecessor lies in the MCU before
+      const bool have = !first || i > 0 || (uy == 0 && u0 == 0);
+      const int last = !first ? zt[(t - JF_N) * ZS] : i > 0 ? zt[((j == 0 ? NL - 1 : j) * JF_N + i - 1) * ZS] : 0;
+      if(have) atomicAdd(h + 512 + 16 * c + jpg_nbits(z[0] - last), 1u);
+      uint64_t m = *(const uint64_t *)(nz + 8 * t) & ~1ull;
+      int prev = 0;
+      const int end = m ? 63 - __clzll(m) : 0;
+      while(m)
+      {
+        const int k = __builtin_ctzll(m);
+        m &= m - 1;
+        int run = k - prev - 1;
+        prev = k;
+        if(run > 15) { atomicAdd(h + 256 * c + 0xf0, (uint32_t)(run >> 4)); run &= 15; }
+        atomicAdd(h + 256 * c + ((run << 4) | jpg_nbits(z[k])), 1u);
+      }
+      if(end < 63) atomicAdd(h + 256 * c, 1u);
+    }
+    __syncthreads();
+  }
+  uint32_t *f = freq + (blockIdx.x % JF_FREQ) * 4 * 257;
+  for(int k = t; k < JF_HIST; k += 256)
+  {
+    uint32_t n = 0;
+#pragma unroll
+    for(int c = 0; c < JF_COPIES; c++) n += hist[c][k];
+    // the tables' order: DC luma, AC luma, DC chroma, AC chroma
+    if(n) atomicAdd(f + (k < 512 ? (2 * (k / 256) + 1) * 257 + k % 256 : 2 * ((k - 512) / 16) * 257 + (k - 512) % 16), n);
+  }
+}
+
+// the DC symbols of each strip's first MCU, whose predecessor another work
+// group made: a thread per strip and component
+__global__ void __launch_bounds__(256) k_jpg_dc0(jpg_geom g, const int16_t *coef, uint32_t *freq, int ntx, int ntiles)
+{
+  __shared__ uint32_t h[32];
+  if(threadIdx.x < 32) h[threadIdx.x] = 0;
+  __syncthreads();
+  const int k = blockIdx.x * 256 + threadIdx.x;
+  const int tile = k / 3, c = k % 3, n0 = g.hs * g.vs;
+  const int uy = tile / ntx, u = uy * g.mx + (tile - uy * ntx) * JF_N;
+  if(k < 3 * ntiles && u > 0)
+  {
+    const int b = u * g.bpm + (c ? n0 + c - 1 : 0), p = jpg_prev(g, b);
+    atomicAdd(h + 16 * (c ? 1 : 0) + jpg_nbits(coef[(long)b * 64] - coef[(long)p * 64]), 1u);
+  }
+  __syncthreads();
+  if(threadIdx.x < 32 && h[threadIdx.x])
+    atomicAdd(freq + (blockIdx.x % JF_FREQ) * 4 * 257 + 2 * (threadIdx.x / 16) * 257 + threadIdx.x % 16, h[threadIdx.x]);
+}
+
+// ---- entropy coding --------------------------------------------------------------
+//
+// A work group codes 256 consecutive blocks, a thread a block: the blocks are
+// staged in LDS (coalesced; reading a block by its own lane fetched 64 cache
+// lines an instruction), each thread walks its nonzero coefficients by their
+// mask, and the code tables lie in LDS too.  EMIT 0: each block's bits and the
+// group's.  EMIT 1: the blocks' bits are scanned and their codes ORed into the group's
+// words in LDS, which leave as whole words; only the first and the last, which
+// the neighbours share, are ORed in memory.  A group of more than JC_WORDS
+// words (over 256 bits a block) ORs its words in memory directly.
+#define JC_WORDS 2048
+struct jpg_codes { uint32_t v[4][256]; };   // code | length << 16
+
+template<int EMIT>
+__global__ void __launch_bounds__(256) k_jpg_code(jpg_geom g, const int16_t *coef, const jpg_codes *hc, uint16_t *blen,
+                                                  uint64_t *gbits, uint32_t *words, uint64_t cap)
+{
+  __shared__ __align__(16) int16_t zt[256 * JF_S];
+  __shared__ __align__(8) uint8_t nz[256 * 8];
+  __shared__ uint32_t tab[4][256];
+  __shared__ uint32_t lw[EMIT ? JC_WORDS : 1];
+  __shared__ uint32_t wsum[4];
+  const int t = threadIdx.x, b0 = blockIdx.x * 256, nb = min(256, g.nb - b0), b = b0 + t;
+  // a stream larger than the buffer: the host sees the total and asks again
+  if(EMIT && gbits[gridDim.x] > cap) return;
+  for(int k = t; k < 1024; k += 256) (&tab[0][0])[k] = (&hc->v[0][0])[k];
+  if(EMIT) for(int k = t; k < JC_WORDS; k += 256) lw[k] = 0;
+#pragma unroll
+  for(int e = t; e < 2048; e += 256)
+  {
+    const uint4 u = e < 8 * nb ? ((const uint4 *)(coef + (long)b0 * 64))[e] : make_uint4(0, 0, 0, 0);
+    *(jpg_u4 *)(zt + (e / 8) * JF_S + 8 * (e % 8)) = u;
+    nz[e] = (uint8_t)jpg_nz8(u);
+  }
+  __syncthreads();
+  int c = 0, bx, by, ii, last = 0;
+  if(t < nb)
+  {
+    jpg_block(g, b, c, bx, by, ii);
+    const int p = jpg_prev(g, b);
+    last = p < 0 ? 0 : p >= b0 ? zt[(p - b0) * JF_S] : coef[(long)p * 64];
+  }
+  const uint32_t *dct = tab[c ? 2 : 0], *act = tab[c ? 3 : 1];
+  const int16_t *z = zt + t * JF_S;
+  const int diff = z[0] - last, dn = jpg_nbits(diff);
+  const uint64_t ac = *(const uint64_t *)(nz + 8 * t) & ~1ull;
+  // every code with its extra bits, at most 16 + 11 together
+  auto walk = [&](auto put) {
+    if(t >= nb) return;
+    const uint32_t d = dct[dn];
+    put(((d & 0xffffu) << dn) | ((uint32_t)(diff < 0 ? diff - 1 : diff) & ((1u << dn) - 1)), (int)(d >> 16) + dn);
+    uint64_t m = ac;
+    int prev = 0;
+    while(m)
+    {
+      const int k = __builtin_ctzll(m);
+      m &= m - 1;
+      int run = k - prev - 1;
+      prev = k;
+      for(; run > 15; run -= 16) { const uint32_t e = act[0xf0]; put(e & 0xffffu, (int)(e >> 16)); }
+      const int v = z[k], s = jpg_nbits(v);
+      const uint32_t e = act[(run << 4) | s];
+      put(((e & 0xffffu) << s) | ((uint32_t)(v < 0 ? v - 1 : v) & ((1u << s) - 1)), (int)(e >> 16) + s);
+    }
+    if(prev < 63) { const uint32_t e = act[0]; put(e & 0xffffu, (int)(e >> 16)); }
+  };
+  uint32_t total = 0;     // at most 64 codes of 27 bits
+  if(EMIT) total = t < nb ? blen[b] : 0u;
+  else
+  {
+    walk([&](uint32_t, int n) { total += n; });
+    if(t < nb) blen[b] = (uint16_t)total;
+  }
+  // inclusive scan of the blocks' bits over the group
+  uint32_t inc = total;
+  for(int o = 1; o < 64; o <<= 1)
+  {
+    const uint32_t y = __shfl_up(inc, o);
+    if(t % 64 >= o) inc += y;
+  }
+  if(t % 64 == 63) wsum[t / 64] = inc;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+#pragma unroll
+  for(int k = 0; k < 4; k++)
+  {
+    if(k < t / 64) before += wsum[k];
+    all += wsum[k];
+  }
+  if(!EMIT) { if(t == 0) gbits[blockIdx.x] = all; return; }
+  const uint64_t g0 = gbits[blockIdx.x];
+  // the free bits of the stream's last byte are ones
+  const uint32_t pad = b0 + nb == g.nb ? (uint32_t)(-(g0 + all) & 7) : 0u;
+  const uint32_t o0 = (uint32_t)(g0 & 31), nw = (o0 + all + pad + 31) / 32;
+  uint32_t *gw = words + (g0 >> 5);
+  const bool lds = nw <= JC_WORDS;
+  uint32_t at = o0 + before + inc - total, w = at >> 5;
+  int used = (int)(at & 31);
+  uint64_t acc = 0;
+  auto flush = [&](uint32_t x) {
+    if(lds) atomicOr(lw + w, x);
+    else atomicOr(gw + w, x);
+  };
   auto put = [&](uint32_t v, int n) {
-    if(!EMIT) { total += n; return; }
     if(!n) return;
     acc |= (uint64_t)v << (64 - used - n);
     used += n;
     if(used >= 32)
     {
-      atomicOr(words + w, (uint32_t)(acc >> 32));
+      flush((uint32_t)(acc >> 32));
       acc <<= 32;
       used -= 32;
       w++;
     }
   };
-  const int diff = z.at(0) - last, n = jpg_nbits(diff);
-  put(dcc[n], dcl[n]);
-  put((uint32_t)(diff < 0 ? diff - 1 : diff) & ((1u << n) - 1), n);
-  int run = 0;
-#pragma unroll
-  for(int k = 1; k < 64; k++)
-  {
-    const int v = z.at(k);
-    if(!v) { run++; continue; }
-    while(run > 15) { put(acc_c[0xf0], acl[0xf0]); run -= 16; }
-    const int s = jpg_nbits(v), sym = (run << 4) | s;
-    put(acc_c[sym], acl[sym]);
-    put((uint32_t)(v < 0 ? v - 1 : v) & ((1u << s) - 1), s);
-    run = 0;
-  }
-  if(run) put(acc_c[0], acl[0]);
-  if(EMIT) { if(used) atomicOr(words + w, (uint32_t)(acc >> 32)); }
-  else bits[b] = total;
-}
-
-// exclusive scan of n u64 in place: 1024 a work group, then the group sums
-__global__ void __launch_bounds__(256) k_scan_local(uint64_t *v, long n, uint64_t *sums)
-{
-  __shared__ uint64_t s[256];
-  const long base = (long)blockIdx.x * 1024 + 4 * threadIdx.x;
-  uint64_t x[4], t = 0;
-  for(int j = 0; j < 4; j++) { x[j] = base + j < n ? v[base + j] : 0; t += x[j]; }
-  s[threadIdx.x] = t;
+  walk(put);
+  if(pad && t == nb - 1) put((1u << pad) - 1u, (int)pad);
+  if(t < nb && used) flush((uint32_t)(acc >> 32));
+  if(!lds) return;
   __syncthreads();
-  for(int o = 1; o < 256; o <<= 1)
-  {
-    const uint64_t a = threadIdx.x >= (unsigned)o ? s[threadIdx.x - o] : 0;
-    __syncthreads();
-    s[threadIdx.x] += a;
-    __syncthreads();
-  }
-  uint64_t run = s[threadIdx.x] - t;
-  for(int j = 0; j < 4; j++) { if(base + j < n) v[base + j] = run; run += x[j]; }
-  if(threadIdx.x == 255) sums[blockIdx.x] = s[255];
+  for(uint32_t k = t; k < nw; k += 256)
+    if(k == 0 || k == nw - 1) { if(lw[k]) atomicOr(gw + k, lw[k]); }
+    else gw[k] = lw[k];
 }
 
-__global__ void __launch_bounds__(256) k_scan_sums(uint64_t *sums, int n, uint64_t *total)
-{ // one work group: exclusive scan of the group sums, and their total
-  __shared__ uint64_t s[256];
-  uint64_t carry = 0;
-  for(int b0 = 0; b0 < n; b0 += 256)
-  {
-    const int k = b0 + threadIdx.x;
-    const uint64_t x = k < n ? sums[k] : 0;
-    s[threadIdx.x] = x;
-    __syncthreads();
-    for(int o = 1; o < 256; o <<= 1)
-    {
-      const uint64_t a = threadIdx.x >= (unsigned)o ? s[threadIdx.x - o] : 0;
-      __syncthreads();
-      s[threadIdx.x] += a;
-      __syncthreads();
-    }
-    if(k < n) sums[k] = carry + s[threadIdx.x] - x;
-    carry += s[255];
-    __syncthreads();
-  }
-  if(threadIdx.x == 0) *total = carry;
-}
-
-__global__ void __launch_bounds__(256) k_scan_add(uint64_t *v, long n, const uint64_t *sums)
+// exclusive scan of n u64 values in place by one work group, the total after
+// them: each thread a run of values
+__global__ void __launch_bounds__(1024) k_jpg_scan(uint64_t *v, int n)
 {
-  const long k = (long)blockIdx.x * 256 + threadIdx.x;
-  if(k < n) v[k] += sums[k / 1024];
+  __shared__ uint64_t ws[16];
+  const int t = threadIdx.x, per = (n + 1023) / 1024, a = min(t * per, n), e = min(a + per, n);
+  uint64_t sum = 0;
+  for(int k = a; k < e; k++) sum += v[k];
+  uint64_t inc = sum;
+  for(int o = 1; o < 64; o <<= 1)
+  {
+    const uint64_t y = __shfl_up(inc, o);
+    if(t % 64 >= o) inc += y;
+  }
+  if(t % 64 == 63) ws[t / 64] = inc;
+  __syncthreads();
+  uint64_t run = inc - sum;
+  for(int k = 0; k < t / 64; k++) run += ws[k];
+  for(int k = a; k < e; k++)
+  {
+    const uint64_t x = v[k];
+    v[k] = run;
+    run += x;
+  }
+  if(t == 1023) v[n] = run;
 }
 
-DEV uint32_t jpg_byte(const uint32_t *words, long i) { return (words[i >> 2] >> (24 - 8 * (i & 3))) & 0xffu; }
+// ---- byte stuffing: a work group 4096 bytes, a thread 16 -------------------------
+#define JS_BYTES 4096
 
-// 0xFF bytes per chunk of 1024
-__global__ void __launch_bounds__(256) k_stuff_count(const uint32_t *words, long nbytes, uint64_t *cnt)
+// the bytes of this thread's four words, and which of them (bit k) are 0xFF;
+// bytes past the stream count as none
+DEV int jpg_bytes16(const uint32_t *words, uint64_t nbytes, uint8_t by[16], uint32_t &ff)
+{
+  const uint64_t i0 = (uint64_t)blockIdx.x * JS_BYTES + 16 * threadIdx.x;
+  ff = 0;
+  if(i0 >= nbytes) return 0;
+  const int n = (int)min((uint64_t)16, nbytes - i0);
+  const uint4 u = *(const uint4 *)(words + i0 / 4);     // the words are padded to whole groups of four
+  const uint32_t w[4] = { u.x, u.y, u.z, u.w };
+#pragma unroll
+  for(int k = 0; k < 16; k++)
+  {
+    by[k] = (uint8_t)(w[k / 4] >> (24 - 8 * (k % 4)));
+    if(k < n && by[k] == 0xffu) ff |= 1u << k;
+  }
+  return n;
+}
+
+// total: the stream's bits; cap: the bits the buffer holds
+__global__ void __launch_bounds__(256) k_stuff_count(const uint32_t *words, const uint64_t *total, uint64_t cap, uint64_t *cnt)
 {
   __shared__ uint32_t s;
   if(threadIdx.x == 0) s = 0;
   __syncthreads();
-  uint32_t c = 0;
-  for(int j = 0; j < 4; j++)
-  {
-    const long i = (long)blockIdx.x * 1024 + 4 * threadIdx.x + j;
-    if(i < nbytes && jpg_byte(words, i) == 0xffu) c++;
-  }
-  if(c) atomicAdd(&s, c);
+  uint8_t by[16];
+  uint32_t ff = 0;
+  if(*total <= cap) jpg_bytes16(words, (*total + 7) / 8, by, ff);
+  if(ff) atomicAdd(&s, (uint32_t)__popc(ff));
   __syncthreads();
   if(threadIdx.x == 0) cnt[blockIdx.x] = s;
 }
 
-__global__ void __launch_bounds__(256) k_stuff_scatter(const uint32_t *words, long nbytes, const uint64_t *off,
-                                                       uint8_t *out)
+// the chunk with its zeros is formed in LDS, at the alignment of its place in
+// the output, and leaves in whole words but for its ends
+__global__ void __launch_bounds__(256) k_stuff_scatter(const uint32_t *words, const uint64_t *total, uint64_t cap,
+                                                       const uint64_t *off, uint8_t *out)
 {
-  __shared__ uint32_t s[256];
-  uint32_t by[4], c = 0;
-  const long i0 = (long)blockIdx.x * 1024 + 4 * threadIdx.x;
-  for(int j = 0; j < 4; j++) { by[j] = i0 + j < nbytes ? jpg_byte(words, i0 + j) : 0u; c += (i0 + j < nbytes && by[j] == 0xffu); }
-  s[threadIdx.x] = c;
-  __syncthreads();
-  for(int o = 1; o < 256; o <<= 1)
+  __shared__ __align__(4) uint8_t o[2 * JS_BYTES + 4];
+  __shared__ uint32_t ws[4];
+  if(*total > cap) return;
+  const uint64_t nbytes = (*total + 7) / 8, c0 = (uint64_t)blockIdx.x * JS_BYTES;
+  if(c0 >= nbytes) return;
+  const int t = threadIdx.x;
+  uint8_t by[16];
+  uint32_t ff;
+  const int n = jpg_bytes16(words, nbytes, by, ff);
+  const uint32_t c = n + __popc(ff);
+  uint32_t inc = c;
+  for(int d = 1; d < 64; d <<= 1)
   {
-    const uint32_t a = threadIdx.x >= (unsigned)o ? s[threadIdx.x - o] : 0;
-    __syncthreads();
-    s[threadIdx.x] += a;
-    __syncthreads();
+    const uint32_t y = __shfl_up(inc, d);
+    if(t % 64 >= d) inc += y;
   }
-  uint64_t at = (uint64_t)i0 + off[blockIdx.x] + s[threadIdx.x] - c;
-  for(int j = 0; j < 4; j++)
+  if(t % 64 == 63) ws[t / 64] = inc;
+  __syncthreads();
+  uint32_t at = inc - c, all = 0;
+#pragma unroll
+  for(int k = 0; k < 4; k++)
   {
-    if(i0 + j >= nbytes) break;
-    out[at++] = (uint8_t)by[j];
-    if(by[j] == 0xffu) out[at++] = 0;
+    if(k < t / 64) at += ws[k];
+    all += ws[k];
+  }
+  const uint64_t dst = c0 + off[blockIdx.x];
+  const uint32_t lead = (uint32_t)((uintptr_t)(out + dst) & 3);
+  at += lead;
+#pragma unroll
+  for(int k = 0; k < 16; k++)
+    if(k < n)
+    {
+      o[at++] = by[k];
+      if(ff & (1u << k)) o[at++] = 0;
+    }
+  __syncthreads();
+  uint8_t *base = out + dst - lead;
+  const uint32_t end = lead + all;
+  for(uint32_t k = 4 * t; k < end; k += 1024)
+  {
+    if(k >= lead && k + 4 <= end) *(uint32_t *)(base + k) = *(const uint32_t *)(o + k);
+    else
+      for(uint32_t q = max(k, lead); q < min(k + 4, end); q++) base[q] = o[q];
   }
 }
 
@@ -641,37 +1011,63 @@ extern "C" int vkdt_hip_jpg_encode_ex(const void *rgba, uint32_t wd, uint32_t ht
         q8[64 * t + k] = q << 3;
     }
 
-  // device: q8 | codes | freq | coef | dummy flags | bits | sums | total
-  const long ngroups = (nbl + 1023) / 1024;
-  const size_t o_q = 0, o_codes = 512, o_freq = o_codes + ((sizeof(jpg_codes) + 255) & ~(size_t)255);
-  const size_t o_coef = o_freq + 4 * 257 * 4 + 256 - (4 * 257 * 4) % 256;
+  // reciprocals of the integer divisors, and the zigzag positions
+  int32_t tables[256 + 16];
+  memcpy(tables, q8, sizeof(q8));
+  for(int k = 0; k < 128; k++)
+    tables[128 + k] = dct == VKDT_JPG_DCT_FLOAT || q8[k] == 1 ? 0 : (int32_t)(uint32_t)(((1ull << 32) + q8[k] - 1) / q8[k]);
+  for(int k = 0; k < 64; k++) ((uint8_t *)(tables + 256))[jz_host[k]] = (uint8_t)k;
+
+  // device: tables | codes | counts | coef | dummy flags | bits per 256 blocks, total | bits per block
+  const int ngroups = (int)((nbl + 255) / 256);
+  const size_t o_codes = 2048, o_freq = o_codes + sizeof(jpg_codes), nfreq = JF_FREQ * 4 * 257;
+  const size_t o_coef = (o_freq + nfreq * 4 + 255) & ~(size_t)255;
   const size_t o_dummy = o_coef + (size_t)nbl * 128;
-  const size_t o_bits = (o_dummy + nbl + 255) & ~(size_t)255;
-  const size_t o_sums = o_bits + (size_t)nbl * 8;
-  const size_t o_total = o_sums + (size_t)(ngroups + 1) * 8;
-  const size_t total = o_total + 256;
+  const size_t o_bits = (o_dummy + (smoothing ? nbl : 0) + 255) & ~(size_t)255;
+  const size_t o_blen = o_bits + (size_t)(ngroups + 1) * 8;
+  const size_t total = o_blen + (size_t)nbl * 2;
   uint8_t *dev = nullptr;
   if(int e = hip_fail(hipMalloc((void **)&dev, total), "jpg scratch")) return e;
   hipStream_t s = (hipStream_t)stream;
   int16_t *coef = (int16_t *)(dev + o_coef);
   uint32_t *freq = (uint32_t *)(dev + o_freq);
-  uint64_t *bits = (uint64_t *)(dev + o_bits), *sums = (uint64_t *)(dev + o_sums), *tot = (uint64_t *)(dev + o_total);
+  uint64_t *bits = (uint64_t *)(dev + o_bits);
+  uint16_t *blen = (uint16_t *)(dev + o_blen);
   uint8_t *words8 = nullptr, *stuffed = nullptr;
-  int err = hip_fail(hipMemcpyAsync(dev + o_q, q8, sizeof(q8), hipMemcpyHostToDevice, s), "jpg tables");
-  uint32_t fr[4 * 257];
+  int err = hip_fail(hipMemcpyAsync(dev, tables, sizeof(tables), hipMemcpyHostToDevice, s), "jpg tables");
+  std::vector<uint32_t> fr(nfreq);
   if(!err)
   {
-    hipLaunchKernelGGL(k_jpg_zero, dim3((4 * 257 + 255) / 256), dim3(256), 0, s, freq, (long)(4 * 257));
-    const auto coef_kernel = dct == VKDT_JPG_DCT_FLOAT ? k_jpg_coef<2> : (dct == VKDT_JPG_DCT_IFAST ? k_jpg_coef<1> : k_jpg_coef<0>);
-    hipLaunchKernelGGL(coef_kernel, dim3((g.nb + 63) / 64), dim3(64), 0, s, g, (const int32_t *)(dev + o_q), coef,
-                       dev + o_dummy);
-    hipLaunchKernelGGL(k_jpg_dummy, dim3((g.nb + 255) / 256), dim3(256), 0, s, g, coef, (const uint8_t *)(dev + o_dummy), 1);
-    hipLaunchKernelGGL(k_jpg_dummy, dim3((g.nb + 255) / 256), dim3(256), 0, s, g, coef, (const uint8_t *)(dev + o_dummy), 2);
-    hipLaunchKernelGGL(k_jpg_stats, dim3((g.nb + 255) / 256), dim3(256), 0, s, g, (const int16_t *)coef, freq);
+    const int32_t *dq = (const int32_t *)dev;
+    hipLaunchKernelGGL(k_jpg_zero, dim3((unsigned)((nfreq + 255) / 256)), dim3(256), 0, s, freq, (long)nfreq);
+    if(smoothing)
+    {
+      const auto coef_kernel = dct == VKDT_JPG_DCT_FLOAT ? k_jpg_coef<2> : (dct == VKDT_JPG_DCT_IFAST ? k_jpg_coef<1> : k_jpg_coef<0>);
+      hipLaunchKernelGGL(coef_kernel, dim3((g.nb + 63) / 64), dim3(64), 0, s, g, dq, coef, dev + o_dummy);
+      hipLaunchKernelGGL(k_jpg_dummy, dim3((g.nb + 255) / 256), dim3(256), 0, s, g, coef, (const uint8_t *)(dev + o_dummy), 1);
+      hipLaunchKernelGGL(k_jpg_dummy, dim3((g.nb + 255) / 256), dim3(256), 0, s, g, coef, (const uint8_t *)(dev + o_dummy), 2);
+      hipLaunchKernelGGL(k_jpg_stats, dim3((g.nb + 255) / 256), dim3(256), 0, s, g, (const int16_t *)coef, freq);
+    }
+    else
+    {
+      const int ntx = (g.mx + JF_N - 1) / JF_N, ntiles = ntx * g.my;
+      const int vec = (uintptr_t)rgba % 16 == 0 && pitch % 4 == 0;
+      const auto front = [&](auto d) {
+        constexpr int D = decltype(d)::value;
+        // a few strips a work group, so that the counts reach memory rarely
+        hipLaunchKernelGGL((hs == 1 ? k_jpg_front<D, 1, 1> : vs == 1 ? k_jpg_front<D, 2, 1> : k_jpg_front<D, 2, 2>),
+                           dim3((unsigned)std::min(ntiles, 2048)), dim3(256), 0, s, g, dq, dev + 1024, coef, freq, ntx, ntiles, vec);
+      };
+      if(dct == VKDT_JPG_DCT_FLOAT) front(std::integral_constant<int, 2>());
+      else if(dct == VKDT_JPG_DCT_IFAST) front(std::integral_constant<int, 1>());
+      else front(std::integral_constant<int, 0>());
+      hipLaunchKernelGGL(k_jpg_dc0, dim3((3 * ntiles + 255) / 256), dim3(256), 0, s, g, (const int16_t *)coef, freq, ntx, ntiles);
+    }
     err = launch_post("jpg coefficients");
-    if(!err) err = hip_fail(hipMemcpyAsync(fr, freq, sizeof(fr), hipMemcpyDeviceToHost, s), "jpg counts");
+    if(!err) err = hip_fail(hipMemcpyAsync(fr.data(), freq, nfreq * 4, hipMemcpyDeviceToHost, s), "jpg counts");
     if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
   }
+  for(size_t k = 4 * 257; k < nfreq; k++) fr[k % (4 * 257)] += fr[k];
   uint8_t hb[4][17], hv[4][256];
   int nv[4] = { 0, 0, 0, 0 };
   jpg_codes hc;
@@ -680,70 +1076,51 @@ extern "C" int vkdt_hip_jpg_encode_ex(const void *rgba, uint32_t wd, uint32_t ht
   {
     for(int t = 0; t < 4; t++)
     {
-      jpg_huff(fr + 257 * t, hb[t], hv[t], nv + t);
+      jpg_huff(fr.data() + 257 * t, hb[t], hv[t], nv + t);
       int code = 0, k = 0;
       for(int len = 1; len <= 16; len++)
       {
-        for(int j = 0; j < hb[t][len]; j++, k++) { hc.code[t][hv[t][k]] = (uint16_t)code++; hc.len[t][hv[t][k]] = (uint8_t)len; }
+        for(int j = 0; j < hb[t][len]; j++, k++) hc.v[t][hv[t][k]] = (uint32_t)code++ | ((uint32_t)len << 16);
         code <<= 1;
       }
     }
     err = hip_fail(hipMemcpyAsync(dev + o_codes, &hc, sizeof(hc), hipMemcpyHostToDevice, s), "jpg codes");
   }
   uint64_t nbits = 0;
+  const jpg_codes *dhc = (const jpg_codes *)(dev + o_codes);
   if(!err)
   {
-    const jpg_codes *dhc = (const jpg_codes *)(dev + o_codes);
-    hipLaunchKernelGGL(k_jpg_code<0>, dim3((g.nb + 255) / 256), dim3(256), 0, s, g, (const int16_t *)coef, dhc, bits,
-                       (uint32_t *)nullptr);
-    hipLaunchKernelGGL(k_scan_local, dim3((unsigned)ngroups), dim3(256), 0, s, bits, nbl, sums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(256), 0, s, sums, (int)ngroups, tot);
-    hipLaunchKernelGGL(k_scan_add, dim3((unsigned)((nbl + 255) / 256)), dim3(256), 0, s, bits, nbl, (const uint64_t *)sums);
+    hipLaunchKernelGGL(k_jpg_code<0>, dim3((unsigned)ngroups), dim3(256), 0, s, g, (const int16_t *)coef, dhc, blen, bits,
+                       (uint32_t *)nullptr, (uint64_t)0);
+    hipLaunchKernelGGL(k_jpg_scan, dim3(1), dim3(1024), 0, s, bits, ngroups);
     err = launch_post("jpg lengths");
-    if(!err) err = hip_fail(hipMemcpyAsync(&nbits, tot, 8, hipMemcpyDeviceToHost, s), "jpg total");
+    if(!err) err = hip_fail(hipMemcpyAsync(&nbits, bits + ngroups, 8, hipMemcpyDeviceToHost, s), "jpg total");
     if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
   }
   const long nbytes = (long)((nbits + 7) / 8);
-  const long nwords = (long)((nbits + 31) / 32) + 1, nchunks = (nbytes + 1023) / 1024;
+  const long nwords = (nbytes + 15) / 16 * 4, nchunks = (nbytes + JS_BYTES - 1) / JS_BYTES;
   uint64_t nff = 0;
   if(!err)
-  { // words | chunk counts and their sums | stuffed bytes (at most twice)
-    const size_t wbytes = (size_t)nwords * 4, cbytes = (size_t)(nchunks + 1) * 8, gsum = (size_t)((nchunks + 1023) / 1024 + 1) * 8;
-    err = hip_fail(hipMalloc((void **)&words8, wbytes + 2 * cbytes + gsum + 256 + 2 * (size_t)nbytes + 16), "jpg stream");
-    if(!err)
+  { // words | 0xFF bytes before each chunk, their total | stuffed bytes (at most twice)
+    const size_t wbytes = ((size_t)nwords * 4 + 255) & ~(size_t)255, cbytes = ((size_t)(nchunks + 1) * 8 + 255) & ~(size_t)255;
+    err = hip_fail(hipMalloc((void **)&words8, wbytes + cbytes + 2 * (size_t)nbytes + 16), "jpg stream");
+    if(!err && nbytes > 0)
     {
       uint32_t *words = (uint32_t *)words8;
-      uint64_t *cnt = (uint64_t *)(words8 + wbytes), *csum = cnt + nchunks + 1, *ctot = csum + (nchunks + 1024) / 1024 + 1;
-      stuffed = words8 + wbytes + 2 * cbytes + gsum + 256;
+      uint64_t *cnt = (uint64_t *)(words8 + wbytes);
+      const uint64_t *tot = bits + ngroups;
+      stuffed = words8 + wbytes + cbytes;
       hipLaunchKernelGGL(k_jpg_zero, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, s, words, nwords);
-      hipLaunchKernelGGL(k_jpg_code<1>, dim3((g.nb + 255) / 256), dim3(256), 0, s, g, (const int16_t *)coef,
-                         (const jpg_codes *)(dev + o_codes), bits, words);
-      err = launch_post("jpg emit");
-      if(!err && (nbits & 7))
-      { // the last byte's free bits are ones
-        const uint32_t pad = (1u << (8 - (nbits & 7))) - 1u;
-        uint32_t wlast = 0;
-        const long wi = (long)((nbits - 1) >> 5);
-        err = hip_fail(hipMemcpyAsync(&wlast, words + wi, 4, hipMemcpyDeviceToHost, s), "jpg pad");
-        if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
-        const int byte_in_word = (int)(((nbits - 1) >> 3) & 3);
-        wlast |= pad << (24 - 8 * byte_in_word);
-        if(!err) err = hip_fail(hipMemcpyAsync(words + wi, &wlast, 4, hipMemcpyHostToDevice, s), "jpg pad");
-      }
-      if(!err && nbytes > 0)
-      {
-        hipLaunchKernelGGL(k_stuff_count, dim3((unsigned)nchunks), dim3(256), 0, s, (const uint32_t *)words, nbytes, cnt);
-        const long ng2 = (nchunks + 1023) / 1024;
-        hipLaunchKernelGGL(k_scan_local, dim3((unsigned)ng2), dim3(256), 0, s, cnt, nchunks, csum);
-        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(256), 0, s, csum, (int)ng2, ctot);
-        hipLaunchKernelGGL(k_scan_add, dim3((unsigned)((nchunks + 255) / 256)), dim3(256), 0, s, cnt, nchunks,
-                           (const uint64_t *)csum);
-        hipLaunchKernelGGL(k_stuff_scatter, dim3((unsigned)nchunks), dim3(256), 0, s, (const uint32_t *)words, nbytes,
-                           (const uint64_t *)cnt, stuffed);
-        err = launch_post("jpg stuffing");
-        if(!err) err = hip_fail(hipMemcpyAsync(&nff, ctot, 8, hipMemcpyDeviceToHost, s), "jpg stuffed");
-        if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
-      }
+      hipLaunchKernelGGL(k_jpg_code<1>, dim3((unsigned)ngroups), dim3(256), 0, s, g, (const int16_t *)coef, dhc, blen, bits, words,
+                         (uint64_t)nwords * 32);
+      hipLaunchKernelGGL(k_stuff_count, dim3((unsigned)nchunks), dim3(256), 0, s, (const uint32_t *)words, tot,
+                         (uint64_t)nwords * 32, cnt);
+      hipLaunchKernelGGL(k_jpg_scan, dim3(1), dim3(1024), 0, s, cnt, (int)nchunks);
+      hipLaunchKernelGGL(k_stuff_scatter, dim3((unsigned)nchunks), dim3(256), 0, s, (const uint32_t *)words, tot,
+                         (uint64_t)nwords * 32, (const uint64_t *)cnt, stuffed);
+      err = launch_post("jpg stuffing");
+      if(!err) err = hip_fail(hipMemcpyAsync(&nff, cnt + nchunks, 8, hipMemcpyDeviceToHost, s), "jpg stuffed");
+      if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
     }
   }
   out_t o;
