@@ -67,6 +67,29 @@ def test_many_images_one_launch(hip):
         buf.free()
 
 
+@pytest.mark.parametrize("W,Hh,comp,flat", [(1024, 1024, 1, (400, 528)), (512, 900, 2, None), (300, 200, 4, None),
+                                             (37, 5, 1, None), (258, 31, 1, None)],
+                         ids=["never-resynchronises", "3-work-groups", "4-components", "one-subsequence", "odd-lines"])
+def test_subsequences_and_line_groups(hip, W, Hh, comp, flat):
+    """one stream per image: a flat stretch whose symbols are all the same
+    three bits, where a decode from a wrong phase never falls into step (768
+    subsequences in a row, across work groups); streams of several work
+    groups, of less than one subsequence, and line counts that leave a
+    group of lines partly empty"""
+    rng = np.random.default_rng(W + Hh)
+    d = np.where(rng.random((Hh, W)) < 0.5, 1, -1) * (1 << rng.integers(0, 7, (Hh, W)))
+    if flat:
+        d[flat[0]:flat[1]] = 0
+        d[:flat[0]][rng.random((flat[0], W)) < 0.04] = 0
+    cfa = ((8192 + np.cumsum(d.reshape(Hh, -1, comp), axis=1).reshape(Hh, W)) & 0x3fff).astype(np.uint16)
+    stream = lj92.encode(cfa, 14, 1, comp)
+    blob, tiles = H.lj92_tiles([stream], W, Hh, W, Hh)
+    buf = hip.DeviceBuffer(W, Hh, 1, H.FMT_UI16)
+    H.lj92_decode(blob, tiles, [(buf.ptr, W, Hh, W)])
+    assert np.array_equal(buf.download(), cfa)
+    buf.free()
+
+
 @pytest.mark.parametrize("pred", [1, 6])
 def test_corrupt_entropy_data_refused(hip, pred):
     """entropy data of all ones (stuffed 0xff bytes): the tables reserve that

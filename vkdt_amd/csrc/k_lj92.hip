@@ -426,18 +426,32 @@ __global__ void __launch_bounds__(64) k_lj92(const lj92_job *jobs, int n, int *s
 // symbols of a wrong start:
 //   unstuff   one work group per stream: the segment without its stuffed
 //             zero bytes, up to the first marker, into aligned words
-//   first     lane g decodes subsequence k = bits [k S, (k+1) S) from k S:
-//             its symbol count and where its last symbol ends
-//   sync      while any lane's start differs from its predecessor's end, it
-//             decodes again from there (ping-pong ends; converges in as many
-//             rounds as the longest chain of wrong starts, a few)
+//   first     lane t of a work group decodes subsequence k = bits [k S, (k+1) S)
+//             from k S: its symbol count and where its last symbol ends; then
+//             while a lane's start differs from its predecessor's end it decodes
+//             again from there.  The first LJ92_WARM lanes repeat the end of
+//             the previous work group's range, so that its own first
+//             subsequences start right without waiting for it
+//   sync      the same rule across work groups, a round a launch (ping-pong
+//             ends): it finds nothing to change but for chains of wrong
+//             starts longer than the warm-up
 //   scan      symbol offsets per subsequence (one work group per stream)
 //   write     every lane decodes its subsequence once more into the
 //             differences; the last lane of a stream continues past the
 //             segment's end on zero bits as the serial decoder does
 //   col0/rows predictor 1 is two prefix sums: down the first column of
 //             each component, then along each scan line.
+// A decode is a chain of table lookups, so latency bounds it: the code table
+// and the work group's words lie in LDS.  24 MP in 384 tiles, unstuff to rows:
+// 1230 -> 665 us against lookups and words from memory and a launch per
+// synchronisation round (14 of them here).  Of the 665, `first` takes 378, most
+// of it the work groups whose subsequences lie in a clipped area: equal
+// symbols keep a wrong phase, so each waits for the one before.
 #define LJ92_SUB 512
+#define LJ92_WARM 32                  // warm-up subsequences of a work group
+#define LJ92_OWN (256 - LJ92_WARM)    // and its own
+#define LJ92_SW (LJ92_SUB / 32)       // words a subsequence
+#define LJ92_WROWS 4                  // scan lines a wave
 
 struct lj92_pst
 {
@@ -445,7 +459,8 @@ struct lj92_pst
   uint32_t *clean;         // unstuffed bytes as words, zero past the data
   uint32_t len, cwords;    // segment bytes; words of the clean region
   uint32_t sbase, K;       // first subsequence, subsequences (len * 8 / S rounded up)
-  uint32_t rbase;          // first scan line in the numbering of all streams
+  uint32_t bbase;          // first work group of LJ92_OWN subsequences
+  uint32_t rbase, qbase;   // first scan line, and group of LJ92_WROWS lines, in the numbering of all streams
   uint32_t S;              // samples of the scan
   const lj92_tab *tab;
   uint16_t *diff;          // S differences
@@ -505,7 +520,7 @@ __device__ static inline void lj92_cfill(lj92_cbits &b)
 // one symbol at the reader: its difference, and the bits it took; a prefix no
 // code matches takes one bit and yields no symbol (ok = 0), so that a decode
 // from any bit position is a function of that position alone
-__device__ static inline int lj92_csym(lj92_cbits &b, const lj92_tab *t, int &used, int &ok)
+template<class R> __device__ static inline int lj92_csym(R &b, const lj92_tab *t, int &used, int &ok)
 {
   lj92_cfill(b);
   const int c0 = b.cnt;
@@ -530,15 +545,14 @@ __device__ static inline int lj92_csym(lj92_cbits &b, const lj92_tab *t, int &us
   return diff;
 }
 
-// the stream and subsequence of global subsequence g (streams sorted by sbase)
-__device__ static inline int lj92_find(const lj92_pst *ps, int np, uint32_t g, bool rows)
+// the stream whose range of a numbering (sbase, bbase, ...: ascending) holds g
+__device__ static inline int lj92_find(const lj92_pst *ps, int np, uint32_t g, uint32_t lj92_pst::*base)
 {
   int lo = 0, hi = np - 1;
   while(lo < hi)
   {
     const int mid = (lo + hi + 1) >> 1;
-    const uint32_t b = rows ? lj92_ld(&ps[mid].rbase) : lj92_ld(&ps[mid].sbase);
-    if(b <= g) lo = mid; else hi = mid - 1;
+    if(lj92_ld(&(ps[mid].*base)) <= g) lo = mid; else hi = mid - 1;
   }
   return lo;
 }
@@ -561,88 +575,289 @@ __device__ static inline uint32_t lj92_count(const lj92_pst &p, uint32_t pos, ui
   return pos;
 }
 
+// inclusive sum over a work group of 256; ws: its waves' sums (4 words)
+__device__ static inline uint32_t lj92_scan256(uint32_t v, uint32_t *ws, uint32_t &all)
+{
+  const int t = threadIdx.x;
+  for(int o = 1; o < 64; o <<= 1)
+  {
+    const uint32_t y = __shfl_up(v, o);
+    if(t % 64 >= o) v += y;
+  }
+  __syncthreads();
+  if(t % 64 == 63) ws[t / 64] = v;
+  __syncthreads();
+  all = 0;
+  uint32_t before = 0;
+#pragma unroll
+  for(int k = 0; k < 4; k++)
+  {
+    if(k < t / 64) before += ws[k];
+    all += ws[k];
+  }
+  return v + before;
+}
+
+// 4096 bytes a round, 16 a thread (aligned word loads, shifted into place);
+// the kept bytes are packed in LDS and leave as whole words, a partial last
+// word waits for the next round.  The words read round the segment lie inside
+// the upload's allocation.  (One byte a load and 1024 bytes a round: 200 us for
+// 24 MP in 384 tiles.)
 __global__ void __launch_bounds__(256) k_lj92_unstuff(const lj92_pst *ps, uint32_t *nbits)
 {
-  __shared__ uint32_t s_sum[256];
+  __shared__ uint32_t ws[4];
   __shared__ uint32_t s_mark;
+  __shared__ uint32_t out[4096 / 4 + 2];
   const lj92_pst &p = ps[blockIdx.x];
   const uint8_t *src = p.src;
-  uint8_t *dst = (uint8_t *)p.clean;
+  uint32_t *dst = p.clean;
+  uint8_t *ob = (uint8_t *)out;
   const uint32_t len = p.len, t = threadIdx.x;
+  const int sh = 8 * (int)((uintptr_t)src & 3);
+  const uint32_t *sw = (const uint32_t *)((uintptr_t)src & ~(uintptr_t)3);
+  const uint32_t wlast = (len - 1 + sh / 8) / 4;       // the word of the segment's last byte
   uint32_t kept = 0;
   bool ended = false;
-  for(uint32_t base = 0; base < len && !ended; base += 256 * 4)
+  for(uint32_t base = 0; base < len && !ended; base += 4096)
   {
-    const uint32_t i0 = base + 4 * t;
-    uint32_t by[6];                                    // bytes i0-1 .. i0+4, zero outside
-    for(int j = 0; j < 6; j++)
+    const uint32_t i0 = base + 16 * t;
+    // bytes i0 .. i0 + 15 as little-endian words, the byte before and the one after
+    uint32_t w[6], x[5], pv = 0, nx = 0;
+    const uint32_t q = i0 / 4;
+#pragma unroll
+    for(int j = 0; j < 6; j++) w[j] = lj92_ld(sw + min(q + (uint32_t)j, wlast));
+    const uint32_t wp = lj92_ld(sw + (q ? min(q - 1, wlast) : 0u));
+#pragma unroll
+    for(int j = 0; j < 5; j++) x[j] = (uint32_t)((((uint64_t)w[j + 1] << 32) | w[j]) >> sh);
+    if(i0 > 0) pv = (uint32_t)((((uint64_t)w[0] << 32) | wp) >> sh) >> 24;
+    nx = x[4] & 0xff;
+    uint32_t mark = 0xffffffffu, keep = 0, last = pv;
+#pragma unroll
+    for(int j = 0; j < 16; j++)
     {
-      const long i = (long)i0 - 1 + j;
-      by[j] = i >= 0 && i < (long)len ? lj92_ld(src + i) : 0u;
+      const uint32_t c = (x[j / 4] >> (8 * (j % 4))) & 0xff, n = j < 15 ? (x[(j + 1) / 4] >> (8 * ((j + 1) % 4))) & 0xff : nx;
+      const uint32_t i = i0 + j;
+      if(i < len && mark == 0xffffffffu && c == 0xff && (i + 1 >= len || n != 0)) mark = i;
+      if(i < len && !(c == 0 && last == 0xff)) keep |= 1u << j;
+      last = c;
     }
-    uint32_t mark = 0xffffffffu;                       // first marker among this lane's bytes
-    for(int j = 3; j >= 0; j--)
-      if(i0 + j < len && by[j + 1] == 0xff && (i0 + j + 1 >= len || by[j + 2] != 0)) mark = i0 + j;
     if(t == 0) s_mark = 0xffffffffu;
     __syncthreads();
     if(mark != 0xffffffffu) atomicMin(&s_mark, mark);
     __syncthreads();
     const uint32_t m = s_mark;
-    // kept: before the marker and not a zero stuffed after 0xff
-    uint32_t keep = 0;
-    for(int j = 0; j < 4; j++)
-    {
-      const uint32_t i = i0 + j;
-      if(i < len && i < m && !(by[j + 1] == 0 && by[j] == 0xff && i > 0)) keep |= 1u << j;
-    }
-    // exclusive scan of the kept counts over the work group
-    uint32_t c = __popc(keep);
-    s_sum[t] = c;
+    if(m < i0 + 16) keep &= m > i0 ? (1u << (m - i0)) - 1 : 0u;      // kept: before the first marker
+    const uint32_t c = __popc(keep), lead = kept & 3;
+    uint32_t all;
+    uint32_t at = lead + lj92_scan256(c, ws, all) - c;
+#pragma unroll
+    for(int j = 0; j < 16; j++)
+      if(keep & (1u << j)) ob[at++] = (uint8_t)(x[j / 4] >> (8 * (j % 4)));
     __syncthreads();
-    for(int o = 1; o < 256; o <<= 1)
-    {
-      const uint32_t v = t >= (uint32_t)o ? s_sum[t - o] : 0u;
-      __syncthreads();
-      s_sum[t] += v;
-      __syncthreads();
-    }
-    uint32_t at = kept + s_sum[t] - c;
-    for(int j = 0; j < 4; j++)
-      if(keep & (1u << j)) lj92_st(dst + at++, (uint8_t)by[j + 1]);
-    kept += s_sum[255];
+    const uint32_t nw = (lead + all) / 4;
+    for(uint32_t k = t; k < nw; k += 256) lj92_st(dst + kept / 4 + k, out[k]);
+    kept += all;
     ended = m != 0xffffffffu;
+    const uint32_t rest = out[nw];
     __syncthreads();
+    if(t == 0) out[0] = rest;                          // the bytes of the partial word
   }
-  // zeros after the data up to the end of the clean region
-  for(uint32_t i = kept + t; i < p.cwords * 4; i += 256) lj92_st(dst + i, (uint8_t)0);
+  __syncthreads();
+  // the partial word, then zeros up to the end of the clean region
+  if(t == 0 && (kept & 3)) lj92_st(dst + kept / 4, out[0] & ((1u << (8 * (kept & 3))) - 1));
+  for(uint32_t k = (kept + 3) / 4 + t; k < p.cwords; k += 256) lj92_st(dst + k, 0u);
   if(t == 0) nbits[blockIdx.x] = kept * 8;
 }
 
-__global__ void __launch_bounds__(256) k_lj92_first(const lj92_pst *ps, int np, uint32_t ntot, const uint32_t *nbits,
-                                                    uint32_t *start, uint32_t *end, uint32_t *cnt)
+// the words of a work group's subsequences in LDS, most significant byte
+// first, one word of padding after a subsequence's (the lanes of a wave then
+// read different banks); a few more for the last lane's look-ahead.  e: the
+// symbol at the next LJ92_WIDE bits, code length | category << 5 | bits taken
+// << 10, LJ92_NONE (one bit taken, no symbol) where no code matches and 0 where
+// the code is longer
+#define LJ92_WIDE 11
+#define LJ92_NONE (31u | (1u << 10))
+#define LJ92_LW (256 * LJ92_SW + 4)
+struct lj92_lds
 {
-  const uint32_t g = blockIdx.x * 256 + threadIdx.x;
-  if(g >= ntot) return;
-  const int i = lj92_find(ps, np, g, false);
-  const lj92_pst &p = ps[i];
-  const uint32_t k = g - p.sbase, B = nbits[i];
-  const uint32_t s0 = k * LJ92_SUB, lim = min(s0 + LJ92_SUB, B);
-  uint32_t n;
-  start[g] = s0;
-  end[g] = lj92_count(p, s0, lim, n);
-  cnt[g] = n;
+  lj92_tab tab;
+  uint16_t e[1 << LJ92_WIDE];
+  uint32_t w[LJ92_LW + LJ92_LW / LJ92_SW + 1];
+};
+
+// code length and category of the symbol at the top of window x; length 0
+// where no code matches
+__device__ static inline int lj92_code(const lj92_tab &t, uint32_t x, int &cat)
+{
+  const uint16_t f = t.fast[x >> (32 - LJ92_FAST)];
+  cat = f >> 8;
+  if(f) return f & 0xff;
+  for(int l = LJ92_FAST + 1; l <= 16; l++)
+  {
+    const int code = (int)(x >> (32 - l));
+    if(code <= t.maxcode[l])
+    {
+      cat = t.val[code + t.delta[l]];
+      return l;
+    }
+  }
+  return 0;
 }
 
-__global__ void __launch_bounds__(256) k_lj92_sync(const lj92_pst *ps, int np, uint32_t ntot, const uint32_t *nbits,
-                                                   uint32_t *start, const uint32_t *end_in, uint32_t *end_out,
-                                                   uint32_t *cnt, int *changed)
+__device__ static inline uint32_t lj92_entry(int len, int cat)
 {
-  const uint32_t g = blockIdx.x * 256 + threadIdx.x;
-  if(g >= ntot) return;
-  const int i = lj92_find(ps, np, g, false);
+  return len ? (uint32_t)(len | (cat << 5) | ((len + (cat == 16 ? 0 : cat)) << 10)) : LJ92_NONE;
+}
+
+__device__ static inline void lj92_stage(lj92_lds &l, const lj92_pst &p, uint32_t w0)
+{
+  const uint32_t *src = (const uint32_t *)p.tab;
+  for(uint32_t k = threadIdx.x; k < sizeof(lj92_tab) / 4; k += 256) ((uint32_t *)&l.tab)[k] = lj92_ld(src + k);
+  // 16-byte loads, all in flight (the clean region is whole 16-byte groups)
+  constexpr int N = (LJ92_LW / 4 + 255) / 256;
+  lj92_u32x4 v[N];
+#pragma unroll
+  for(int j = 0; j < N; j++)
+  {
+    const uint32_t k = 4 * (threadIdx.x + 256 * j);
+    v[j] = lj92_u32x4{ 0, 0, 0, 0 };
+    if(k < LJ92_LW && w0 + k < p.cwords) v[j] = lj92_ld((const lj92_u32x4 *)(p.clean + w0 + k));
+  }
+#pragma unroll
+  for(int j = 0; j < N; j++)
+  {
+    const uint32_t k = 4 * (threadIdx.x + 256 * j);
+    if(k < LJ92_LW)
+#pragma unroll
+      for(int i = 0; i < 4; i++) l.w[k + i + k / LJ92_SW] = lj92_bswap(v[j][i]);
+  }
+  __syncthreads();
+  // canonical codes fill the code space from 0 without gaps: past their end
+  // (left-justified to 16 bits) nothing matches
+  int end = 0;
+#pragma unroll
+  for(int b = 1; b <= 16; b++) end = max(end, (l.tab.maxcode[b] + 1) << (16 - b));
+  for(uint32_t k = threadIdx.x; k < (1 << LJ92_WIDE); k += 256)
+  {
+    int cat;
+    const int len = lj92_code(l.tab, k << (32 - LJ92_WIDE), cat);
+    const bool none = (int)(k << (16 - LJ92_WIDE)) >= end;
+    l.e[k] = (uint16_t)(none ? LJ92_NONE : len && len <= LJ92_WIDE ? lj92_entry(len, cat) : 0u);
+  }
+  __syncthreads();
+}
+
+// 32 bits from bit position rel, counted from the first staged word and below
+// 32 (LJ92_LW - 1)
+__device__ static inline uint32_t lj92_window(const lj92_lds &l, uint32_t rel)
+{
+  const uint32_t a = rel >> 5, b = a + 1;
+  return (uint32_t)((((uint64_t)l.w[a + a / LJ92_SW] << 32) | l.w[b + b / LJ92_SW]) >> (32 - (rel & 31)));
+}
+
+// the symbol at window x as lj92_entry, LJ92_NONE where none is: a table
+// look-up, or the canonical search for long codes
+__device__ static inline uint32_t lj92_sym(const lj92_lds &l, uint32_t x)
+{
+  uint32_t e = l.e[x >> (32 - LJ92_WIDE)];
+  if(!e)
+  {
+    int cat;
+    const int len = lj92_code(l.tab, x, cat);
+    e = lj92_entry(len, cat);
+  }
+  return e;
+}
+
+__global__ void __launch_bounds__(256) k_lj92_first(const lj92_pst *ps, int np, const uint32_t *nbits, uint32_t *start,
+                                                    uint32_t *end, uint32_t *cnt)
+{
+  __shared__ lj92_lds l;
+  __shared__ uint32_t on[256 * (LJ92_SW + 1)];   // symbol starts of each lane's first decode, a bit a position
+  __shared__ uint32_t s_end[256];
+  const int i = lj92_find(ps, np, blockIdx.x, &lj92_pst::bbase);
   const lj92_pst &p = ps[i];
-  const uint32_t k = g - p.sbase;
-  const uint32_t e = end_in[g];
+  const int t = threadIdx.x;
+  const uint32_t kb = (blockIdx.x - p.bbase) * LJ92_OWN, B = nbits[i];
+  const uint32_t k0 = kb ? kb - LJ92_WARM : 0, own0 = kb ? LJ92_WARM : 0;
+  const uint32_t k = k0 + t, s0 = k * LJ92_SUB, lim = min(s0 + LJ92_SUB, B);
+  const bool live = k < p.K && s0 < B;
+  lj92_stage(l, p, k0 * LJ92_SW);
+  uint32_t *my = on + t * (LJ92_SW + 1);
+  for(int j = 0; j < LJ92_SW; j++) my[j] = 0;
+  const uint32_t bit0 = k0 * LJ92_SUB;
+  uint32_t st = s0, en = s0, n = 0, en0;
+  if(live)
+  {
+    uint32_t pos = s0, word = 0, cur = 0;
+    while(pos < lim)
+    {
+      const uint32_t r = pos - s0;
+      if((r >> 5) != word) { my[word] = cur; cur = 0; word = r >> 5; }
+      const uint32_t e = lj92_sym(l, lj92_window(l, pos - bit0)), ok = (e & 31) != 31;
+      cur |= ok << (r & 31);
+      pos += e >> 10;
+      n += ok;
+    }
+    my[word] = cur;
+    en = pos;
+  }
+  en0 = en;
+  s_end[t] = en;
+  // each round a lane at least settles, so 256 rounds end it; a decode from
+  // another start mostly falls into the first one's positions after a few
+  // symbols, and from there on its count and end are known
+  for(int round = 0; round < 256; round++)
+  {
+    __syncthreads();
+    const uint32_t ns = live && t > 0 ? s_end[t - 1] : st;
+    const bool moved = ns != st;
+    if(moved)
+    {
+      st = ns;
+      uint32_t pos = ns;
+      n = 0;
+      en = ns;
+      if(pos < lim)
+      {
+        bool met = false;
+        while(pos < lim)
+        {
+          const uint32_t r = pos - s0;
+          if((my[r >> 5] >> (r & 31)) & 1) { met = true; break; }
+          const uint32_t e = lj92_sym(l, lj92_window(l, pos - bit0));
+          pos += e >> 10;
+          n += (e & 31) != 31;
+        }
+        en = pos;
+        if(met)
+        {
+          const uint32_t r = pos - s0;
+          n += __popc(my[r >> 5] >> (r & 31));
+          for(uint32_t j = (r >> 5) + 1; j < LJ92_SW; j++) n += __popc(my[j]);
+          en = en0;
+        }
+      }
+    }
+    if(!__syncthreads_or(moved)) break;
+    s_end[t] = en;
+  }
+  if(t >= (int)own0 && t < (int)own0 + LJ92_OWN && k < p.K)
+  {
+    start[p.sbase + k] = st;
+    end[p.sbase + k] = en;
+    cnt[p.sbase + k] = n;
+  }
+}
+
+__global__ void __launch_bounds__(256) k_lj92_sync(const lj92_pst *ps, int np, const uint32_t *nbits, uint32_t *start,
+                                                   const uint32_t *end_in, uint32_t *end_out, uint32_t *cnt, int *changed)
+{
+  const int i = lj92_find(ps, np, blockIdx.x, &lj92_pst::bbase);
+  const lj92_pst &p = ps[i];
+  const uint32_t k = (blockIdx.x - p.bbase) * LJ92_OWN + threadIdx.x;
+  if(threadIdx.x >= LJ92_OWN || k >= p.K) return;
+  const uint32_t g = p.sbase + k, e = end_in[g];
   // past the data a subsequence holds no symbol whatever its start: left alone,
   // it does not hand a changed start down the rest of the stream one round at a time
   if(k == 0 || end_in[g - 1] == start[g] || k * LJ92_SUB >= nbits[i]) { end_out[g] = e; return; }
@@ -656,7 +871,7 @@ __global__ void __launch_bounds__(256) k_lj92_sync(const lj92_pst *ps, int np, u
 
 __global__ void __launch_bounds__(256) k_lj92_scan(const lj92_pst *ps, const uint32_t *cnt, uint32_t *off)
 {
-  __shared__ uint32_t s_sum[256];
+  __shared__ uint32_t ws[4];
   const lj92_pst &p = ps[blockIdx.x];
   const uint32_t t = threadIdx.x;
   uint32_t carry = 0;
@@ -664,48 +879,43 @@ __global__ void __launch_bounds__(256) k_lj92_scan(const lj92_pst *ps, const uin
   {
     const uint32_t k = k0 + t;
     const uint32_t c = k < p.K ? cnt[p.sbase + k] : 0u;
-    s_sum[t] = c;
-    __syncthreads();
-    for(int o = 1; o < 256; o <<= 1)
-    {
-      const uint32_t v = t >= (uint32_t)o ? s_sum[t - o] : 0u;
-      __syncthreads();
-      s_sum[t] += v;
-      __syncthreads();
-    }
-    if(k < p.K) off[p.sbase + k] = carry + s_sum[t] - c;
-    carry += s_sum[255];
-    __syncthreads();
+    uint32_t all;
+    const uint32_t inc = lj92_scan256(c, ws, all);
+    if(k < p.K) off[p.sbase + k] = carry + inc - c;
+    carry += all;
   }
 }
 
-__global__ void __launch_bounds__(256) k_lj92_write(const lj92_pst *ps, int np, uint32_t ntot, const uint32_t *nbits,
+__global__ void __launch_bounds__(256) k_lj92_write(const lj92_pst *ps, int np, const uint32_t *nbits,
                                                     const uint32_t *start, const uint32_t *off, int *status)
 {
-  const uint32_t g = blockIdx.x * 256 + threadIdx.x;
-  if(g >= ntot) return;
-  const int i = lj92_find(ps, np, g, false);
+  __shared__ lj92_lds l;
+  const int i = lj92_find(ps, np, blockIdx.x, &lj92_pst::bbase);
   const lj92_pst &p = ps[i];
-  const uint32_t k = g - p.sbase, B = nbits[i];
+  const uint32_t kb = (blockIdx.x - p.bbase) * LJ92_OWN, k = kb + threadIdx.x, B = nbits[i];
+  lj92_stage(l, p, kb * LJ92_SW);
+  if(threadIdx.x >= LJ92_OWN || k >= p.K) return;
+  const uint32_t g = p.sbase + k;
   const uint32_t kreal = (B + LJ92_SUB - 1) / LJ92_SUB;
   const bool tail = k == (kreal ? kreal - 1 : 0);     // continues to the scan's last sample
   uint32_t pos = start[g];
   const uint32_t lim = min(k * LJ92_SUB + LJ92_SUB, B);
   uint32_t o = off[g];
   if(!(pos < lim || tail) || o >= p.S) return;
-  lj92_cbits b;
-  lj92_cinit(b, p, pos);
-  const lj92_tab *t = p.tab;
   uint16_t *diff = p.diff;
   // samples up to a multiple of four one by one, then four to a store
   uint64_t pack = 0;
   int npk = 0;
   while((pos < lim || tail) && o < p.S)
   {
-    int used, ok;
-    const int d = lj92_csym(b, t, used, ok);
-    pos += used;
-    if(!ok) { atomicAdd(status, 1); return; }      // a sample of the scan with no valid code
+    // a tail runs on into the zeros after the data, which reach past the staged words
+    const uint32_t x = lj92_window(l, min(pos - kb * LJ92_SUB, 32u * (LJ92_LW - 2))), e = lj92_sym(l, x);
+    if((e & 31) == 31) { atomicAdd(status, 1); return; }      // a sample of the scan with no valid code
+    pos += e >> 10;
+    const uint32_t len = e & 31, cat = (e >> 5) & 31;
+    // the category's bits; a leading zero marks a negative difference
+    int d = cat == 16 ? 32768 : (int)(((x << len) >> 1) >> (31 - cat));
+    if(cat < 16 && d < (1 << cat) >> 1) d -= (1 << cat) - 1;
     if(npk == 0 && (o & 3)) lj92_st(diff + o, (uint16_t)d);
     else
     {
@@ -764,7 +974,7 @@ __global__ void __launch_bounds__(256) k_lj92_rows(const lj92_pst *ps, int np, u
 {
   const uint32_t g = blockIdx.x * 256 + threadIdx.x;
   if(g >= nrows) return;
-  const int i = lj92_find(ps, np, g, true);
+  const int i = lj92_find(ps, np, g, &lj92_pst::rbase);
   const lj92_pst &p = ps[i];
   const int r = g - p.rbase, C = p.comp, L = p.fwd * C;
   const uint16_t *d = p.diff + (size_t)r * L;
@@ -793,82 +1003,130 @@ __global__ void __launch_bounds__(256) k_lj92_rows(const lj92_pst *ps, int np, u
   }
 }
 
-// one wave per scan line where the components are 1, 2 or 4 (every lane's
-// four samples start at component 0): coalesced loads of four differences a
-// lane, their sums per component scanned over the wave in 16-bit lanes, the
-// first column's values in place of its differences
-__device__ static inline uint64_t lj92_shfl_up(uint64_t v, int d)
+// LJ92_WROWS scan lines a wave where the components are 1, 2 or 4 (every
+// lane's four samples start at component 0): coalesced loads of four
+// differences a lane, all lines' in flight, their sums per component scanned
+// over the wave in packed 16-bit adds, the first column's values in place of
+// its differences.  A line a wave spent most of its time finding its stream:
+// 89 us for 24 MP in 384 tiles, 96 MB moved.
+typedef unsigned short lj92_us2 __attribute__((ext_vector_type(2)));
+
+__device__ static inline lj92_us2 lj92_dpp_add(lj92_us2 v, uint32_t o)
 {
-  const uint32_t lo = __shfl_up((uint32_t)v, d), hi = __shfl_up((uint32_t)(v >> 32), d);
-  return ((uint64_t)hi << 32) | lo;
+  return v + __builtin_bit_cast(lj92_us2, o);
 }
 
-__global__ void __launch_bounds__(256) k_lj92_rows4(const lj92_pst *ps, int np, uint32_t nrows)
+// inclusive sum over the wave: by rows of 16, then across them (lanes with
+// no source add 0)
+__device__ static inline lj92_us2 lj92_wave_scan(lj92_us2 v)
 {
-  const uint32_t g = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if(g >= nrows) return;                               // whole waves: g is uniform in a wave
-  const int i = lj92_find(ps, np, g, true);
-  const lj92_pst &p = ps[i];
-  const int r = g - p.rbase, C = p.comp, L = p.fwd * C;
-  const uint16_t *d = p.diff + (size_t)r * L;
-  const uint64_t c0 = lj92_ld(p.col0 + r);
+#define LJ92_DPP(ctrl, rows) \
+  v = lj92_dpp_add(v, (uint32_t)__builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, rows, 0xf, false))
+  LJ92_DPP(0x111, 0xf);   // row_shr 1, 2, 4, 8
+  LJ92_DPP(0x112, 0xf);
+  LJ92_DPP(0x114, 0xf);
+  LJ92_DPP(0x118, 0xf);
+  LJ92_DPP(0x142, 0xa);   // row_bcast 15: rows 1 and 3
+  LJ92_DPP(0x143, 0xc);   // row_bcast 31: rows 2 and 3
+#undef LJ92_DPP
+  return v;
+}
+
+// C components: 1 (sums in the low half), 2, or 4 (components 2 and 3 in hi)
+template<int C>
+__device__ static inline void lj92_row_group(const lj92_pst &p, int r0, int lane)
+{
+  const int L = p.fwd * C, nr = min(LJ92_WROWS, p.fht - r0);
   const bool direct = L == p.tile_wd && p.x0 >= 0 && p.x0 + p.tile_wd <= p.img_wd;   // scan line = tile line inside the window
-  const long s0 = (long)r * L;
-  const int ty0 = (int)(s0 / p.tile_wd);
   const bool wide = (L & 3) == 0;                      // lines start on 8-byte boundaries of the differences
-  uint64_t carry = 0;
+  lj92_us2 lo[LJ92_WROWS] = {}, hi[LJ92_WROWS] = {};   // the sums before this chunk
+  uint64_t c0[LJ92_WROWS];
+#pragma unroll
+  for(int q = 0; q < LJ92_WROWS; q++) c0[q] = q < nr ? lj92_ld(p.col0 + r0 + q) : 0ull;
   for(int k0 = 0; k0 < L; k0 += 256)
   {
     const int k = k0 + 4 * lane;
-    uint32_t dd[4];
-    if(wide && k + 3 < L)
+    uint64_t dd[LJ92_WROWS];
+#pragma unroll
+    for(int q = 0; q < LJ92_WROWS; q++)
     {
-      const uint64_t w = lj92_ld((const uint64_t *)(d + k));
-      for(int j = 0; j < 4; j++) dd[j] = (uint32_t)(w >> (16 * j)) & 0xffff;
+      const uint16_t *d = p.diff + (size_t)(r0 + q) * L;
+      dd[q] = 0;
+      if(q >= nr) continue;
+      if(wide) { if(k < L) dd[q] = lj92_ld((const uint64_t *)(d + k)); }
+      else
+        for(int j = 0; j < 4; j++)
+          if(k + j < L) dd[q] |= (uint64_t)lj92_ld(d + k + j) << (16 * j);
     }
-    else
-      for(int j = 0; j < 4; j++) dd[j] = k + j < L ? lj92_ld(d + k + j) : 0u;
-    for(int j = 0; j < 4; j++)
-      if(k + j < C) dd[j] = (uint32_t)(c0 >> (16 * (k + j))) & 0xffff;
-    uint64_t loc = 0;
-    for(int j = 0; j < 4; j++) loc = lj92_add4(loc, (uint64_t)dd[j] << (16 * (j % C)));
-    uint64_t inc = loc;
-    for(int o = 1; o < 64; o <<= 1)
+#pragma unroll
+    for(int q = 0; q < LJ92_WROWS; q++)
     {
-      const uint64_t y = lj92_shfl_up(inc, o);
-      if(lane >= o) inc = lj92_add4(inc, y);
-    }
-    uint64_t run = lj92_shfl_up(inc, 1);
-    run = lj92_add4(carry, lane ? run : 0ull);
-    const uint64_t last = __shfl(inc, 63);
-    carry = lj92_add4(carry, last);
-    uint32_t v4[4];
-    for(int j = 0; j < 4; j++)
-    {
-      const int c = j % C;
-      run = lj92_add4(run, (uint64_t)dd[j] << (16 * c));
-      v4[j] = ((uint32_t)(run >> (16 * c)) & 0xffff) << p.pt;
-    }
-    uint16_t *dst = p.out + (long)(p.y0 + ty0) * p.pitch + p.x0 + k;
-    if(direct && k + 3 < L && p.y0 + ty0 >= 0 && p.y0 + ty0 < p.img_ht && ((uintptr_t)dst & 7) == 0)
-    {
-      lj92_st((uint64_t *)dst, (uint64_t)(v4[0] & 0xffff) | ((uint64_t)(v4[1] & 0xffff) << 16) |
-                                ((uint64_t)(v4[2] & 0xffff) << 32) | ((uint64_t)(v4[3] & 0xffff) << 48));
-      continue;
-    }
-    for(int j = 0; j < 4; j++)
-    {
-      const int kk = k + j;
-      if(kk >= L) break;
-      const uint32_t v = v4[j];
-      int tx, ty;
-      if(direct) { tx = kk; ty = ty0; }
-      else { const long sm = s0 + kk; tx = (int)(sm % p.tile_wd); ty = (int)(sm / p.tile_wd); }
-      if(p.y0 + ty >= 0 && p.y0 + ty < p.img_ht && p.x0 + tx >= 0 && p.x0 + tx < p.img_wd)
-        lj92_st(p.out + (long)(p.y0 + ty) * p.pitch + p.x0 + tx, (uint16_t)v);
+      if(q >= nr) continue;
+      uint32_t e[4];
+#pragma unroll
+      for(int j = 0; j < 4; j++)
+      {
+        e[j] = (uint32_t)(dd[q] >> (16 * j)) & 0xffff;
+        if(k + j < C) e[j] = (uint32_t)(c0[q] >> (16 * (k + j))) & 0xffff;
+      }
+      // each sample's sum within the lane, and the lane's total
+      lj92_us2 a[4], b[4], sl = { 0, 0 }, sh = { 0, 0 };
+#pragma unroll
+      for(int j = 0; j < 4; j++)
+      {
+        const int c = j % C;
+        if(c < 2) sl += lj92_us2{ (unsigned short)(c == 0 ? e[j] : 0), (unsigned short)(c == 1 ? e[j] : 0) };
+        else sh += lj92_us2{ (unsigned short)(c == 2 ? e[j] : 0), (unsigned short)(c == 3 ? e[j] : 0) };
+        a[j] = sl; b[j] = sh;
+      }
+      const lj92_us2 il = lj92_wave_scan(sl), ol = lo[q] + (il - sl);
+      lj92_us2 oh = hi[q];
+      if(C == 4)
+      {
+        const lj92_us2 ih = lj92_wave_scan(sh);
+        oh = hi[q] + (ih - sh);
+        hi[q] += __builtin_bit_cast(lj92_us2, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ih), 63));
+      }
+      lo[q] += __builtin_bit_cast(lj92_us2, __builtin_amdgcn_readlane(__builtin_bit_cast(int, il), 63));
+      uint32_t v4[4];
+#pragma unroll
+      for(int j = 0; j < 4; j++)
+      {
+        const int c = j % C;
+        const lj92_us2 v = c < 2 ? ol + a[j] : oh + b[j];
+        v4[j] = ((uint32_t)v[c & 1] << p.pt) & 0xffff;
+      }
+      const long s0 = (long)(r0 + q) * L;
+      const int ty0 = direct ? r0 + q : 0;
+      uint16_t *dst = p.out + (long)(p.y0 + ty0) * p.pitch + p.x0 + k;
+      if(direct && k + 3 < L && p.y0 + ty0 >= 0 && p.y0 + ty0 < p.img_ht && ((uintptr_t)dst & 7) == 0)
+      {
+        lj92_st((uint64_t *)dst, (uint64_t)(v4[0] | (v4[1] << 16)) | ((uint64_t)(v4[2] | (v4[3] << 16)) << 32));
+        continue;
+      }
+      for(int j = 0; j < 4; j++)
+      {
+        const int kk = k + j;
+        if(kk >= L) break;
+        int tx, ty;
+        if(direct) { tx = kk; ty = ty0; }
+        else { const long sm = s0 + kk; tx = (int)(sm % p.tile_wd); ty = (int)(sm / p.tile_wd); }
+        if(p.y0 + ty >= 0 && p.y0 + ty < p.img_ht && p.x0 + tx >= 0 && p.x0 + tx < p.img_wd)
+          lj92_st(p.out + (long)(p.y0 + ty) * p.pitch + p.x0 + tx, (uint16_t)v4[j]);
+      }
     }
   }
+}
+
+__global__ void __launch_bounds__(256) k_lj92_rows4(const lj92_pst *ps, int np, uint32_t ngroups)
+{
+  const uint32_t g = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if(g >= ngroups) return;                               // whole waves: g is uniform in a wave
+  const lj92_pst &p = ps[lj92_find(ps, np, g, &lj92_pst::qbase)];
+  const int r0 = (int)(g - p.qbase) * LJ92_WROWS, lane = threadIdx.x & 63;
+  if(p.comp == 1) lj92_row_group<1>(p, r0, lane);
+  else if(p.comp == 2) lj92_row_group<2>(p, r0, lane);
+  else lj92_row_group<4>(p, r0, lane);
 }
 
 __global__ void k_lj92_zero(int *p, int n)
@@ -968,7 +1226,7 @@ extern "C" int vkdt_hip_lj92_decode(const uint8_t *data, size_t data_len, const 
   const int nser = n - count[4], npar = count[4];
   // the many-lanes streams: subsequences, scan lines, clean words, samples
   std::vector<lj92_pst> pst(npar);
-  size_t nsub = 0, nrows = 0, cwords = 0, nsamp = 0, maxk = 0;
+  size_t nsub = 0, nblk = 0, nrows = 0, nquad = 0, cwords = 0, nsamp = 0, maxk = 0;
   bool all124 = true;                             // scan lines by waves (k_lj92_rows4)
   for(int i = 0, q = 0; i < n; i++)
   {
@@ -981,7 +1239,9 @@ extern "C" int vkdt_hip_lj92_decode(const uint8_t *data, size_t data_len, const 
     p.cwords = (uint32_t)(((size_t)p.len + 16 + 15) / 16 * 4);
     p.S = (uint32_t)((size_t)h.wd * h.ht * h.comp);
     p.sbase = (uint32_t)nsub; nsub += p.K;
+    p.bbase = (uint32_t)nblk; nblk += (p.K + LJ92_OWN - 1) / LJ92_OWN;
     p.rbase = (uint32_t)nrows; nrows += h.ht;
+    p.qbase = (uint32_t)nquad; nquad += (h.ht + LJ92_WROWS - 1) / LJ92_WROWS;
     maxk = p.K > maxk ? p.K : maxk;
     all124 &= h.comp != 3;
     cwords += p.cwords;
@@ -1011,9 +1271,10 @@ extern "C" int vkdt_hip_lj92_decode(const uint8_t *data, size_t data_len, const 
     if(int e = lj92_table(tables[k].data(), tables[k].data() + 16, &tabs[k])) return e;
   uint8_t *dev = nullptr;
   if(int e = hip_fail(hipMalloc((void **)&dev, total), "lj92 scratch")) return e;
-  // the jobs grouped by kind, then a zero status word; the row caches need
+  // the jobs grouped by kind, then two zero status words (one lane a stream,
+  // many lanes); the row caches need
   // no clearing: the first line reads none
-  std::vector<uint8_t> jobbuf(off_st - off_job + sizeof(int), 0);
+  std::vector<uint8_t> jobbuf(off_st - off_job + 2 * sizeof(int), 0);
   lj92_job *jobs = (lj92_job *)jobbuf.data();
   int first[4], next[4];
   for(int k = 0, f = 0; k < 4; f += count[k++]) first[k] = next[k] = f;
@@ -1065,7 +1326,7 @@ extern "C" int vkdt_hip_lj92_decode(const uint8_t *data, size_t data_len, const 
     err = hip_fail(hipMemcpyAsync(dev + off_pst, pst.data(), sizeof(lj92_pst) * npar, hipMemcpyHostToDevice, s),
                    "lj92 streams");
   const lj92_job *dj = (const lj92_job *)(dev + off_job);
-  int *st = (int *)(dev + off_st);
+  int *st = (int *)(dev + off_st), bad[2] = { 0, 0 };
   for(int k = 0; k < 4 && !err; k++)
   {
     if(!count[k]) continue;
@@ -1083,45 +1344,57 @@ extern "C" int vkdt_hip_lj92_decode(const uint8_t *data, size_t data_len, const 
     uint32_t *sub = (uint32_t *)(dev + off_sub);
     uint32_t *start = sub, *endA = sub + nsub, *endB = sub + 2 * nsub, *cnt = sub + 3 * nsub, *off = sub + 4 * nsub;
     int *flags = (int *)(dev + off_flag);
-    const uint32_t ns = (uint32_t)nsub, nr = (uint32_t)nrows;
-    const dim3 gsub((ns + 255) / 256), grow((nr + 255) / 256), b256(256);
-    hipLaunchKernelGGL(k_lj92_zero, dim3((maxit + 255) / 256), b256, 0, s, flags, maxit);
-    hipLaunchKernelGGL(k_lj92_unstuff, dim3(npar), b256, 0, s, dp, nb);
-    hipLaunchKernelGGL(k_lj92_first, gsub, b256, 0, s, dp, npar, ns, (const uint32_t *)nb, start, endA, cnt);
-    err = launch_post("lj92 first");
-    // resynchronise, two rounds per look at the flags, until a round changes nothing
-    for(int it = 0; it < maxit && !err; it += 2)
-    {
-      int ch[2] = { 1, 1 };
+    const uint32_t nr = (uint32_t)nrows, nq = (uint32_t)nquad;
+    const dim3 gblk((uint32_t)nblk), grow((nr + 255) / 256), b256(256);
+    auto sync2 = [&](int it) {
       for(int u = 0; u < 2 && it + u < maxit; u++)
       {
-        hipLaunchKernelGGL(k_lj92_sync, gsub, b256, 0, s, dp, npar, ns, (const uint32_t *)nb, start,
-                           (const uint32_t *)endA, endB, cnt, flags + it + u);
+        hipLaunchKernelGGL(k_lj92_sync, gblk, b256, 0, s, dp, npar, (const uint32_t *)nb, start, (const uint32_t *)endA, endB,
+                           cnt, flags + it + u);
         uint32_t *tmp = endA; endA = endB; endB = tmp;
       }
-      err = launch_post("lj92 sync");
-      if(!err) err = hip_fail(hipMemcpyAsync(ch, flags + it, sizeof(int) * (it + 1 < maxit ? 2 : 1),
-                                             hipMemcpyDeviceToHost, s), "lj92 sync flags");
-      if(!err) err = hip_fail(hipStreamSynchronize(s), "lj92 sync wait");
-      if(!err && (ch[0] == 0 || (it + 1 < maxit && ch[1] == 0))) break;
-      if(!err && it + 2 >= maxit) err = vkdt_set_error(VKDT_HIP_INCOMPLETE, "lj92: subsequences did not synchronise");
-    }
-    if(!err)
-    {
+    };
+    auto finish = [&]() {
       hipLaunchKernelGGL(k_lj92_scan, dim3(npar), b256, 0, s, dp, (const uint32_t *)cnt, off);
-      hipLaunchKernelGGL(k_lj92_write, gsub, b256, 0, s, dp, npar, ns, (const uint32_t *)nb, (const uint32_t *)start,
-                         (const uint32_t *)off, st);
+      hipLaunchKernelGGL(k_lj92_write, gblk, b256, 0, s, dp, npar, (const uint32_t *)nb, (const uint32_t *)start,
+                         (const uint32_t *)off, st + 1);
       hipLaunchKernelGGL(k_lj92_col0, dim3(npar), b256, 0, s, dp);
-      if(all124) hipLaunchKernelGGL(k_lj92_rows4, dim3((nr + 3) / 4), b256, 0, s, dp, npar, nr);
+      if(all124) hipLaunchKernelGGL(k_lj92_rows4, dim3((nq + 3) / 4), b256, 0, s, dp, npar, nq);
       else hipLaunchKernelGGL(k_lj92_rows, grow, b256, 0, s, dp, npar, nr);
-      err = launch_post("lj92 write");
+      return launch_post("lj92 write");
+    };
+    hipLaunchKernelGGL(k_lj92_zero, dim3((maxit + 255) / 256), b256, 0, s, flags, maxit);
+    hipLaunchKernelGGL(k_lj92_unstuff, dim3(npar), b256, 0, s, dp, nb);
+    hipLaunchKernelGGL(k_lj92_first, gblk, b256, 0, s, dp, npar, (const uint32_t *)nb, start, endA, cnt);
+    // two rounds across the work groups, then on to the samples; the flags are
+    // looked at once those are through, and only where a round still changed
+    // something do further rounds (two per look) and the samples follow again
+    sync2(0);
+    err = finish();
+    int it = 0;
+    for(; !err; it += 2)
+    {
+      int ch[2] = { 0, 0 };
+      err = hip_fail(hipMemcpyAsync(ch, flags + it, sizeof(int) * (it + 1 < maxit ? 2 : 1), hipMemcpyDeviceToHost, s),
+                     "lj92 sync flags");
+      if(!err) err = hip_fail(hipMemcpyAsync(bad, st, sizeof(bad), hipMemcpyDeviceToHost, s), "lj92 status");
+      if(!err) err = hip_fail(hipStreamSynchronize(s), "lj92 sync wait");
+      if(err || ch[0] == 0 || (it + 1 < maxit && ch[1] == 0)) break;
+      if(it + 2 >= maxit) { err = vkdt_set_error(VKDT_HIP_INCOMPLETE, "lj92: subsequences did not synchronise"); break; }
+      sync2(it + 2);
+      err = launch_post("lj92 sync");
+    }
+    if(!err && it > 0)
+    {
+      hipLaunchKernelGGL(k_lj92_zero, dim3(1), b256, 0, s, st + 1, 1);
+      err = finish();
     }
   }
-  int bad = 0;
-  if(!err) err = hip_fail(hipMemcpyAsync(&bad, dev + off_st, sizeof(int), hipMemcpyDeviceToHost, s), "lj92 status");
+  if(!err) err = hip_fail(hipMemcpyAsync(bad, st, sizeof(bad), hipMemcpyDeviceToHost, s), "lj92 status");
   if(!err) err = hip_fail(hipStreamSynchronize(s), "lj92 sync");
   (void)hipFree(dev);
   if(err) return err;
-  if(bad) return vkdt_set_error(VKDT_HIP_INCOMPLETE, "lj92: %d tiles with corrupt entropy-coded data", bad);
+  if(bad[0] + bad[1])
+    return vkdt_set_error(VKDT_HIP_INCOMPLETE, "lj92: %d tiles with corrupt entropy-coded data", bad[0] + bad[1]);
   return VKDT_HIP_OK;
 }
