@@ -74,6 +74,17 @@ def test_batch_equals_plain_graphs(cases, tune):
     check_equal(outs, cases, f"eager tune {tune}")
 
 
+@pytest.mark.parametrize("W,Hh,kw", [(400, 300, dict(numgamma=32)), (320, 200, dict(levels=2)), (320, 200, dict(levels=3)),
+                                     (1200, 24, dict()), (1030, 770, dict(numgamma=4))],
+                         ids=["32-curves", "no-coarse-levels", "3-levels", "flat", "4-curves"])
+def test_coarse_levels_equal_the_plain_graph(tmp_path, hip, W, Hh, kw):
+    """the coarsest pyramid levels, which the batch runs in one work group:
+    few and many curves, pyramids too short to have any, a flat image"""
+    c = plain_and_planned(tmp_path, "bayer", W, Hh, 61, kw)
+    check_equal(batch.develop([c[0]], [c[1]]), [c], f"{W}x{Hh} {kw}")
+    c[0].close()
+
+
 def test_alone_equals_in_the_mix(cases):
     """each image developed in a batch of one equals its plain run too"""
     for i, c in enumerate(cases):

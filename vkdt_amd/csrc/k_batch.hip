@@ -20,7 +20,8 @@
 //                      fix/colour/filmcurv run in registers -> rgba f16
 //   group 7  pyr1      llap/curve + llap/reduce to level 1, fused: the
 //                      full-resolution curve planes exist only in LDS
-//   group 8  pyramid   llap/reduce levels 2.., llap/assemble levels nl-2..1
+//   group 8  pyramid   llap/reduce levels 2.., llap/assemble levels nl-2..1;
+//                      the coarsest levels in one launch (kb_tail)
 //   group 9  final     llap/assemble level 0 + llap/colour, fused: level 0
 //                      planes are re-evaluated from the filmcurv output
 //
@@ -565,7 +566,13 @@ __global__ void __launch_bounds__(256) kb_pyr1(bt_launch L)
   });
 }
 
-// reduce level l from l-1, four outputs per thread (256 x 4 per tile)
+// reduce level l from l-1, four outputs per thread (256 x 4 per tile).  SPLIT:
+// a plane per tile instead of a thread's loop over the planes, for launches of
+// at most LL_SPLIT coarse texels, where that loop's serial loads are all the
+// launch waits for (a 4096 x 2160 frame's levels 3 to 6: 9.2 us each -> 5.4);
+// on larger ones the tiles' set-up costs more than it gains
+#define LL_SPLIT (1 << 18)
+template<int SPLIT>
 __global__ void __launch_bounds__(256) kb_reduce(bt_launch L)
 {
   dimg in, o;
@@ -574,8 +581,16 @@ __global__ void __launch_bounds__(256) kb_reduce(bt_launch L)
     const bt_img &im = L.img[jb.img];
     in = rfl(im.lp[jb.level - 1]); o = rfl(im.lp[jb.level]); planes = rfl(im.ll.num_gamma + 1);
   }, [&](const bt_job &jb, int lt) {
+    dimg i1 = in, o1 = o;
+    if(SPLIT)
+    {
+      const int per = jb.tiles_x * ((o.ht + BY - 1) / BY), pl = lt / per;
+      lt -= pl * per;
+      i1.p = (__half *)in.p + (long)pl * in.pstride;
+      o1.p = (__half *)o.p + (long)pl * o.pstride;
+    }
     const int x0 = ((lt % jb.tiles_x) * BX + threadIdx.x) * 4, y = (lt / jb.tiles_x) * BY + threadIdx.y;
-    if(x0 < o.wd && y < o.ht) ll_reduce_px4(in, o, planes, x0, y, 2 | 4);
+    if(x0 < o.wd && y < o.ht) ll_reduce_px4(i1, o1, SPLIT ? 1 : planes, x0, y, 2 | 4);
   });
 }
 
@@ -615,6 +630,111 @@ __global__ void __launch_bounds__(256) kb_asm(bt_launch L)
       if(x < fine.wd && y < fine.ht) st_h1(o, x, y, res[k]);
     }
   });
+}
+
+// the same a texel a thread, reading the coarse footprint straight from
+// memory, for launches of at most LL_SMALL texels (as k_ll_assemble_small:
+// staging the planes in LDS costs those several dependent round trips)
+__global__ void __launch_bounds__(256) kb_asm_small(bt_launch L)
+{
+  __shared__ ll_args a;
+  dimg fine, l1, coarse, o;
+  int first = 0;
+  bt_tiles(L, [&](const bt_job &jb) {
+    const bt_img &im = L.img[jb.img];
+    const int l = jb.level;
+    lds_copy(a, im.ll);
+    first = rfl((int)(l == im.nl - 2));
+    fine = rfl(im.lp[l]); l1 = rfl(im.lp[l + 1]); coarse = rfl(first ? im.lp[l + 1] : im.la[l + 1]); o = rfl(im.la[l]);
+  }, [&](const bt_job &jb, int lt) {
+    const int x = (lt % jb.tiles_x) * BX + threadIdx.x, y = (lt / jb.tiles_x) * BY + threadIdx.y;
+    if(x >= fine.wd || y >= fine.ht) return;
+    st_h1(o, x, y, ll_assemble_direct(a, first, l1.wd, l1.ht, x, y, [&](int p) { return ld_h1(fine, x, y, p); },
+                                      [&](int gx, int gy, int p) { return ld_h1(l1, gx, gy, p); },
+                                      [&](int gx, int gy) { return ld_h1(coarse, gx, gy); }));
+  });
+}
+
+// The coarsest levels of one image in one work group: level T (jb.level) is
+// reduced from T-1 into LDS, the levels below it from LDS to LDS, and the
+// assembles run back up to T; T's planes and reconstruction go to memory, for
+// the assemble of T-1.  Each
+// of these levels was two launches of a few work groups, 8 to 15 us apiece
+// that waited on memory latency.  With the direct and split kernels above a
+// 4096 x 2160 frame takes 777 us instead of 889.  T is the finest level whose
+// planes, with those below, fit LL_TAIL_BYTES (60 KB: 791 us, the one work
+// group then works longer than the launches it saves); the sums
+// are ll_reduce_px's and k_ll_assemble_small's, rounded to binary16 as stored.
+#define LL_TAIL_BYTES (20 * 1024)
+#define LL_TAIL_Y 16
+__global__ void __launch_bounds__(BX * LL_TAIL_Y) kb_tail(bt_launch L)
+{
+  extern __shared__ __half sm[];
+  __shared__ ll_args a;
+  const bt_job jb = rfl(L.job[blockIdx.x]);
+  const bt_img &im = L.img[jb.img];
+  const int tid = threadIdx.y * BX + threadIdx.x, N = BX * LL_TAIL_Y, T = jb.level, nl = rfl(im.nl), G = rfl(im.ll.num_gamma) + 1;
+  for(int i = tid; i < (int)(sizeof(ll_args) / 4); i += N) ((int *)&a)[i] = ((const int *)&im.ll)[i];
+  const dimg src = rfl(im.lp[T - 1]), lo = rfl(im.lp[T]), dst = rfl(im.la[T]);
+  int w = (src.wd - 1) / 2 + 1, h = (src.ht - 1) / 2 + 1;
+  constexpr int U = 4;   // texels whose loads are in flight together
+  for(int i0 = tid; i0 < G * w * h; i0 += U * N)
+  {
+    float v[U];
+    int x[U], y[U], z[U];
+#pragma unroll
+    for(int u = 0; u < U; u++)
+    {
+      const int i = min(i0 + u * N, G * w * h - 1), r = i % (w * h);
+      z[u] = i / (w * h); y[u] = r / w; x[u] = r - y[u] * w;
+      v[u] = ll_reduce_at(src.wd, src.ht, x[u], y[u], [&](int gx, int gy) { return ld_h1(src, gx, gy, z[u]); });
+    }
+#pragma unroll
+    for(int u = 0; u < U; u++)
+      if(i0 + u * N < G * w * h)
+      {
+        sm[i0 + u * N] = f2h(v[u]);
+        st_h1(lo, x[u], y[u], v[u], z[u]);
+      }
+  }
+  // levels T..nl-1 one after the other, then the reconstructions
+  __half *p = sm;
+  for(int l = T + 1; l < nl; l++)
+  {
+    __half *q = p + G * w * h;
+    const int w1 = (w - 1) / 2 + 1, h1 = (h - 1) / 2 + 1;
+    __syncthreads();
+    for(int i = tid; i < G * w1 * h1; i += N)
+    {
+      const int z = i / (w1 * h1), r = i - z * w1 * h1, y = r / w1, x = r - y * w1;
+      q[i] = f2h(ll_reduce_at(w, h, x, y, [&](int gx, int gy) { return h2f(p[(z * h + gy) * w + gx]); }));
+    }
+    p = q;
+    w = w1;
+    h = h1;
+  }
+  __half *rec = p + G * w * h, *coarse = nullptr;
+  for(int l = nl - 2; l >= T; l--)
+  {
+    const int fw = l == T ? dst.wd : rfl(im.lp[l].wd), fh = l == T ? dst.ht : rfl(im.lp[l].ht);
+    const __half *c = p, *f = p - G * fw * fh;
+    const int cw = w, ch = h, first = l == nl - 2;
+    __syncthreads();
+    for(int i = tid; i < fw * fh; i += N)
+    {
+      const int y = i / fw, x = i - y * fw;
+      const float v = ll_assemble_direct(a, first, cw, ch, x, y, [&](int g) { return h2f(f[(g * fh + y) * fw + x]); },
+                                         [&](int gx, int gy, int g) { return h2f(c[(g * ch + gy) * cw + gx]); },
+                                         [&](int gx, int gy) { return h2f(coarse[gy * cw + gx]); });
+      if(l == T) st_h1(dst, x, y, v);
+      else rec[i] = f2h(v);
+    }
+    coarse = rec;
+    rec += fw * fh;
+    p = (__half *)f;
+    w = fw;
+    h = fh;
+  }
 }
 
 // assemble level 0 + llap/colour: level 0 planes from the filmcurv output.
@@ -661,8 +781,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 namespace {
 
 enum kind_t { K_HALF, K_DOWNCOV, K_DOWN, K_DNASM, K_DOUB, K_HL_HALF, K_HL_REDUCE, K_HL_ASM, K_HL_DOUB, K_GAUSS,
-              K_DEVELOP, K_DEVELOP_XT, K_PYR1, K_REDUCE, K_ASM, K_FINAL };
-const int kind_group[] = { 0, 1, 1, 2, 3, 4, 4, 4, 4, 5, 6, 6, 7, 8, 8, 9 };
+              K_DEVELOP, K_DEVELOP_XT, K_PYR1, K_REDUCE, K_REDUCE_SPLIT, K_TAIL, K_ASM_SMALL, K_ASM, K_FINAL };
+const int kind_group[] = { 0, 1, 1, 2, 3, 4, 4, 4, 4, 5, 6, 6, 7, 8, 8, 8, 8, 8, 9 };
 const char *group_name[VKDT_BATCH_STAGES] = { "half", "wavelet", "dnasm", "doub", "hilite", "gauss", "develop",
                                               "pyr1", "pyramid", "final" };
 
@@ -682,6 +802,8 @@ struct dims_t
 {
   int W, H, qw, qh, cw, ch, nl, ng, block;
   int lw[BT_LEVELS], lh[BT_LEVELS];
+  int tail;                            // kb_tail's finest level, nl where it has none
+  size_t tail_lds;                     // and its LDS
   int hl, hn;                          // hilite on, its coarse levels L
   int hw[HL_LEVELS], hh[HL_LEVELS];    // hilite level extents (0: the block grid)
 };
@@ -709,6 +831,16 @@ int image_dims(const vkdt_develop_image_t &d, dims_t &m, int idx)
   m.ng = d.ll_numgamma;
   m.lw[0] = m.W; m.lh[0] = m.H;
   for(int l = 1; l < m.nl; l++) { m.lw[l] = (m.lw[l - 1] - 1) / 2 + 1; m.lh[l] = (m.lh[l - 1] - 1) / 2 + 1; }
+  m.tail = m.nl;
+  m.tail_lds = 0;
+  size_t below = 0;
+  for(int l = m.nl - 1; l >= 2; l--)
+  { // the planes of levels l.., and the reconstructions between
+    const size_t px = (size_t)m.lw[l] * m.lh[l];
+    below += (size_t)(m.ng + 1 + (l < m.nl - 1)) * px * 2;
+    if(below > LL_TAIL_BYTES) break;
+    if(l <= m.nl - 2) { m.tail = l; m.tail_lds = below; }
+  }
   m.hl = d.hl_on != 0;
   m.hn = 0;
   if(m.hl)
@@ -918,7 +1050,9 @@ static int tiles_of(int kind, const dims_t &m, int level, int rows, int &tx)
     case K_GAUSS: w = m.cw; h = m.ch; th = BY * rows; break;
     case K_DEVELOP: case K_DEVELOP_XT: w = m.W; h = m.H; th = BY * DEV_R; break;
     case K_PYR1: w = m.lw[1]; h = m.lh[1]; break;
-    case K_REDUCE: w = m.lw[level]; h = m.lh[level]; tw = 4 * BX; break;
+    case K_REDUCE: case K_REDUCE_SPLIT: w = m.lw[level]; h = m.lh[level]; tw = 4 * BX; break;
+    case K_TAIL: tx = 1; return 1;
+    case K_ASM_SMALL: w = m.lw[level]; h = m.lh[level]; break;
     case K_ASM: w = m.lw[level]; h = m.lh[level]; th = BY * ASM_R; break;
     default: w = m.W; h = m.H; th = BY * ASM_R; break;   // K_FINAL
   }
@@ -938,17 +1072,18 @@ static void build_launches(vkdt_batch_t *b)
     for(int i = 0; i < b->n; i++)
     {
       const dims_t &m = b->dm[i];
-      if(kind == K_REDUCE && level >= m.nl) continue;
-      if(kind == K_ASM && level > m.nl - 2) continue;
+      if((kind == K_REDUCE || kind == K_REDUCE_SPLIT) && level >= std::min(m.nl, m.tail)) continue;
+      if((kind == K_ASM || kind == K_ASM_SMALL) && level > std::min(m.nl - 2, m.tail - 1)) continue;
+      if(kind == K_TAIL && m.tail >= m.nl) continue;
       if(kind == K_DEVELOP && m.block == 3) continue;      // Bayer and X-Trans develop
       if(kind == K_DEVELOP_XT && m.block != 3) continue;   // run as two launches
       if(kind >= K_HL_HALF && kind <= K_HL_DOUB && !m.hl) continue;
       if(kind == K_HL_REDUCE && level > m.hn) continue;
       if(kind == K_HL_ASM && level >= m.hn) continue;
       int tx;
-      const int t = tiles_of(kind, m, level, rows, tx);
+      const int t = tiles_of(kind, m, level, rows, tx) * (kind == K_REDUCE_SPLIT ? m.ng + 1 : 1);
       if(t <= 0) continue;
-      b->job.push_back(bt_job{ i, tx, L.total, level });
+      b->job.push_back(bt_job{ i, tx, L.total, kind == K_TAIL ? m.tail : level });
       L.total += t;
       L.njob++;
     }
@@ -968,8 +1103,19 @@ static void build_launches(vkdt_batch_t *b)
   add(K_DEVELOP, 0, 0);
   add(K_DEVELOP_XT, 0, 0);
   add(K_PYR1, 1, sizeof(__half) * (b->max_ng + 1) * P1_N);
-  for(int l = 2; l < b->max_nl; l++) add(K_REDUCE, l, 0);
-  for(int l = b->max_nl - 2; l >= 1; l--) add(K_ASM, l, asm_lds);
+  // a level's launch by the texels it has over all images
+  auto texels = [&](int l) {
+    size_t n = 0;
+    for(const dims_t &m : b->dm) if(l < m.nl) n += (size_t)m.lw[l] * m.lh[l];
+    return n;
+  };
+  size_t tail_lds = 0;
+  for(const dims_t &m : b->dm) tail_lds = std::max(tail_lds, m.tail_lds);
+  for(int l = 2; l < b->max_nl; l++) add(texels(l) <= LL_SPLIT ? K_REDUCE_SPLIT : K_REDUCE, l, 0);
+  add(K_TAIL, 0, tail_lds);
+  for(int l = b->max_nl - 2; l >= 1; l--)
+    if(texels(l) <= LL_SMALL) add(K_ASM_SMALL, l, 0);
+    else add(K_ASM, l, asm_lds);
   add(K_FINAL, 0, asm_lds);
   b->dirty = 1;
 }
@@ -1053,7 +1199,7 @@ static int enqueue(vkdt_batch_t *b, hipStream_t s, int timed)
     const int persist = tune_persist(b->tune[g]);
     const int rows = is_pixel_stage(L.kind) ? tune_rows(b->tune[g]) : 1;
     bt_launch a = { b->d_img, b->d_job + L.job0, L.njob, L.total, b->d_ctr + L.ctr0, persist, rows };
-    const dim3 grid(persist ? b->ncu * persist : L.total), blk(BX, BY);
+    const dim3 grid(persist && L.kind != K_TAIL ? b->ncu * persist : L.total), blk(BX, BY);
     switch(L.kind)
     {
       case K_HALF:    hipLaunchKernelGGL(kb_half, grid, blk, 0, s, a); break;
@@ -1069,7 +1215,10 @@ static int enqueue(vkdt_batch_t *b, hipStream_t s, int timed)
       case K_DEVELOP: hipLaunchKernelGGL(kb_develop<0>, grid, blk, 0, s, a); break;
       case K_DEVELOP_XT: hipLaunchKernelGGL(kb_develop<1>, grid, blk, 0, s, a); break;
       case K_PYR1:    hipLaunchKernelGGL(kb_pyr1, grid, blk, L.lds, s, a); break;
-      case K_REDUCE:  hipLaunchKernelGGL(kb_reduce, grid, blk, 0, s, a); break;
+      case K_REDUCE:  hipLaunchKernelGGL(kb_reduce<0>, grid, blk, 0, s, a); break;
+      case K_REDUCE_SPLIT: hipLaunchKernelGGL(kb_reduce<1>, grid, blk, 0, s, a); break;
+      case K_TAIL:    hipLaunchKernelGGL(kb_tail, grid, dim3(BX, LL_TAIL_Y), L.lds, s, a); break;
+      case K_ASM_SMALL: hipLaunchKernelGGL(kb_asm_small, grid, blk, 0, s, a); break;
       case K_ASM:     hipLaunchKernelGGL(kb_asm, grid, blk, L.lds, s, a); break;
       default:        hipLaunchKernelGGL(kb_final, grid, blk, L.lds, s, a); break;
     }

@@ -128,46 +128,14 @@ __global__ void __launch_bounds__(256) k_ll_assemble(dimg coarse, dimg l0, dimg 
   }
 }
 
-// The coarse levels, at most LL_SMALL texels: one thread a texel reads its
-// coarse footprint straight from memory (L2 holds these levels) instead of
-// staging the tile's planes in LDS, which costs the tiny levels several
-// dependent memory round trips; the values, weights and the order of the
-// sums are those of ll_assemble_tile, so the result is the same bit for bit.
-#define LL_SMALL (1 << 19)
+// the coarse levels (ll_assemble_direct)
 __global__ void __launch_bounds__(256) k_ll_assemble_small(dimg coarse, dimg l0, dimg l1, dimg out, ll_args a)
 {
   const int x = tid_x(), y = tid_y();
   if(x >= out.wd || y >= out.ht) return;
-  const float v = ld_h1(l0, x, y, a.num_gamma);
-  const int h = gamma_hi_from_v(v, a);
-  const float pv0 = ld_h1(l0, x, y, h - 1), pv1 = ld_h1(l0, x, y, h);
-  const ll_expand_w wx = ll_expand_weights(x & 1), wy = ll_expand_weights(y & 1);
-  const float al = clampf((v - a.gam[h - 1]) / (a.gam[h] - a.gam[h - 1]), 0.0f, 1.0f);
-  float sc[5], s0[5], s1[5];
-#pragma unroll
-  for(int j = 0; j < 5; j++)
-  {
-    const int gy = mirror(y / 2 - 2 + j, l1.ht);
-    float c[5], r0[5], r1[5];
-#pragma unroll
-    for(int i = 0; i < 5; i++)
-    {
-      const int gx = mirror(x / 2 - 2 + i, l1.wd);
-      c[i] = a.first <= 0 ? ld_h1(coarse, gx, gy) : ld_h1(l1, gx, gy, a.num_gamma);
-      r0[i] = ld_h1(l1, gx, gy, h - 1);
-      r1[i] = ld_h1(l1, gx, gy, h);
-    }
-    sc[j] = ll_expand5(wx, c[0], c[1], c[2], c[3], c[4]);
-    s0[j] = ll_expand5(wx, r0[0], r0[1], r0[2], r0[3], r0[4]);
-    s1[j] = ll_expand5(wx, r1[0], r1[1], r1[2], r1[3], r1[4]);
-  }
-  const float rs = 0.25f * ll_expand5(wy, sc[0], sc[1], sc[2], sc[3], sc[4]);
-  const float e0 = 0.25f * ll_expand5(wy, s0[0], s0[1], s0[2], s0[3], s0[4]);
-  const float e1 = 0.25f * ll_expand5(wy, s1[0], s1[1], s1[2], s1[3], s1[4]);
-  const float s = 1.0f / 9.0f;
-  const float lv0 = pv0 - e0 * s;
-  const float lv1 = pv1 - e1 * s;
-  st_h1(out, x, y, rs * s + lv0 * (1.0f - al) + lv1 * al);
+  st_h1(out, x, y, ll_assemble_direct(a, a.first, l1.wd, l1.ht, x, y, [&](int p) { return ld_h1(l0, x, y, p); },
+                                      [&](int gx, int gy, int p) { return ld_h1(l1, gx, gy, p); },
+                                      [&](int gx, int gy) { return ld_h1(coarse, gx, gy); }));
 }
 
 // colour.comp:221-240; output rgba f16 or f32 (f32 when it feeds the export sink)

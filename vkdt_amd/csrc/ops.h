@@ -995,7 +995,19 @@ DEV float ll_lum(float4 t)
 }
 
 // reduce.comp:17-35 (sample_semisoft at 2*o+.5): [1 2 1]/4 x [1 2 1]/4 on
-// texel 2*o, mirrored, for `planes` planes of one output texel
+// texel 2*o, mirrored; at(x, y): the plane of extent wd x ht
+template<typename At>
+DEV float ll_reduce_at(int wd, int ht, int x, int y, At at)
+{
+  const int xm = mirror(2 * x - 1, wd), x0 = mirror(2 * x, wd), xp = mirror(2 * x + 1, wd);
+  const int ym = mirror(2 * y - 1, ht), y0 = mirror(2 * y, ht), yp = mirror(2 * y + 1, ht);
+  const float a = at(xm, ym) + 2.0f * at(x0, ym) + at(xp, ym);
+  const float b = at(xm, y0) + 2.0f * at(x0, y0) + at(xp, y0);
+  const float c = at(xm, yp) + 2.0f * at(x0, yp) + at(xp, yp);
+  return (a + 2.0f * b + c) * (1.0f / 16.0f);
+}
+
+// the same for `planes` planes of one output texel
 DEV void ll_reduce_px(const dimg &in, const dimg &out, int planes, int x, int y)
 {
   const int xm = mirror(2 * x - 1, in.wd), x0 = mirror(2 * x, in.wd), xp = mirror(2 * x + 1, in.wd);
@@ -1208,6 +1220,49 @@ DEV void ll_assemble_tile(const dimg &coarse, const dimg &l1, int owd, int oht, 
     const float lv1 = pv1[k] - e1 * s;
     res[k] = rs * s + lv0 * (1.0f - al) + lv1 * al;
   }
+}
+
+// The coarse levels, at most LL_SMALL texels: one thread a texel reads its
+// coarse footprint straight from memory (L2 holds these levels) instead of
+// staging the tile's planes in LDS, which costs the tiny levels several
+// dependent memory round trips; the values, weights and the order of the
+// sums are those of ll_assemble_tile, so the result is the same bit for bit.
+//   fine(p): the texel's plane p; lo(x, y, p): the coarse planes (extent
+//   cw x ch); rec(x, y): the coarse reconstruction (unused with `first`)
+#define LL_SMALL (1 << 19)
+template<typename Fine, typename Lo, typename Rec>
+DEV float ll_assemble_direct(const ll_args &a, int first, int cw, int ch, int x, int y, Fine fine, Lo lo, Rec rec)
+{
+  const float v = fine(a.num_gamma);
+  const int h = gamma_hi_from_v(v, a);
+  const float pv0 = fine(h - 1), pv1 = fine(h);
+  const ll_expand_w wx = ll_expand_weights(x & 1), wy = ll_expand_weights(y & 1);
+  const float al = clampf((v - a.gam[h - 1]) / (a.gam[h] - a.gam[h - 1]), 0.0f, 1.0f);
+  float sc[5], s0[5], s1[5];
+#pragma unroll
+  for(int j = 0; j < 5; j++)
+  {
+    const int gy = mirror(y / 2 - 2 + j, ch);
+    float c[5], r0[5], r1[5];
+#pragma unroll
+    for(int i = 0; i < 5; i++)
+    {
+      const int gx = mirror(x / 2 - 2 + i, cw);
+      c[i] = first <= 0 ? rec(gx, gy) : lo(gx, gy, a.num_gamma);
+      r0[i] = lo(gx, gy, h - 1);
+      r1[i] = lo(gx, gy, h);
+    }
+    sc[j] = ll_expand5(wx, c[0], c[1], c[2], c[3], c[4]);
+    s0[j] = ll_expand5(wx, r0[0], r0[1], r0[2], r0[3], r0[4]);
+    s1[j] = ll_expand5(wx, r1[0], r1[1], r1[2], r1[3], r1[4]);
+  }
+  const float rs = 0.25f * ll_expand5(wy, sc[0], sc[1], sc[2], sc[3], sc[4]);
+  const float e0 = 0.25f * ll_expand5(wy, s0[0], s0[1], s0[2], s0[3], s0[4]);
+  const float e1 = 0.25f * ll_expand5(wy, s1[0], s1[1], s1[2], s1[3], s1[4]);
+  const float s = 1.0f / 9.0f;
+  const float lv0 = pv0 - e0 * s;
+  const float lv1 = pv1 - e1 * s;
+  return rs * s + lv0 * (1.0f - al) + lv1 * al;
 }
 
 // colour.comp:221-240: black rolloff and luminance transfer
