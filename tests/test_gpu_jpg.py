@@ -110,6 +110,42 @@ def test_strip_and_group_edges(hip, W, Hh, q, hs, vs, dct):
     assert gpu_jpg(hip, img, q, hs, vs, **ex) == oracle_jpg(img, q, hs, vs, dct or 0, 0)
 
 
+def test_threads_and_sizes_share_the_scratch(hip):
+    """encodes and lossless-JPEG decodes of alternating sizes from several
+    threads, each on its own stream: the pooled scratch blocks change hands,
+    every result is the one of a lone call"""
+    import threading
+    from vkdt_amd import lj92
+    rng = np.random.default_rng(9)
+    imgs = [rng.integers(0, 256, (h, w, 3), dtype=np.uint8) // 3 + 60 for h, w in ((40, 56), (200, 300), (8, 8), (500, 700))]
+    want = [oracle_jpg(i, 90, 2, 2) for i in imgs]
+    cfa = rng.integers(0, 4096, (64, 96)).astype(np.uint16)
+    blob, tiles = H.lj92_tiles([lj92.encode(cfa, 14, 1, 1)], 96, 64, 96, 64)
+    errs = []
+
+    def work(k):
+        try:
+            st = H.Stream()
+            out = hip.DeviceBuffer(96, 64, 1, H.FMT_UI16)
+            for r in range(6):
+                i = (k + r) % len(imgs)
+                rgba = np.dstack([imgs[i], np.full(imgs[i].shape[:2], 255, np.uint8)])
+                buf = hip.DeviceBuffer(rgba.shape[1], rgba.shape[0], 4, H.FMT_UI8)
+                buf.upload(rgba, st.ptr)
+                assert H.jpg_encode(buf.ptr, rgba.shape[1], rgba.shape[0], rgba.shape[1], 90, 2, 2, stream=st.ptr) == want[i]
+                buf.free()
+                H.lj92_decode(blob, tiles, [(out.ptr, 96, 64, 96)], st.ptr)
+                assert np.array_equal(out.download(st.ptr), cfa)
+            out.free()
+        except Exception as e:   # noqa: BLE001 -- reported below
+            errs.append((k, repr(e)))
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not errs, errs
+
+
 def test_24mp_timing(hip):
     rng = np.random.default_rng(5)
     W, Hh = 6000, 4000

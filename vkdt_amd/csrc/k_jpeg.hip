@@ -871,6 +871,14 @@ __global__ void k_jpg_zero(uint32_t *p, long n)
   if(i < n) p[i] = 0;
 }
 
+// zeros for the stream's words (total bits, where they fit cap)
+__global__ void __launch_bounds__(256) k_jpg_zero_words(uint4 *w, const uint64_t *total, uint64_t cap)
+{
+  if(*total > cap) return;
+  const uint64_t n = (*total + 127) / 128;
+  for(uint64_t k = (uint64_t)blockIdx.x * 256 + threadIdx.x; k < n; k += (uint64_t)gridDim.x * 256) w[k] = make_uint4(0, 0, 0, 0);
+}
+
 // ---- host ------------------------------------------------------------------
 
 // optimal code lengths (T.81 K.2: the two smallest frequencies merged, ties to
@@ -1026,16 +1034,21 @@ extern "C" int vkdt_hip_jpg_encode_ex(const void *rgba, uint32_t wd, uint32_t ht
   const size_t o_bits = (o_dummy + (smoothing ? nbl : 0) + 255) & ~(size_t)255;
   const size_t o_blen = o_bits + (size_t)(ngroups + 1) * 8;
   const size_t total = o_blen + (size_t)nbl * 2;
-  uint8_t *dev = nullptr;
-  if(int e = hip_fail(hipMalloc((void **)&dev, total), "jpg scratch")) return e;
+  scratch_t sc, st = {};
+  if(int e = scratch_get(sc, total, "jpg scratch")) return e;
+  uint8_t *dev = sc.dev;
   hipStream_t s = (hipStream_t)stream;
   int16_t *coef = (int16_t *)(dev + o_coef);
   uint32_t *freq = (uint32_t *)(dev + o_freq);
   uint64_t *bits = (uint64_t *)(dev + o_bits);
   uint16_t *blen = (uint16_t *)(dev + o_blen);
-  uint8_t *words8 = nullptr, *stuffed = nullptr;
-  int err = hip_fail(hipMemcpyAsync(dev, tables, sizeof(tables), hipMemcpyHostToDevice, s), "jpg tables");
-  std::vector<uint32_t> fr(nfreq);
+  // pinned: tables, then codes | counts | the stream's bits and 0xFF bytes
+  static_assert(sizeof(jpg_codes) + JF_FREQ * 4 * 257 * 4 + 16 <= SCRATCH_PINNED, "pinned staging");
+  jpg_codes *hc = (jpg_codes *)sc.pin;
+  uint32_t *fr = (uint32_t *)(sc.pin + sizeof(jpg_codes));
+  uint64_t *sizes = (uint64_t *)(sc.pin + sizeof(jpg_codes) + JF_FREQ * 4 * 257 * 4);
+  memcpy(sc.pin, tables, sizeof(tables));
+  int err = hip_fail(hipMemcpyAsync(dev, sc.pin, sizeof(tables), hipMemcpyHostToDevice, s), "jpg tables");
   if(!err)
   {
     const int32_t *dq = (const int32_t *)dev;
@@ -1064,65 +1077,71 @@ extern "C" int vkdt_hip_jpg_encode_ex(const void *rgba, uint32_t wd, uint32_t ht
       hipLaunchKernelGGL(k_jpg_dc0, dim3((3 * ntiles + 255) / 256), dim3(256), 0, s, g, (const int16_t *)coef, freq, ntx, ntiles);
     }
     err = launch_post("jpg coefficients");
-    if(!err) err = hip_fail(hipMemcpyAsync(fr.data(), freq, nfreq * 4, hipMemcpyDeviceToHost, s), "jpg counts");
+    if(!err) err = hip_fail(hipMemcpyAsync(fr, freq, nfreq * 4, hipMemcpyDeviceToHost, s), "jpg counts");
     if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
   }
-  for(size_t k = 4 * 257; k < nfreq; k++) fr[k % (4 * 257)] += fr[k];
   uint8_t hb[4][17], hv[4][256];
   int nv[4] = { 0, 0, 0, 0 };
-  jpg_codes hc;
-  memset(&hc, 0, sizeof(hc));
+  const jpg_codes *dhc = (const jpg_codes *)(dev + o_codes);
   if(!err)
   {
+    for(size_t k = 4 * 257; k < nfreq; k++) fr[k % (4 * 257)] += fr[k];
+    memset(hc, 0, sizeof(*hc));
     for(int t = 0; t < 4; t++)
     {
-      jpg_huff(fr.data() + 257 * t, hb[t], hv[t], nv + t);
+      jpg_huff(fr + 257 * t, hb[t], hv[t], nv + t);
       int code = 0, k = 0;
       for(int len = 1; len <= 16; len++)
       {
-        for(int j = 0; j < hb[t][len]; j++, k++) hc.v[t][hv[t][k]] = (uint32_t)code++ | ((uint32_t)len << 16);
+        for(int j = 0; j < hb[t][len]; j++, k++) hc->v[t][hv[t][k]] = (uint32_t)code++ | ((uint32_t)len << 16);
         code <<= 1;
       }
     }
-    err = hip_fail(hipMemcpyAsync(dev + o_codes, &hc, sizeof(hc), hipMemcpyHostToDevice, s), "jpg codes");
+    err = hip_fail(hipMemcpyAsync(dev + o_codes, hc, sizeof(*hc), hipMemcpyHostToDevice, s), "jpg codes");
   }
-  uint64_t nbits = 0;
-  const jpg_codes *dhc = (const jpg_codes *)(dev + o_codes);
   if(!err)
   {
     hipLaunchKernelGGL(k_jpg_code<0>, dim3((unsigned)ngroups), dim3(256), 0, s, g, (const int16_t *)coef, dhc, blen, bits,
                        (uint32_t *)nullptr, (uint64_t)0);
     hipLaunchKernelGGL(k_jpg_scan, dim3(1), dim3(1024), 0, s, bits, ngroups);
     err = launch_post("jpg lengths");
-    if(!err) err = hip_fail(hipMemcpyAsync(&nbits, bits + ngroups, 8, hipMemcpyDeviceToHost, s), "jpg total");
-    if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
   }
-  const long nbytes = (long)((nbits + 7) / 8);
-  const long nwords = (nbytes + 15) / 16 * 4, nchunks = (nbytes + JS_BYTES - 1) / JS_BYTES;
-  uint64_t nff = 0;
-  if(!err)
+  // The stream is written into room for 4 bits a coefficient, so that its
+  // length need not come back first; the kernels leave a longer one alone, and
+  // it is written again into room for its length
+  const uint64_t *tot = bits + ngroups;
+  uint64_t nbits = 0, nff = 0;
+  uint8_t *stuffed = nullptr;
+  size_t cap = (size_t)nbl * 32;
+  for(int pass = 0; pass < 2 && !err; pass++)
   { // words | 0xFF bytes before each chunk, their total | stuffed bytes (at most twice)
+    const long nwords = (long)((cap + 15) / 16 * 4), nchunks = (long)((cap + JS_BYTES - 1) / JS_BYTES);
     const size_t wbytes = ((size_t)nwords * 4 + 255) & ~(size_t)255, cbytes = ((size_t)(nchunks + 1) * 8 + 255) & ~(size_t)255;
-    err = hip_fail(hipMalloc((void **)&words8, wbytes + cbytes + 2 * (size_t)nbytes + 16), "jpg stream");
-    if(!err && nbytes > 0)
-    {
-      uint32_t *words = (uint32_t *)words8;
-      uint64_t *cnt = (uint64_t *)(words8 + wbytes);
-      const uint64_t *tot = bits + ngroups;
-      stuffed = words8 + wbytes + cbytes;
-      hipLaunchKernelGGL(k_jpg_zero, dim3((unsigned)((nwords + 255) / 256)), dim3(256), 0, s, words, nwords);
-      hipLaunchKernelGGL(k_jpg_code<1>, dim3((unsigned)ngroups), dim3(256), 0, s, g, (const int16_t *)coef, dhc, blen, bits, words,
-                         (uint64_t)nwords * 32);
-      hipLaunchKernelGGL(k_stuff_count, dim3((unsigned)nchunks), dim3(256), 0, s, (const uint32_t *)words, tot,
-                         (uint64_t)nwords * 32, cnt);
-      hipLaunchKernelGGL(k_jpg_scan, dim3(1), dim3(1024), 0, s, cnt, (int)nchunks);
-      hipLaunchKernelGGL(k_stuff_scatter, dim3((unsigned)nchunks), dim3(256), 0, s, (const uint32_t *)words, tot,
-                         (uint64_t)nwords * 32, (const uint64_t *)cnt, stuffed);
-      err = launch_post("jpg stuffing");
-      if(!err) err = hip_fail(hipMemcpyAsync(&nff, cnt + nchunks, 8, hipMemcpyDeviceToHost, s), "jpg stuffed");
-      if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
-    }
+    err = scratch_get(st, wbytes + cbytes + 2 * cap + 16, "jpg stream");
+    if(err) break;
+    uint32_t *words = (uint32_t *)st.dev;
+    uint64_t *cnt = (uint64_t *)(st.dev + wbytes);
+    stuffed = st.dev + wbytes + cbytes;
+    hipLaunchKernelGGL(k_jpg_zero_words, dim3((unsigned)std::min((nwords / 4 + 255) / 256, 2048l)), dim3(256), 0, s, (uint4 *)words, tot,
+                       (uint64_t)cap * 8);
+    hipLaunchKernelGGL(k_jpg_code<1>, dim3((unsigned)ngroups), dim3(256), 0, s, g, (const int16_t *)coef, dhc, blen, bits, words,
+                       (uint64_t)cap * 8);
+    hipLaunchKernelGGL(k_stuff_count, dim3((unsigned)nchunks), dim3(256), 0, s, (const uint32_t *)words, tot, (uint64_t)cap * 8, cnt);
+    hipLaunchKernelGGL(k_jpg_scan, dim3(1), dim3(1024), 0, s, cnt, (int)nchunks);
+    hipLaunchKernelGGL(k_stuff_scatter, dim3((unsigned)nchunks), dim3(256), 0, s, (const uint32_t *)words, tot, (uint64_t)cap * 8,
+                       (const uint64_t *)cnt, stuffed);
+    err = launch_post("jpg stuffing");
+    if(!err) err = hip_fail(hipMemcpyAsync(sizes, tot, 8, hipMemcpyDeviceToHost, s), "jpg total");
+    if(!err) err = hip_fail(hipMemcpyAsync(sizes + 1, cnt + nchunks, 8, hipMemcpyDeviceToHost, s), "jpg stuffed");
+    if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
+    if(err) break;
+    nbits = sizes[0];
+    nff = sizes[1];
+    if(nbits <= (uint64_t)cap * 8) break;
+    scratch_put(st, true);
+    cap = (size_t)((nbits + 7) / 8);
   }
+  const size_t nbytes = (size_t)((nbits + 7) / 8);
   out_t o;
   if(!err)
   {
@@ -1159,20 +1178,28 @@ extern "C" int vkdt_hip_jpg_encode_ex(const void *rgba, uint32_t wd, uint32_t ht
     o.w(0xffda); o.w(12); o.b(3);
     o.b(1); o.b(0x00); o.b(2); o.b(0x11); o.b(3); o.b(0x11);
     o.b(0); o.b(63); o.b(0);
-    const size_t head = o.d.size(), body = (size_t)nbytes + (size_t)nff;
-    o.d.resize(head + body);
-    if(body) err = hip_fail(hipMemcpyAsync(o.d.data() + head, stuffed, body, hipMemcpyDeviceToHost, s), "jpg download");
-    if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
-    o.w(0xffd9);
+    // the file in the caller's memory, the stream straight from the device
+    const size_t head = o.d.size(), body = nbytes + (size_t)nff;
+    uint8_t *f = (uint8_t *)malloc(head + body + 2);
+    if(!f) err = vkdt_set_error(VKDT_HIP_OOM, "jpg: out of memory");
+    else
+    {
+      memcpy(f, o.d.data(), head);
+      if(body) err = hip_fail(hipMemcpyAsync(f + head, stuffed, body, hipMemcpyDeviceToHost, s), "jpg download");
+      if(!err) err = hip_fail(hipStreamSynchronize(s), "jpg sync");
+      f[head + body] = 0xff;
+      f[head + body + 1] = 0xd9;
+      if(err) free(f);
+      else
+      {
+        *out = f;
+        *out_len = head + body + 2;
+      }
+    }
   }
-  (void)hipFree(dev);
-  if(words8) (void)hipFree(words8);
-  if(err) return err;
-  *out = (uint8_t *)malloc(o.d.size());
-  if(!*out) return vkdt_set_error(VKDT_HIP_OOM, "jpg: out of memory");
-  memcpy(*out, o.d.data(), o.d.size());
-  *out_len = o.d.size();
-  return VKDT_HIP_OK;
+  scratch_put(sc, !err);
+  scratch_put(st, !err);
+  return err;
 }
 
 extern "C" void vkdt_jpg_free(uint8_t *p) { free(p); }

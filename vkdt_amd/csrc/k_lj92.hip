@@ -1269,8 +1269,9 @@ extern "C" int vkdt_hip_lj92_decode(const uint8_t *data, size_t data_len, const 
   std::vector<lj92_tab> tabs(tables.size());
   for(size_t k = 0; k < tables.size(); k++)
     if(int e = lj92_table(tables[k].data(), tables[k].data() + 16, &tabs[k])) return e;
-  uint8_t *dev = nullptr;
-  if(int e = hip_fail(hipMalloc((void **)&dev, total), "lj92 scratch")) return e;
+  scratch_t sc;
+  if(int e = scratch_get(sc, total, "lj92 scratch")) return e;
+  uint8_t *dev = sc.dev;
   // the jobs grouped by kind, then two zero status words (one lane a stream,
   // many lanes); the row caches need
   // no clearing: the first line reads none
@@ -1392,7 +1393,7 @@ extern "C" int vkdt_hip_lj92_decode(const uint8_t *data, size_t data_len, const 
   }
   if(!err) err = hip_fail(hipMemcpyAsync(bad, st, sizeof(bad), hipMemcpyDeviceToHost, s), "lj92 status");
   if(!err) err = hip_fail(hipStreamSynchronize(s), "lj92 sync");
-  (void)hipFree(dev);
+  scratch_put(sc, !err);
   if(err) return err;
   if(bad[0] + bad[1])
     return vkdt_set_error(VKDT_HIP_INCOMPLETE, "lj92: %d tiles with corrupt entropy-coded data", bad[0] + bad[1]);

@@ -43,8 +43,9 @@ extern "C" int vkdt_hip_unpack_msb16(const uint8_t *packed, size_t bytes, void *
   if(bits < 1 || bits > 16) return vkdt_set_error(VKDT_HIP_INCOMPLETE, "unpack: %d bits per sample", bits);
   if(n == 0) return VKDT_HIP_OK;
   if(!out || !packed) return vkdt_set_error(VKDT_HIP_INCOMPLETE, "unpack: no buffer");
-  uint8_t *dev = nullptr;
-  if(int e = hip_fail(hipMalloc((void **)&dev, bytes + 8), "unpack staging")) return e;
+  scratch_t sc;
+  if(int e = scratch_get(sc, bytes + 8, "unpack staging")) return e;
+  uint8_t *dev = sc.dev;
   hipStream_t s = (hipStream_t)stream;
   int err = hip_fail(hipMemcpyAsync(dev, packed, bytes, hipMemcpyHostToDevice, s), "unpack upload");
   if(!err)
@@ -55,6 +56,6 @@ extern "C" int vkdt_hip_unpack_msb16(const uint8_t *packed, size_t bytes, void *
     err = launch_post("unpack");
   }
   if(!err) err = hip_fail(hipStreamSynchronize(s), "unpack sync");
-  (void)hipFree(dev);
+  scratch_put(sc, !err);
   return err;
 }

@@ -225,10 +225,15 @@ def lj92_decode_host(blob, tile, W, H):
     return out
 
 
+def _view(data):
+    """the caller's bytes as an array, not copied"""
+    return np.frombuffer(data, np.uint8) if len(data) else np.zeros(1, np.uint8)
+
+
 def unpack_msb16(packed, out, n, bits, stream=None):
     """bit-packed samples (bytes, Magic Lantern layout) into a uint16 device buffer"""
-    buf = (C.c_uint8 * max(1, len(packed))).from_buffer_copy(packed or b"\0")
-    check(lib().vkdt_hip_unpack_msb16(buf, len(packed), out, n, bits, stream), "unpack")
+    buf = _view(packed)
+    check(lib().vkdt_hip_unpack_msb16(buf.ctypes.data, len(packed), out, n, bits, stream), "unpack")
 
 
 JPG_DCT_ISLOW, JPG_DCT_IFAST, JPG_DCT_FLOAT = 0, 1, 2
@@ -253,7 +258,7 @@ def jpg_encode(rgba_dev, wd, ht, pitch, quality=95, hs=1, vs=1, stream=None, dct
 def lj92_decode(blob, tiles, images, stream=None):
     """tiles of several images on the GPU; images: [(device ptr, W, H, pitch[, x0, y0])], each a
     window of W x H sites from (x0, y0) on of its tiles' image"""
-    buf = (C.c_uint8 * len(blob)).from_buffer_copy(blob)
+    buf = _view(blob)
     t = (Lj92Tile * len(tiles))(*tiles)
     im = (Lj92Image * len(images))(*[Lj92Image(*(tuple(i) + (0, 0))[:6]) for i in images])
-    check(lib().vkdt_hip_lj92_decode(buf, len(blob), t, len(tiles), im, len(images), stream), "lj92 decode")
+    check(lib().vkdt_hip_lj92_decode(buf.ctypes.data, len(blob), t, len(tiles), im, len(images), stream), "lj92 decode")
