@@ -85,6 +85,15 @@ def test_coarse_levels_equal_the_plain_graph(tmp_path, hip, W, Hh, kw):
     c[0].close()
 
 
+@pytest.mark.parametrize("W,Hh,kw", [(96, 24, dict()), (294, 81, dict()), (390, 123, dict(extra=["param:demosaic:01:colour:1"]))],
+                         ids=["one-tile", "inner-tile", "radius-3"])
+def test_xtrans_tiles_equal_the_plain_graph(tmp_path, hip, W, Hh, kw):
+    """the fused X-Trans develop tiles of 96x24: none, one and several inside"""
+    c = plain_and_planned(tmp_path, "xtrans", W, Hh, 62, kw)
+    check_equal(batch.develop([c[0]], [c[1]]), [c], f"{W}x{Hh} {kw}")
+    c[0].close()
+
+
 def test_alone_equals_in_the_mix(cases):
     """each image developed in a batch of one equals its plain run too"""
     for i, c in enumerate(cases):

@@ -67,3 +67,24 @@ def test_demosaic_down_node(hip, kind):
     host = parity.run_gpu_graph(hip, bufs, nodes, mos)
     rep = parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))
     assert rep[0][2] <= 1
+
+
+@pytest.mark.parametrize("fmt", [gs.F16, gs.UI16], ids=["f16", "unorm16"])
+@pytest.mark.parametrize("W,H", [(6, 6), (96, 24), (291, 75), (294, 78), (297, 123), (390, 99)])
+def test_xtrans_tiles(hip, fmt, W, H):
+    """splat and fix on X-Trans mosaics of every tile case: smaller than a
+    tile of 96x24, no tile inside the image, the first extents with one (96 +
+    96 + taps), partial tiles: against the oracle on the same inputs"""
+    import numpy as np
+    rng = np.random.default_rng(W * H + fmt)
+    mos = rng.uniform(0.05, 1, size=(H, W)).astype(np.float16) if fmt == gs.F16 else rng.integers(2000, 65536, (H, W), dtype=np.uint16)
+    p = gs.DevelopParams(kind="xtrans")
+    pc = gs.mixed_blob([("f", 1.0)] * 4 + [("i", p.filters)])
+    par = gs.mixed_blob([("i", 0), ("i", 0)])
+    bufs = {"raw": (W, H, 1, fmt, 1), "cov": (W // 3, H // 3, 4, gs.F16, 1), "green": (W, H, 1, gs.F16, 1),
+            "out": (W, H, 4, gs.F16, 1)}
+    nodes = [dict(module="demosaic", kernel="gauss", pc=pc, params=par, conn=["raw", "raw", "cov"], wd=W // 3, ht=H // 3, dp=1, out=2),
+             dict(module="demosaic", kernel="splat", pc=pc, params=par, conn=["raw", "cov", "green"], wd=W, ht=H, dp=1, out=2),
+             dict(module="demosaic", kernel="fix", pc=pc, params=par, conn=["raw", "green", "cov", "out"], wd=W, ht=H, dp=1, out=3)]
+    host = parity.run_gpu_graph(hip, bufs, nodes, mos)
+    parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))

@@ -127,10 +127,14 @@ DEV int bt_next(const bt_launch &L, int &tried)
 // image; fn(job, local tile) does one tile.  Both may use __syncthreads
 // (every thread calls them alike).  Persistent work groups keep the image
 // of their last tile and redo setup only when the queue moves them on.
-template<typename S, typename F>
+// P: persistent, fixed at compile time: a kernel with both loops held its
+// stage twice and registers for the two together (develop 80 -> 57, dnasm
+// 72 -> 63, final spills 37 -> 13): ten stills of 284 MP 22.3 -> 19.9 ms, with
+// X-Trans develop by phase.
+template<int P, typename S, typename F>
 DEV void bt_tiles(const bt_launch &L, S setup, F fn)
 {
-  if(!L.persist)
+  if(!P)
   { // one tile per work group, XCD k on the k-th eighth of the list
     const int n = gridDim.x, b = blockIdx.x;
     const int q = n / NUM_XCD, r = n - q * NUM_XCD, k = b % NUM_XCD;
@@ -189,11 +193,12 @@ DEV void lds_copy(T &dst, const T &src)
 
 // ---- denoise -----------------------------------------------------------------
 
+template<int P>
 __global__ void __launch_bounds__(256) kb_half(bt_launch L)
 {
   __shared__ dn_args a;
   dimg cfa, o;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.dn_half);
     cfa = rfl(im.cfa); o = rfl(im.qh);
@@ -209,12 +214,13 @@ __global__ void __launch_bounds__(256) kb_half(bt_launch L)
   });
 }
 
+template<int P>
 __global__ void __launch_bounds__(256) kb_downcov(bt_launch L)
 {
   __shared__ dn_cov_smem<COV_R> s;
   __shared__ dn_args a;
   dimg in, o;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.dn_down[0]);
     in = rfl(im.qh); o = rfl(im.qd[0]);
@@ -225,12 +231,13 @@ __global__ void __launch_bounds__(256) kb_downcov(bt_launch L)
 }
 
 // at most 72 VGPRs (7 waves per SIMD), measured faster than the compiler's choice
+template<int P>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) kb_down(bt_launch L)
 {
   __shared__ float4 tile[DN_TN(DOWN_R)];
   __shared__ dn_args a;
   dimg in, o;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.dn_down[jb.level]);
     in = rfl(im.qd[jb.level - 1]); o = rfl(im.qd[jb.level]);
@@ -240,11 +247,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) k
 }
 
 // at most 72 VGPRs (7 waves per SIMD), measured faster than the compiler's choice
+template<int P>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) kb_dnasm(bt_launch L, asm_mats m)
 {
   __shared__ dn_args a;
   dimg s0, s1, s2, s3, s4, o;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.dn_asm);
     s0 = rfl(im.qh); s1 = rfl(im.qd[0]); s2 = rfl(im.qd[1]); s3 = rfl(im.qd[2]); s4 = rfl(im.qd[3]); o = rfl(im.qa);
@@ -260,11 +268,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) k
   });
 }
 
+template<int P>
 __global__ void __launch_bounds__(256) kb_doub(bt_launch L)
 {
   __shared__ dn_args a;
   dimg cfa, crs0, crs1, o;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.dn_doub);
     cfa = rfl(im.cfa); crs0 = rfl(im.qa); crs1 = rfl(im.qh); o = rfl(im.dmos);
@@ -296,12 +305,13 @@ __global__ void __launch_bounds__(256) kb_doub(bt_launch L)
 
 // ---- hilite -----------------------------------------------------------------
 
+template<int P>
 __global__ void __launch_bounds__(256) kb_hl_half(bt_launch L)
 {
   __shared__ hl_args a;
   dimg in, o;
   int xt = 0;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.hl);
     in = rfl(im.dmos); o = rfl(im.hq[0]); xt = rfl(im.xt);
@@ -318,12 +328,13 @@ __global__ void __launch_bounds__(256) kb_hl_half(bt_launch L)
 }
 
 // reduce to level jb.level: tiles of BX x BY coarse texels
+template<int P>
 __global__ void __launch_bounds__(256) kb_hl_reduce(bt_launch L)
 {
   __shared__ hl_lds t;
   __shared__ hl_args a;
   dimg in, o;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.hl);
     in = rfl(im.hq[jb.level - 1]); o = rfl(im.hq[jb.level]);
@@ -333,11 +344,12 @@ __global__ void __launch_bounds__(256) kb_hl_reduce(bt_launch L)
 }
 
 // assemble of level jb.level from its fine level and the next coarser one
+template<int P>
 __global__ void __launch_bounds__(256) kb_hl_asm(bt_launch L)
 {
   __shared__ hl_args a;
   dimg fine, crs, o;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.hl);
     fine = rfl(im.hq[jb.level]); crs = rfl(im.ha[jb.level + 1]); o = rfl(im.ha[jb.level]);
@@ -355,12 +367,13 @@ __global__ void __launch_bounds__(256) kb_hl_asm(bt_launch L)
 
 // back onto the mosaic: one thread per block
 // at most 64 VGPRs (8 waves per SIMD), measured faster than the compiler's choice
+template<int P>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) kb_hl_doub(bt_launch L)
 {
   __shared__ hl_args a;
   dimg in, crs, o;
   int xt = 0, nx = 0, ny = 0;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.hl);
     in = rfl(im.dmos); crs = rfl(im.ha[0]); o = rfl(im.mos);
@@ -381,11 +394,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) k
 
 // ---- demosaic + colour + filmcurv --------------------------------------------
 
+template<int P>
 __global__ void __launch_bounds__(256) kb_gauss(bt_launch L)
 {
   dimg in, o;
   int xt = 0;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     in = rfl(im.mos); o = rfl(im.cov); xt = rfl(im.xt);
   }, [&](const bt_job &jb, int lt) {
@@ -413,41 +427,63 @@ __global__ void __launch_bounds__(256) kb_gauss(bt_launch L)
 // mosaic through the bounds-checked global path.  Both see the same values.
 #define DEV_M 5   // r + rs <= 3 + 2
 
-// (row, column) of the elements i0, i0 + step, ... of a row-major tile w
-// wide, stepped without a division per element
-struct tile_walk
-{
-  int ty, tx, dq, dr, w;
-  __device__ tile_walk(int i0, int step, int w_) : w(w_)
-  {
-    ty = i0 / w; tx = i0 - ty * w;
-    dq = step / w; dr = step - dq * w;
-  }
-  __device__ void next()
-  {
-    tx += dr; ty += dq;
-    if(tx >= w) { tx -= w; ty++; }
-  }
-};
+// tile of the develop stage: 64x16 texels, X-Trans 96x24 (whole 3x3 cells and
+// whole waves of each phase)
+template<int XT> struct dev_tile { static constexpr int W = XT ? XT_TW : BX, H = XT ? XT_TH : BY * DEV_R; };
 
 template<int XT>
 DEV void develop_tile(const dimg &mos, const dimg &cov, const dimg &film, const co_args &co, const fc_args &fc,
                       int r, int X0, int Y0, float *gt, float *mt)
 {
-  constexpr int rs = XT ? 2 : 1;
-  const int gw = BX + 2 * r, gh = BY * DEV_R + 2 * r;
+  constexpr int rs = XT ? 2 : 1, DW = dev_tile<XT>::W, DH = dev_tile<XT>::H;
+  const int gw = DW + 2 * r, gh = DH + 2 * r;
   const int W = film.wd, H = film.ht;
-  const int m = r + rs, mw = BX + 2 * m, mh = BY * DEV_R + 2 * m;
+  const int m = r + rs, mw = DW + 2 * m, mh = DH + 2 * m;
   const int tid = threadIdx.y * BX + threadIdx.x;
-  const int x = X0 + threadIdx.x;
   auto green = [&](int px, int py) { return gt[(py - Y0 + r) * gw + (px - X0 + r)]; };
-  if(X0 - m >= 0 && Y0 - m >= 0 && X0 + BX + m <= W && Y0 + BY * DEV_R + m <= H)
+  auto finish = [&](float4 f, int x, int y) { st_h4(film, x, y, fc_px_basic(r16(co_px(r16(f), co)), fc)); };
+  if(X0 - m >= 0 && Y0 - m >= 0 && X0 + DW + m <= W && Y0 + DH + m <= H)
   {
     tile_walk wm(tid, BX * BY, mw);
     for(int i = tid; i < mw * mh; i += BX * BY, wm.next())
       mt[i] = ld_h1(mos, X0 - m + wm.tx, Y0 - m + wm.ty);
     __syncthreads();
     auto mosl = [&](int px, int py) { return mt[(py - Y0 + m) * mw + (px - X0 + m)]; };
+    if(XT && r == 2)
+    { // each wave one phase of the CFA cells at a time (dm_splat_xt): the tile
+      // starts on a cell, and its halo of 2 holds 33 or 34 by 9 or 10 sites of a
+      // phase, dealt to the waves 64 at a time
+      const int wv = threadIdx.y, l = threadIdx.x, c0x = X0 / 3, c0y = Y0 / 3;
+#pragma unroll 1
+      for(int ph = 0; ph < 9; ph++)
+        xt_phase(ph, [&](auto px, auto py) {
+          constexpr int PX = decltype(px)::value, PY = decltype(py)::value;
+          constexpr int NX = PX == 1 ? XT_TW / 3 + 2 : XT_TW / 3 + 1, NY = PY == 1 ? XT_TH / 3 + 2 : XT_TH / 3 + 1;
+          for(int s0 = ((wv + 2 * ph) & 3) * 64; s0 < NX * NY; s0 += 256)
+          {
+            const int s = s0 + l, sy = s / NX, sx = s - sy * NX;
+            if(s >= NX * NY) continue;
+            const int cx = c0x + sx - (PX > 0), cy = c0y + sy - (PY > 0);
+            gt[(3 * cy + PY - Y0 + 2) * (XT_TW + 4) + (3 * cx + PX - X0 + 2)] = r16(dm_splat_xt<PX, PY>(mosl, cov, cx, cy));
+          }
+        });
+      __syncthreads();
+#pragma unroll 1
+      for(int ph = 0; ph < 9; ph++)
+      {
+        const int cx = c0x + l % 32, cy = c0y + 2 * wv + l / 32;
+        float4 f;
+        int x, y;
+        xt_phase(ph, [&](auto px, auto py) {
+          constexpr int PX = decltype(px)::value, PY = decltype(py)::value;
+          f = dm_fix_xt<PX, PY>(mosl, cov, cx, cy, green);
+          x = 3 * cx + PX;
+          y = 3 * cy + PY;
+        });
+        finish(f, x, y);
+      }
+      return;
+    }
     if(XT)
     {
       tile_walk wg(tid, BX * BY, gw);
@@ -471,16 +507,20 @@ DEV void develop_tile(const dimg &mos, const dimg &cov, const dimg &film, const 
       }
     }
     __syncthreads();
+    if(XT)
+    {
+      tile_walk wt(tid, BX * BY, DW);
+#pragma unroll 1
+      for(int i = tid; i < DW * DH; i += BX * BY, wt.next())
+        finish(dm_fix_loop<1>(mosl, cov, r, X0 + wt.tx, Y0 + wt.ty, green), X0 + wt.tx, Y0 + wt.ty);
+      return;
+    }
 #pragma unroll 1
     for(int k = 0; k < DEV_R; k++)
     { // Bayer: each wave one CFA colour (bayer_wave_xy) in each 64x4 band
-      const int2 q = XT ? make_int2(x, Y0 + threadIdx.y + BY * k) : bayer_wave_xy(X0, Y0 + BY * k);
-      const int xq = q.x, y = q.y;
-      const float4 f = XT ? dm_fix_r<XT>(mosl, cov, r, xq, y, green)
-                          : (((xq + y) & 1) ? dm_fix_r<XT, 1>(mosl, cov, r, xq, y, green)
-                                            : dm_fix_r<XT, 0>(mosl, cov, r, xq, y, green));
-      const float4 c = r16(co_px(r16(f), co));
-      st_h4(film, xq, y, fc_px_basic(c, fc));
+      const int2 q = bayer_wave_xy(X0, Y0 + BY * k);
+      finish(((q.x + q.y) & 1) ? dm_fix_r<0, 1>(mosl, cov, r, q.x, q.y, green)
+                               : dm_fix_r<0, 0>(mosl, cov, r, q.x, q.y, green), q.x, q.y);
     }
     return;
   }
@@ -488,35 +528,34 @@ DEV void develop_tile(const dimg &mos, const dimg &cov, const dimg &film, const 
   for(int i = tid; i < gw * gh; i += BX * BY, wg.next())
     gt[i] = r16(dm_splat_px<XT>(mos, cov, mirror(X0 - r + wg.tx, W), mirror(Y0 - r + wg.ty, H)));
   __syncthreads();
+  tile_walk wt(tid, BX * BY, DW);
 #pragma unroll 1
-  for(int k = 0; k < DEV_R; k++)
+  for(int i = tid; i < DW * DH; i += BX * BY, wt.next())
   {
-    const int y = Y0 + threadIdx.y + BY * k;
-    if(x >= W || y >= H) continue;
-    const float4 f = dm_fix_px<XT>(mos, cov, r, x, y, green);
-    const float4 c = r16(co_px(r16(f), co));
-    st_h4(film, x, y, fc_px_basic(c, fc));
+    const int x = X0 + wt.tx, y = Y0 + wt.ty;
+    if(x < W && y < H) finish(dm_fix_px<XT>(mos, cov, r, x, y, green), x, y);
   }
 }
 
-// at most 80 VGPRs, 6 waves per SIMD (X-Trans needed 96, 5 waves): the
-// staging and splat phases' memory latency is hidden by the extra waves
-template<int XT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) kb_develop(bt_launch L)
+// Bayer: at most 80 VGPRs, 6 waves per SIMD: the staging and splat phases'
+// memory latency is hidden by the extra waves.  X-Trans: 5, what its LDS holds
+template<int XT, int P>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(XT ? 5 : 6))) kb_develop(bt_launch L)
 {
-  __shared__ float gt[(BX + 6) * (BY * DEV_R + 6)];                 // green, halo r <= 3
-  __shared__ float mt[(BX + 2 * DEV_M) * (BY * DEV_R + 2 * DEV_M)];  // mosaic, halo r + rs
+  constexpr int DW = dev_tile<XT>::W, DH = dev_tile<XT>::H;
+  __shared__ float gt[(DW + 6) * (DH + 6)];                       // green, halo r <= 3
+  __shared__ float mt[(DW + 2 * DEV_M) * (DH + 2 * DEV_M)];       // mosaic, halo r + rs
   __shared__ co_args co;
   __shared__ fc_args fc;
   dimg mos, cov, film;
   int r = 1;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(co, im.co);
     lds_copy(fc, im.fc);
     mos = rfl(im.mos); cov = rfl(im.cov); film = rfl(im.film); r = rfl(im.dm_r);
   }, [&](const bt_job &jb, int lt) {
-    const int X0 = (lt % jb.tiles_x) * BX, Y0 = (lt / jb.tiles_x) * (BY * DEV_R);
+    const int X0 = (lt % jb.tiles_x) * DW, Y0 = (lt / jb.tiles_x) * DH;
     develop_tile<XT>(mos, cov, film, co, fc, r, X0, Y0, gt, mt);
   });
 }
@@ -531,12 +570,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 #define P1_H (2 * BY + 1)
 #define P1_N (P1_W * P1_H)
 
+template<int P>
 __global__ void __launch_bounds__(256) kb_pyr1(bt_launch L)
 {
   extern __shared__ __half pl[];   // (num_gamma + 1) x P1_N
   __shared__ ll_args a;
   dimg f, o;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.ll);
     f = rfl(im.film); o = rfl(im.lp[1]);
@@ -572,12 +612,12 @@ __global__ void __launch_bounds__(256) kb_pyr1(bt_launch L)
 // launch waits for (a 4096 x 2160 frame's levels 3 to 6: 9.2 us each -> 5.4);
 // on larger ones the tiles' set-up costs more than it gains
 #define LL_SPLIT (1 << 18)
-template<int SPLIT>
+template<int SPLIT, int P>
 __global__ void __launch_bounds__(256) kb_reduce(bt_launch L)
 {
   dimg in, o;
   int planes = 1;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     in = rfl(im.lp[jb.level - 1]); o = rfl(im.lp[jb.level]); planes = rfl(im.ll.num_gamma + 1);
   }, [&](const bt_job &jb, int lt) {
@@ -595,6 +635,7 @@ __global__ void __launch_bounds__(256) kb_reduce(bt_launch L)
 }
 
 // assemble level l (1 <= l <= nl-2) from level l+1
+template<int P>
 __global__ void __launch_bounds__(256) kb_asm(bt_launch L)
 {
   extern __shared__ float tile[];
@@ -602,7 +643,7 @@ __global__ void __launch_bounds__(256) kb_asm(bt_launch L)
   __shared__ ll_args a;
   dimg fine, l1, coarse, o;
   int first = 0;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     const int l = jb.level;
     lds_copy(a, im.ll);
@@ -635,12 +676,13 @@ __global__ void __launch_bounds__(256) kb_asm(bt_launch L)
 // the same a texel a thread, reading the coarse footprint straight from
 // memory, for launches of at most LL_SMALL texels (as k_ll_assemble_small:
 // staging the planes in LDS costs those several dependent round trips)
+template<int P>
 __global__ void __launch_bounds__(256) kb_asm_small(bt_launch L)
 {
   __shared__ ll_args a;
   dimg fine, l1, coarse, o;
   int first = 0;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     const int l = jb.level;
     lds_copy(a, im.ll);
@@ -740,6 +782,7 @@ __global__ void __launch_bounds__(BX * LL_TAIL_Y) kb_tail(bt_launch L)
 // assemble level 0 + llap/colour: level 0 planes from the filmcurv output.
 // At most 80 VGPRs (6 waves per SIMD instead of 5): its dependent phases
 // (rows, plane range, staging) need the extra waves to hide memory latency
+template<int P>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) kb_final(bt_launch L)
 {
   extern __shared__ float tile[];
@@ -747,7 +790,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
   __shared__ ll_args a;
   dimg f, l1, coarse, o;
   int first = 0;
-  bt_tiles(L, [&](const bt_job &jb) {
+  bt_tiles<P>(L, [&](const bt_job &jb) {
     const bt_img &im = L.img[jb.img];
     lds_copy(a, im.ll);
     first = rfl((int)(im.nl == 2));
@@ -1048,7 +1091,8 @@ static int tiles_of(int kind, const dims_t &m, int level, int rows, int &tx)
     case K_HL_ASM: w = m.hw[level]; h = m.hh[level]; th = BY * rows; break;
     case K_HL_DOUB: w = std::min((m.qw + 7) / 8 * 8, m.W); h = std::min((m.qh + 7) / 8 * 8, m.H); th = BY * rows; break;
     case K_GAUSS: w = m.cw; h = m.ch; th = BY * rows; break;
-    case K_DEVELOP: case K_DEVELOP_XT: w = m.W; h = m.H; th = BY * DEV_R; break;
+    case K_DEVELOP: w = m.W; h = m.H; tw = dev_tile<0>::W; th = dev_tile<0>::H; break;
+    case K_DEVELOP_XT: w = m.W; h = m.H; tw = dev_tile<1>::W; th = dev_tile<1>::H; break;
     case K_PYR1: w = m.lw[1]; h = m.lh[1]; break;
     case K_REDUCE: case K_REDUCE_SPLIT: w = m.lw[level]; h = m.lh[level]; tw = 4 * BX; break;
     case K_TAIL: tx = 1; return 1;
@@ -1200,28 +1244,33 @@ static int enqueue(vkdt_batch_t *b, hipStream_t s, int timed)
     const int rows = is_pixel_stage(L.kind) ? tune_rows(b->tune[g]) : 1;
     bt_launch a = { b->d_img, b->d_job + L.job0, L.njob, L.total, b->d_ctr + L.ctr0, persist, rows };
     const dim3 grid(persist && L.kind != K_TAIL ? b->ncu * persist : L.total), blk(BX, BY);
-    switch(L.kind)
-    {
-      case K_HALF:    hipLaunchKernelGGL(kb_half, grid, blk, 0, s, a); break;
-      case K_DOWNCOV: hipLaunchKernelGGL(kb_downcov, grid, blk, 0, s, a); break;
-      case K_DOWN:    hipLaunchKernelGGL(kb_down, grid, blk, 0, s, a); break;
-      case K_DNASM:   hipLaunchKernelGGL(kb_dnasm, grid, blk, 0, s, a, b->mats); break;
-      case K_DOUB:    hipLaunchKernelGGL(kb_doub, grid, blk, 0, s, a); break;
-      case K_HL_HALF: hipLaunchKernelGGL(kb_hl_half, grid, blk, 0, s, a); break;
-      case K_HL_REDUCE: hipLaunchKernelGGL(kb_hl_reduce, grid, blk, 0, s, a); break;
-      case K_HL_ASM:  hipLaunchKernelGGL(kb_hl_asm, grid, blk, 0, s, a); break;
-      case K_HL_DOUB: hipLaunchKernelGGL(kb_hl_doub, grid, blk, 0, s, a); break;
-      case K_GAUSS:   hipLaunchKernelGGL(kb_gauss, grid, blk, 0, s, a); break;
-      case K_DEVELOP: hipLaunchKernelGGL(kb_develop<0>, grid, blk, 0, s, a); break;
-      case K_DEVELOP_XT: hipLaunchKernelGGL(kb_develop<1>, grid, blk, 0, s, a); break;
-      case K_PYR1:    hipLaunchKernelGGL(kb_pyr1, grid, blk, L.lds, s, a); break;
-      case K_REDUCE:  hipLaunchKernelGGL(kb_reduce<0>, grid, blk, 0, s, a); break;
-      case K_REDUCE_SPLIT: hipLaunchKernelGGL(kb_reduce<1>, grid, blk, 0, s, a); break;
-      case K_TAIL:    hipLaunchKernelGGL(kb_tail, grid, dim3(BX, LL_TAIL_Y), L.lds, s, a); break;
-      case K_ASM_SMALL: hipLaunchKernelGGL(kb_asm_small, grid, blk, 0, s, a); break;
-      case K_ASM:     hipLaunchKernelGGL(kb_asm, grid, blk, L.lds, s, a); break;
-      default:        hipLaunchKernelGGL(kb_final, grid, blk, L.lds, s, a); break;
-    }
+    const auto run = [&](auto persistent) {
+      constexpr int P = decltype(persistent)::value;
+      switch(L.kind)
+      {
+        case K_HALF:    hipLaunchKernelGGL(kb_half<P>, grid, blk, 0, s, a); break;
+        case K_DOWNCOV: hipLaunchKernelGGL(kb_downcov<P>, grid, blk, 0, s, a); break;
+        case K_DOWN:    hipLaunchKernelGGL(kb_down<P>, grid, blk, 0, s, a); break;
+        case K_DNASM:   hipLaunchKernelGGL(kb_dnasm<P>, grid, blk, 0, s, a, b->mats); break;
+        case K_DOUB:    hipLaunchKernelGGL(kb_doub<P>, grid, blk, 0, s, a); break;
+        case K_HL_HALF: hipLaunchKernelGGL(kb_hl_half<P>, grid, blk, 0, s, a); break;
+        case K_HL_REDUCE: hipLaunchKernelGGL(kb_hl_reduce<P>, grid, blk, 0, s, a); break;
+        case K_HL_ASM:  hipLaunchKernelGGL(kb_hl_asm<P>, grid, blk, 0, s, a); break;
+        case K_HL_DOUB: hipLaunchKernelGGL(kb_hl_doub<P>, grid, blk, 0, s, a); break;
+        case K_GAUSS:   hipLaunchKernelGGL(kb_gauss<P>, grid, blk, 0, s, a); break;
+        case K_DEVELOP: hipLaunchKernelGGL((kb_develop<0, P>), grid, blk, 0, s, a); break;
+        case K_DEVELOP_XT: hipLaunchKernelGGL((kb_develop<1, P>), grid, blk, 0, s, a); break;
+        case K_PYR1:    hipLaunchKernelGGL(kb_pyr1<P>, grid, blk, L.lds, s, a); break;
+        case K_REDUCE:  hipLaunchKernelGGL((kb_reduce<0, P>), grid, blk, 0, s, a); break;
+        case K_REDUCE_SPLIT: hipLaunchKernelGGL((kb_reduce<1, P>), grid, blk, 0, s, a); break;
+        case K_TAIL:    hipLaunchKernelGGL(kb_tail, grid, dim3(BX, LL_TAIL_Y), L.lds, s, a); break;
+        case K_ASM_SMALL: hipLaunchKernelGGL(kb_asm_small<P>, grid, blk, 0, s, a); break;
+        case K_ASM:     hipLaunchKernelGGL(kb_asm<P>, grid, blk, L.lds, s, a); break;
+        default:        hipLaunchKernelGGL(kb_final<P>, grid, blk, L.lds, s, a); break;
+      }
+    };
+    if(persist) run(int_c<1>());
+    else run(int_c<0>());
     if(int e = hip_fail(hipGetLastError(), group_name[g])) return e;
   }
   if(timed)

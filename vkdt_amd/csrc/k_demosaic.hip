@@ -63,28 +63,23 @@ DEV int2 cfa_xy()
   return bayer_wave_xy(t.x * BX, t.y * BY);
 }
 
-template<int XT, int U16, int PAR>
+template<int U16, int PAR>
 DEV float dm_splat_node(const dimg &in, const dimg &ga, int x, int y)
 {
-  constexpr int R = XT ? 2 : 1;
-  if(__all(x >= R && y >= R && x + R < in.wd && y + R < in.ht))
-    return dm_splat_at<XT, PAR>([&](int px, int py) { return ld_mt<U16>(in, px, py); }, in.wd, in.ht, ga, x, y);
-  return dm_splat_px<XT, U16, PAR>(in, ga, x, y);
+  if(__all(x >= 1 && y >= 1 && x + 1 < in.wd && y + 1 < in.ht))
+    return dm_splat_at<0, PAR>([&](int px, int py) { return ld_mt<U16>(in, px, py); }, in.wd, in.ht, ga, x, y);
+  return dm_splat_px<0, U16, PAR>(in, ga, x, y);
 }
 
 // Bayer waves are colour-uniform (cfa_xy), so the branch on the site's
 // parity is uniform too, and each wave weights only its colour's taps
-template<int XT, int U16>
+template<int U16>
 __global__ void __launch_bounds__(256) k_dm_splat(dimg in, dimg ga, dimg out)
 {
-  const int2 p = cfa_xy<XT>();
+  const int2 p = cfa_xy<0>();
   const int x = p.x, y = p.y;
   if(x >= out.wd || y >= out.ht) return;
-  float v;
-  if(XT) v = dm_splat_node<XT, U16, -1>(in, ga, x, y);
-  else if((x + y) & 1) v = dm_splat_node<XT, U16, 0>(in, ga, x, y);
-  else v = dm_splat_node<XT, U16, 1>(in, ga, x, y);
-  st_h1(out, x, y, v);
+  st_h1(out, x, y, ((x + y) & 1) ? dm_splat_node<U16, 0>(in, ga, x, y) : dm_splat_node<U16, 1>(in, ga, x, y));
 }
 
 template<int XT, int U16, int PAR>
@@ -107,6 +102,82 @@ __global__ void __launch_bounds__(256) k_dm_fix(dimg in, dimg gr, dimg cv, dimg 
   else if((x + y) & 1) v = dm_fix_node<XT, U16, 1>(in, gr, cv, r, x, y);
   else v = dm_fix_node<XT, U16, 0>(in, gr, cv, r, x, y);
   st_h4(out, x, y, v);
+}
+
+// X-Trans by phase (dm_splat_xt, dm_fix_xt): a tile of 32x8 cells with its
+// halo staged in LDS, each wave two rows of cells, one phase of them at a
+// time; tiles whose taps leave the image take the general path per site
+template<int U16>
+__global__ void __launch_bounds__(256) k_dm_splat_xt(dimg in, dimg ga, dimg out)
+{
+  __shared__ float mt[(XT_TW + 4) * (XT_TH + 4)];
+  __shared__ __half o[XT_TW * XT_TH];
+  constexpr int mw = XT_TW + 4;
+  const int2 t = xcd_block();
+  const int X0 = t.x * XT_TW, Y0 = t.y * XT_TH, wv = threadIdx.y, l = threadIdx.x, tid = wv * BX + l;
+  if(X0 >= 2 && Y0 >= 2 && X0 + XT_TW + 2 <= in.wd && Y0 + XT_TH + 2 <= in.ht && X0 + XT_TW <= out.wd && Y0 + XT_TH <= out.ht)
+  {
+    tile_walk wm(tid, 256, mw);
+    for(int i = tid; i < mw * (XT_TH + 4); i += 256, wm.next()) mt[i] = ld_mt<U16>(in, X0 - 2 + wm.tx, Y0 - 2 + wm.ty);
+    __syncthreads();
+    auto mos = [&](int px, int py) { return mt[(py - Y0 + 2) * mw + (px - X0 + 2)]; };
+    const int sx = l % 32, sy = 2 * wv + l / 32;
+#pragma unroll 1
+    for(int ph = 0; ph < 9; ph++)
+      xt_phase(ph, [&](auto px, auto py) {
+        constexpr int PX = decltype(px)::value, PY = decltype(py)::value;
+        o[(3 * sy + PY) * XT_TW + 3 * sx + PX] = f2h(dm_splat_xt<PX, PY>(mos, ga, X0 / 3 + sx, Y0 / 3 + sy));
+      });
+    __syncthreads();
+    tile_walk ws(tid, 256, XT_TW);
+    for(int i = tid; i < XT_TW * XT_TH; i += 256, ws.next())
+      ((__half *)out.p)[(long)(Y0 + ws.ty) * out.pitch + X0 + ws.tx] = o[i];
+    return;
+  }
+  tile_walk ws(tid, 256, XT_TW);
+  for(int i = tid; i < XT_TW * XT_TH; i += 256, ws.next())
+  {
+    const int x = X0 + ws.tx, y = Y0 + ws.ty;
+    if(x < out.wd && y < out.ht) st_h1(out, x, y, dm_splat_px<1, U16>(in, ga, x, y));
+  }
+}
+
+// fix with the default radius 2
+template<int U16>
+__global__ void __launch_bounds__(256) k_dm_fix_xt(dimg in, dimg gr, dimg cv, dimg out)
+{
+  __shared__ float mt[(XT_TW + 4) * (XT_TH + 4)], gt[(XT_TW + 4) * (XT_TH + 4)];
+  constexpr int mw = XT_TW + 4;
+  const int2 t = xcd_block();
+  const int X0 = t.x * XT_TW, Y0 = t.y * XT_TH, wv = threadIdx.y, l = threadIdx.x, tid = wv * BX + l;
+  if(X0 >= 2 && Y0 >= 2 && X0 + XT_TW + 2 <= min(in.wd, gr.wd) && Y0 + XT_TH + 2 <= min(in.ht, gr.ht) &&
+     X0 + XT_TW <= out.wd && Y0 + XT_TH <= out.ht)
+  {
+    tile_walk wm(tid, 256, mw);
+    for(int i = tid; i < mw * (XT_TH + 4); i += 256, wm.next())
+    {
+      mt[i] = ld_mt<U16>(in, X0 - 2 + wm.tx, Y0 - 2 + wm.ty);
+      gt[i] = ld_h1(gr, X0 - 2 + wm.tx, Y0 - 2 + wm.ty);
+    }
+    __syncthreads();
+    auto mos = [&](int px, int py) { return mt[(py - Y0 + 2) * mw + (px - X0 + 2)]; };
+    auto green = [&](int px, int py) { return gt[(py - Y0 + 2) * mw + (px - X0 + 2)]; };
+    const int cx = X0 / 3 + l % 32, cy = Y0 / 3 + 2 * wv + l / 32;
+#pragma unroll 1
+    for(int ph = 0; ph < 9; ph++)
+      xt_phase(ph, [&](auto px, auto py) {
+        constexpr int PX = decltype(px)::value, PY = decltype(py)::value;
+        st_h4(out, 3 * cx + PX, 3 * cy + PY, dm_fix_xt<PX, PY>(mos, cv, cx, cy, green));
+      });
+    return;
+  }
+  tile_walk ws(tid, 256, XT_TW);
+  for(int i = tid; i < XT_TW * XT_TH; i += 256, ws.next())
+  {
+    const int x = X0 + ws.tx, y = Y0 + ws.ty;
+    if(x < out.wd && y < out.ht)
+      st_h4(out, x, y, dm_fix_px<1, U16>(in, cv, 2, x, y, [&](int px, int py) { return centre_h1(gr, px, py); }));
+  }
 }
 
 // ---- halfsize (halfsize.comp:19-50): one rgba texel per CFA block --------
@@ -145,6 +216,8 @@ __global__ void __launch_bounds__(256) k_dm_halfsize(dimg in, dimg out)
 // the <XT, U16> instantiation of a demosaic kernel: CFA and mosaic format
 #define DM_PICK(kern, xt, u16) \
   ((xt) ? ((u16) ? kern<1, 1> : kern<1, 0>) : ((u16) ? kern<0, 1> : kern<0, 0>))
+
+static dim3 xt_grid(const node_call &c) { return dim3((c.wd + XT_TW - 1) / XT_TW, (c.ht + XT_TH - 1) / XT_TH, 1); }
 
 static int decode(dm_args &a, const node_call &c, const char *what)
 {
@@ -188,8 +261,12 @@ int launch_demosaic_splat(const node_call &c)
   if(c.conn[0].wd < 6 || c.conn[0].ht < 6)
     return vkdt_set_error(VKDT_HIP_INCOMPLETE, "demosaic/splat: input smaller than 6x6");
   const int u16 = c.conn[0].format == VKDT_FMT_UI16;
-  hipLaunchKernelGGL(DM_PICK(k_dm_splat, a.filters == 9, u16), grid2d(c.wd, c.ht, 1), dim3(BX, BY), 0, c.stream,
-                     to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]));
+  if(a.filters == 9)
+    hipLaunchKernelGGL(u16 ? k_dm_splat_xt<1> : k_dm_splat_xt<0>, xt_grid(c), dim3(BX, BY), 0, c.stream,
+                       to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]));
+  else
+    hipLaunchKernelGGL(u16 ? k_dm_splat<1> : k_dm_splat<0>, grid2d(c.wd, c.ht, 1), dim3(BX, BY), 0, c.stream,
+                       to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]));
   return launch_post("demosaic/splat");
 }
 
@@ -205,7 +282,11 @@ int launch_demosaic_fix(const node_call &c)
   if(a.filters == 9) { r = a.fixup + 2; r = r < 2 ? 2 : (r > 3 ? 3 : r); }
   else               { r = a.fixup + 1; r = r < 1 ? 1 : (r > 2 ? 2 : r); }
   const int u16 = c.conn[0].format == VKDT_FMT_UI16;
-  hipLaunchKernelGGL(DM_PICK(k_dm_fix, a.filters == 9, u16), grid2d(c.wd, c.ht, 1), dim3(BX, BY), 0, c.stream,
+  if(a.filters == 9 && r == 2)
+    hipLaunchKernelGGL(u16 ? k_dm_fix_xt<1> : k_dm_fix_xt<0>, xt_grid(c), dim3(BX, BY), 0, c.stream,
+                       to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]), to_dimg(c.conn[3]));
+  else
+    hipLaunchKernelGGL(DM_PICK(k_dm_fix, a.filters == 9, u16), grid2d(c.wd, c.ht, 1), dim3(BX, BY), 0, c.stream,
                      to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]), to_dimg(c.conn[3]), r);
   return launch_post("demosaic/fix");
 }
