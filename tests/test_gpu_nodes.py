@@ -88,3 +88,33 @@ def test_xtrans_tiles(hip, fmt, W, H):
              dict(module="demosaic", kernel="fix", pc=pc, params=par, conn=["raw", "green", "cov", "out"], wd=W, ht=H, dp=1, out=3)]
     host = parity.run_gpu_graph(hip, bufs, nodes, mos)
     parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))
+
+
+@pytest.mark.parametrize("kind,W,H,cx,cy", [("bayer", 2, 2, 0, 0), ("bayer", 67, 35, 1, 3), ("bayer", 130, 18, 4, 2),
+                                            ("xtrans", 3, 3, 0, 0), ("xtrans", 97, 26, 0, 0), ("xtrans", 100, 25, 6, 3),
+                                            ("xtrans", 195, 51, 1, 2)])
+def test_doub_blocks(hip, kind, W, H, cx, cy):
+    """denoise/doub, a block or cell per thread, where the last ones are cut
+    (one and two columns and rows left), the output is one block, and the crop
+    moves it over the mosaic's mirrored edge: against the oracle on the same
+    inputs"""
+    import numpy as np
+    rng = np.random.default_rng(W * H + cx)
+    raw = rng.integers(500, 16384, (H, W), dtype=np.uint16)
+    p = gs.DevelopParams(kind=kind)
+    blk = 3 if kind == "xtrans" else 2
+    qw, qh = -(-W // blk), -(-H // blk)
+    black, white = np.float32(512 / 65535.0), np.float32(16383 / 65535.0)
+    rgbc = [("f", 1.0)] * 4 + [("f", black)] * 4 + [("f", white)] * 4 + [("i", v) for v in (cx, cy, W + cx, H + cy)]
+    par = gs.mixed_blob([("f", 0.6), ("f", 0.3), ("f", 0.7), ("f", 0.0)] + [("f", 1.0)] * 4 + [("i", 1)])
+    bufs = {"raw": (W, H, 1, gs.UI16, 1), "half": (qw, qh, 4, gs.F16, 1), "s0": (qw, qh, 4, gs.F16, 1), "dn": (W, H, 1, gs.F16, 1)}
+    lv = rgbc[:12] + [("i", 0)] * 4
+    nodes = [dict(module="denoise", kernel="half", pc=gs.mixed_blob(rgbc + [("i", p.filters)]), params=par,
+                  conn=["raw", "half"], wd=qw, ht=qh, dp=1, out=1),
+             dict(module="denoise", kernel="downcov", pc=gs.mixed_blob(lv + [("f", 1e-4), ("f", 1e-6), ("i", 0), ("i", blk)]),
+                  params=par, conn=["half", "s0"], wd=qw, ht=qh, dp=1, out=1),
+             dict(module="denoise", kernel="doub",
+                  pc=gs.mixed_blob(rgbc + [("i", p.filters), ("f", 1e-4), ("f", 1e-6), ("i", 0)] + [("i", 0)] * 4), params=par,
+                  conn=["raw", "s0", "half", "dn"], wd=W, ht=H, dp=1, out=3)]
+    host = parity.run_gpu_graph(hip, bufs, nodes, raw)
+    parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))

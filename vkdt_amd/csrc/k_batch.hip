@@ -268,9 +268,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) k
   });
 }
 
-template<int P>
+// Bayer: 2x2 blocks per thread, tiles of 2 BX x 2 BY rows texels; X-Trans: 3x3
+// cells.  Instructions bound both.  Two kernels: in one, X-Trans took a texel
+// per thread with the registers of the Bayer branch (four waves per SIMD);
+// doub of ten stills, 283 MP of both kinds, went from 3240 to 1559 us
+template<int XT, int P>
 __global__ void __launch_bounds__(256) kb_doub(bt_launch L)
 {
+  constexpr int B = XT ? 3 : 2;
   __shared__ dn_args a;
   dimg cfa, crs0, crs1, o;
   bt_tiles<P>(L, [&](const bt_job &jb) {
@@ -278,27 +283,23 @@ __global__ void __launch_bounds__(256) kb_doub(bt_launch L)
     lds_copy(a, im.dn_doub);
     cfa = rfl(im.cfa); crs0 = rfl(im.qa); crs1 = rfl(im.qh); o = rfl(im.dmos);
   }, [&](const bt_job &jb, int lt) {
-    if(a.filters != 9u)
-    { // Bayer: 2x2 blocks per thread, tiles of 2 BX x 2 BY rows texels
-      const int x = ((lt % jb.tiles_x) * BX + threadIdx.x) * 2, Y0 = (lt / jb.tiles_x) * (BY * L.rows);
-#pragma unroll 1
-      for(int k = 0; k < L.rows; k++)
-      {
-        const int y = (Y0 + threadIdx.y + BY * k) * 2;
-        if(x >= o.wd || y >= o.ht) continue;
-        float v[4];
-        dn_doub_quad(cfa, crs0, crs1, o.wd, o.ht, a, x, y, v);
-        st_h1_quad(o, x, y, v);
-      }
-      return;
-    }
-    PIX_TILE(L, jb, lt, X0, Y0);
-    const int x = X0 + threadIdx.x;
+    const int cx = (lt % jb.tiles_x) * BX + threadIdx.x, Y0 = (lt / jb.tiles_x) * (BY * L.rows);
 #pragma unroll 1
     for(int k = 0; k < L.rows; k++)
     {
-      const int y = Y0 + threadIdx.y + BY * k;
-      if(x < o.wd && y < o.ht) st_h1(o, x, y, dn_doub_px(cfa, crs0, crs1, o.wd, o.ht, a, x, y));
+      const int cy = Y0 + threadIdx.y + BY * k;
+      if(B * cx >= o.wd || B * cy >= o.ht) continue;
+      float v[B * B];
+      if(XT)
+      {
+        dn_doub_cell(cfa, crs0, crs1, o.wd, o.ht, a, cx, cy, v);
+        st_h1_cell(o, cx, cy, v);
+      }
+      else
+      {
+        dn_doub_quad(cfa, crs0, crs1, o.wd, o.ht, a, 2 * cx, 2 * cy, v);
+        st_h1_quad(o, 2 * cx, 2 * cy, v);
+      }
     }
   });
 }
@@ -823,9 +824,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 
 namespace {
 
-enum kind_t { K_HALF, K_DOWNCOV, K_DOWN, K_DNASM, K_DOUB, K_HL_HALF, K_HL_REDUCE, K_HL_ASM, K_HL_DOUB, K_GAUSS,
+enum kind_t { K_HALF, K_DOWNCOV, K_DOWN, K_DNASM, K_DOUB, K_DOUB_XT, K_HL_HALF, K_HL_REDUCE, K_HL_ASM, K_HL_DOUB, K_GAUSS,
               K_DEVELOP, K_DEVELOP_XT, K_PYR1, K_REDUCE, K_REDUCE_SPLIT, K_TAIL, K_ASM_SMALL, K_ASM, K_FINAL };
-const int kind_group[] = { 0, 1, 1, 2, 3, 4, 4, 4, 4, 5, 6, 6, 7, 8, 8, 8, 8, 8, 9 };
+const int kind_group[] = { 0, 1, 1, 2, 3, 3, 4, 4, 4, 4, 5, 6, 6, 7, 8, 8, 8, 8, 8, 9 };
 const char *group_name[VKDT_BATCH_STAGES] = { "half", "wavelet", "dnasm", "doub", "hilite", "gauss", "develop",
                                               "pyr1", "pyramid", "final" };
 
@@ -960,7 +961,7 @@ struct vkdt_batch_t
 
 // the device tables at the end of the scratch: image records, job lists
 // (at most one job per image and launch) and the tile counters
-#define BT_MAX_LAUNCH (10 + 2 * BT_LEVELS + 2 * HL_LEVELS)
+#define BT_MAX_LAUNCH (12 + 2 * BT_LEVELS + 2 * HL_LEVELS)
 static size_t table_bytes(int n)
 {
   return align256(sizeof(bt_img) * n) + align256(sizeof(bt_job) * (size_t)BT_MAX_LAUNCH * n)
@@ -1068,7 +1069,7 @@ static int build_image(bt_img &b, const vkdt_develop_image_t &d, const dims_t &m
 
 static int is_pixel_stage(int kind)
 {
-  return kind == K_HALF || kind == K_DNASM || kind == K_DOUB || kind == K_GAUSS || kind == K_HL_HALF ||
+  return kind == K_HALF || kind == K_DNASM || kind == K_DOUB || kind == K_DOUB_XT || kind == K_GAUSS || kind == K_HL_HALF ||
          kind == K_HL_ASM || kind == K_HL_DOUB;
 }
 
@@ -1085,7 +1086,7 @@ static int tiles_of(int kind, const dims_t &m, int level, int rows, int &tx)
     case K_HALF: case K_DNASM: w = m.qw; h = m.qh; th = BY * rows; break;
     case K_DOWNCOV: w = m.qw; h = m.qh; th = BY * COV_R; break;
     case K_DOWN: w = m.qw; h = m.qh; th = BY * DOWN_R; break;
-    case K_DOUB: w = m.block == 2 ? (m.W + 1) / 2 : m.W; h = m.block == 2 ? (m.H + 1) / 2 : m.H; th = BY * rows; break;
+    case K_DOUB: case K_DOUB_XT: w = (m.W + m.block - 1) / m.block; h = (m.H + m.block - 1) / m.block; th = BY * rows; break;
     case K_HL_HALF: w = m.qw; h = m.qh; th = BY * rows; break;
     case K_HL_REDUCE: w = m.hw[level]; h = m.hh[level]; break;
     case K_HL_ASM: w = m.hw[level]; h = m.hh[level]; th = BY * rows; break;
@@ -1119,8 +1120,8 @@ static void build_launches(vkdt_batch_t *b)
       if((kind == K_REDUCE || kind == K_REDUCE_SPLIT) && level >= std::min(m.nl, m.tail)) continue;
       if((kind == K_ASM || kind == K_ASM_SMALL) && level > std::min(m.nl - 2, m.tail - 1)) continue;
       if(kind == K_TAIL && m.tail >= m.nl) continue;
-      if(kind == K_DEVELOP && m.block == 3) continue;      // Bayer and X-Trans develop
-      if(kind == K_DEVELOP_XT && m.block != 3) continue;   // run as two launches
+      if((kind == K_DEVELOP || kind == K_DOUB) && m.block == 3) continue;      // Bayer and X-Trans
+      if((kind == K_DEVELOP_XT || kind == K_DOUB_XT) && m.block != 3) continue;   // run as two launches
       if(kind >= K_HL_HALF && kind <= K_HL_DOUB && !m.hl) continue;
       if(kind == K_HL_REDUCE && level > m.hn) continue;
       if(kind == K_HL_ASM && level >= m.hn) continue;
@@ -1139,6 +1140,7 @@ static void build_launches(vkdt_batch_t *b)
   for(int l = 1; l < 4; l++) add(K_DOWN, l, 0);
   add(K_DNASM, 0, 0);
   add(K_DOUB, 0, 0);
+  add(K_DOUB_XT, 0, 0);
   add(K_HL_HALF, 0, 0);
   for(int l = 1; l <= b->max_hn; l++) add(K_HL_REDUCE, l, 0);
   for(int l = b->max_hn - 1; l >= 0; l--) add(K_HL_ASM, l, 0);
@@ -1252,7 +1254,8 @@ static int enqueue(vkdt_batch_t *b, hipStream_t s, int timed)
         case K_DOWNCOV: hipLaunchKernelGGL(kb_downcov<P>, grid, blk, 0, s, a); break;
         case K_DOWN:    hipLaunchKernelGGL(kb_down<P>, grid, blk, 0, s, a); break;
         case K_DNASM:   hipLaunchKernelGGL(kb_dnasm<P>, grid, blk, 0, s, a, b->mats); break;
-        case K_DOUB:    hipLaunchKernelGGL(kb_doub<P>, grid, blk, 0, s, a); break;
+        case K_DOUB:    hipLaunchKernelGGL((kb_doub<0, P>), grid, blk, 0, s, a); break;
+        case K_DOUB_XT: hipLaunchKernelGGL((kb_doub<1, P>), grid, blk, 0, s, a); break;
         case K_HL_HALF: hipLaunchKernelGGL(kb_hl_half<P>, grid, blk, 0, s, a); break;
         case K_HL_REDUCE: hipLaunchKernelGGL(kb_hl_reduce<P>, grid, blk, 0, s, a); break;
         case K_HL_ASM:  hipLaunchKernelGGL(kb_hl_asm<P>, grid, blk, 0, s, a); break;

@@ -86,18 +86,16 @@ __global__ void __launch_bounds__(256) k_dn_assemble(dimg s0, dimg s1, dimg s2, 
   st_h4(out, x, y, dn_assemble_px(s0, s1, s2, s3, s4, a, m, x, y));
 }
 
-__global__ void __launch_bounds__(256) k_dn_doub(dimg in, dimg crs0, dimg crs1b, dimg out, dimg gm, dn_args a)
+// X-Trans mosaics: one 3x3 cell per thread (dn_doub_cell); the gain map is
+// Bayer's alone.  Bound by instructions; a texel per thread took 161 us at
+// 26 MP, the cell 131
+__global__ void __launch_bounds__(256) k_dn_doub_xtrans(dimg in, dimg crs0, dimg crs1b, dimg out, dn_args a)
 {
-  const int x = tid_x(), y = tid_y();
-  if(x >= out.wd || y >= out.ht) return;
-  float v = dn_doub_px(in, crs0, crs1b, out.wd, out.ht, a, x, y);
-  if(a.gainmap)
-  { // the block's centre on the half-resolution grid of the output
-    const float px = (0.5f + (float)((x + a.crop[0]) / 2)) / (float)(out.wd / 2);
-    const float py = (0.5f + (float)((y + a.crop[1]) / 2)) / (float)(out.ht / 2);
-    v *= dn_gain_at(gm, a, px, py, x, y);
-  }
-  st_h1(out, x, y, v);
+  const int cx = tid_x(), cy = tid_y();
+  if(3 * cx >= out.wd || 3 * cy >= out.ht) return;
+  float v[9];
+  dn_doub_cell(in, crs0, crs1b, out.wd, out.ht, a, cx, cy, v);
+  st_h1_cell(out, cx, cy, v);
 }
 
 // Bayer mosaics: one 2x2 block per thread (dn_doub_quad)
@@ -250,9 +248,8 @@ int launch_denoise_doub(const node_call &c)
   read_params(a, c);
   if(int e = read_gainmap(a, c, 4, pi[19], pf + 20, "denoise/doub gainmap")) return e;
   if(a.filters == 9)
-    hipLaunchKernelGGL(k_dn_doub, grid2d(c.wd, c.ht, 1), dim3(BX, BY), 0, c.stream,
-                       to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]), to_dimg(c.conn[3]),
-                       a.gainmap ? to_dimg(c.conn[4]) : dimg{}, a);
+    hipLaunchKernelGGL(k_dn_doub_xtrans, grid2d((c.wd + 2) / 3, (c.ht + 2) / 3, 1), dim3(BX, BY), 0, c.stream,
+                       to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]), to_dimg(c.conn[3]), a);
   else
     hipLaunchKernelGGL(k_dn_doub_bayer, grid2d((c.wd + 1) / 2, (c.ht + 1) / 2, 1), dim3(BX, BY), 0, c.stream,
                        to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]), to_dimg(c.conn[3]),

@@ -437,11 +437,12 @@ DEV float4 dn_assemble_px(const dimg &s0, const dimg &s1, const dimg &s2, const 
 }
 
 // doub.comp:80-116: the texel's shrinkage against the interpolated coarse
-// levels (channel ch of the upsampled level crs and of the finer one crs1,
-// alpha upw of the upsampled level, threshold T) and its normalisation
-DEV float dn_doub_tail(const dn_args &a, int ch, float crs, float crs1, float upw, float T, float blendw, float val)
+// levels (its channel of the upsampled level crs and of the finer one crs1,
+// alpha upw of the upsampled level, threshold T) and its normalisation by the
+// channel's levels
+DEV float dn_doub_tail(const dn_args &a, float black, float white, float inv_range, float crs, float crs1, float upw, float T,
+                       float blendw, float val)
 {
-  const float black = a.black[ch], white = a.white[ch], inv_range = a.inv_range[ch];
   float sig[3];
   noise_sigma(sig, a, black, inv_range, crs);
   blendw = 0.5f * (blendw + 1.0f);
@@ -456,37 +457,6 @@ DEV float dn_doub_tail(const dn_args &a, int ch, float crs, float crs1, float up
     val = mixf(val, fmaxf(0.0f, crs + sig[1] * signf_(wav) * mixf(fmaxf(0.0f, aw - T), aw, tt)), uw * blendw);
   }
   return fmaxf(0.0f, (val - black) * inv_range);
-}
-
-// doub.comp:35-116: one mosaic texel at full resolution
-DEV float dn_doub_px(const dimg &in, const dimg &crs0, const dimg &crs1b, int owd, int oht, const dn_args &a,
-                     int x, int y)
-{
-  const float sx = ((float)x + 0.5f) / (float)owd, sy = ((float)y + 0.5f) / (float)oht;
-  const float4 upsm = bilin_h4(crs0, sx * (float)crs0.wd, sy * (float)crs0.ht);
-  const float4 down = bilin_h4(crs1b, sx * (float)crs1b.wd, sy * (float)crs1b.ht);
-  int ch = 1;
-  float crs = upsm.y, crs1 = down.y;
-  float T = 0.5f * a.strength * upsm.w, blendw = a.luma;
-  if(a.filters == 9)
-  {
-    const int col = xtrans_colour(x, y);
-    if(col != 1)
-    {
-      ch = col;
-      crs = col == 2 ? upsm.z : upsm.x;
-      crs1 = col == 2 ? down.z : down.x;
-      blendw = 1.0f;
-      T *= frcp(fmaxf(1e-4f, upsm.w));
-    }
-  }
-  else
-  {
-    const int ox = x & 1, oy = y & 1;
-    if(ox == 0 && oy == 0)      { ch = 0; crs = upsm.x; crs1 = down.x; blendw = 1.0f; }
-    else if(ox == 1 && oy == 1) { ch = 2; crs = upsm.z; crs1 = down.z; blendw = 1.0f; }
-  }
-  return dn_doub_tail(a, ch, crs, crs1, upsm.w, T, blendw, centre_u16(in, x + a.crop[0], y + a.crop[1]));
 }
 
 // one axis of a bilinear texture() lookup: the two mirrored taps and the
@@ -536,31 +506,111 @@ DEV float dn_doub_bayer_texel(const dimg &crs0, const dimg &crs1b, const dn_args
 {
   const float2 up = bilin_h4_chan<CH, true>(crs0, ux, uy);
   const float dn = bilin_h4_chan<CH, false>(crs1b, dx, dy).x;
-  return dn_doub_tail(a, CH, up.x, dn, up.y, 0.5f * a.strength * up.y, CH == 1 ? a.luma : 1.0f, val);
+  return dn_doub_tail(a, a.black[CH], a.white[CH], a.inv_range[CH], up.x, dn, up.y, 0.5f * a.strength * up.y,
+                      CH == 1 ? a.luma : 1.0f, val);
 }
 
-// dn_doub_px on Bayer mosaics for the 2x2 block at even (x, y), v in row
-// order: the block's texels share their columns' and rows' taps, and each
+// the taps of N adjacent columns (or rows) from x0 of the full extent `full`
+// in a coarse image of extent n: texture() at (x + 0.5) / full
+template<int N>
+DEV void dn_doub_axes(bl_axis ax[N], int x0, int full, int n)
+{
+#pragma unroll
+  for(int k = 0; k < N; k++) ax[k] = bl_axis_at(((float)(x0 + k) + 0.5f) / (float)full * (float)n, n);
+}
+
+// doub.comp:35-116 on Bayer mosaics for the 2x2 block at even (x, y), v in
+// row order: the block's texels share their columns' and rows' taps, and each
 // interpolates only the channel its colour reads and alpha -- per channel
-// the same arithmetic, so the same values bit for bit
+// bilin_h4's arithmetic.  All addresses are formed before the first load:
+// mirroring branches, and a load after a branch waits for those before it
 DEV void dn_doub_quad(const dimg &in, const dimg &crs0, const dimg &crs1b, int owd, int oht, const dn_args &a,
                       int x, int y, float v[4])
 {
   bl_axis ux[2], uy[2], dx[2], dy[2];
-#pragma unroll
-  for(int k = 0; k < 2; k++)
-  {
-    const float sx = ((float)(x + k) + 0.5f) / (float)owd, sy = ((float)(y + k) + 0.5f) / (float)oht;
-    ux[k] = bl_axis_at(sx * (float)crs0.wd, crs0.wd);
-    dx[k] = bl_axis_at(sx * (float)crs1b.wd, crs1b.wd);
-    uy[k] = bl_axis_at(sy * (float)crs0.ht, crs0.ht);
-    dy[k] = bl_axis_at(sy * (float)crs1b.ht, crs1b.ht);
-  }
+  dn_doub_axes<2>(ux, x, owd, crs0.wd);
+  dn_doub_axes<2>(dx, x, owd, crs1b.wd);
+  dn_doub_axes<2>(uy, y, oht, crs0.ht);
+  dn_doub_axes<2>(dy, y, oht, crs1b.ht);
   const int cx = x + a.crop[0], cy = y + a.crop[1];
-  v[0] = dn_doub_bayer_texel<0>(crs0, crs1b, a, ux[0], uy[0], dx[0], dy[0], centre_u16(in, cx, cy));
-  v[1] = dn_doub_bayer_texel<1>(crs0, crs1b, a, ux[1], uy[0], dx[1], dy[0], centre_u16(in, cx + 1, cy));
-  v[2] = dn_doub_bayer_texel<1>(crs0, crs1b, a, ux[0], uy[1], dx[0], dy[1], centre_u16(in, cx, cy + 1));
-  v[3] = dn_doub_bayer_texel<2>(crs0, crs1b, a, ux[1], uy[1], dx[1], dy[1], centre_u16(in, cx + 1, cy + 1));
+  const int mx[2] = { mirror(cx, in.wd), mirror(cx + 1, in.wd) }, my[2] = { mirror(cy, in.ht), mirror(cy + 1, in.ht) };
+  float raw[4];
+#pragma unroll
+  for(int k = 0; k < 4; k++) raw[k] = ld_u16(in, mx[k & 1], my[k >> 1]);
+  v[0] = dn_doub_bayer_texel<0>(crs0, crs1b, a, ux[0], uy[0], dx[0], dy[0], raw[0]);
+  v[1] = dn_doub_bayer_texel<1>(crs0, crs1b, a, ux[1], uy[0], dx[1], dy[0], raw[1]);
+  v[2] = dn_doub_bayer_texel<1>(crs0, crs1b, a, ux[0], uy[1], dx[0], dy[1], raw[2]);
+  v[3] = dn_doub_bayer_texel<2>(crs0, crs1b, a, ux[1], uy[1], dx[1], dy[1], raw[3]);
+}
+
+// bilinear red (or with `blue` blue) channel and, with ALPHA, channel 3: the
+// channel's word is selected before it is converted
+template<bool ALPHA>
+DEV float2 bilin_h4_rb(const dimg &b, const bl_axis &ax, const bl_axis &ay, bool blue)
+{
+  const __half *p = (const __half *)b.p;
+  const long r0 = (long)ay.i0 * b.pitch, r1 = (long)ay.i1 * b.pitch;
+  uint2 u[4] = { *(const uint2 *)(p + 4 * (r0 + ax.i0)), *(const uint2 *)(p + 4 * (r0 + ax.i1)),
+                 *(const uint2 *)(p + 4 * (r1 + ax.i0)), *(const uint2 *)(p + 4 * (r1 + ax.i1)) };
+  const float s = ax.f, t = ay.f;
+  float c[4], w[4];
+#pragma unroll
+  for(int k = 0; k < 4; k++)
+  {
+    c[k] = h4_chan<0>(make_uint2(blue ? u[k].y : u[k].x, 0u));
+    w[k] = ALPHA ? h4_chan<3>(u[k]) : 0.0f;
+  }
+  float2 r;
+  r.x = (c[0] * (1.f - s) + c[1] * s) * (1.f - t) + (c[2] * (1.f - s) + c[3] * s) * t;
+  r.y = ALPHA ? (w[0] * (1.f - s) + w[1] * s) * (1.f - t) + (w[2] * (1.f - s) + w[3] * s) * t : 0.0f;
+  return r;
+}
+
+// the same on X-Trans mosaics for the 3x3 cell (cx, cy), v in row order: five
+// green texels, and two each of red and blue that swap with the cell's
+// parity.  A texel per thread formed its own axes (four divisions, eight
+// mirrored taps) and interpolated eight channels of which it used three
+DEV void dn_doub_cell(const dimg &in, const dimg &crs0, const dimg &crs1b, int owd, int oht, const dn_args &a,
+                      int cx, int cy, float v[9])
+{
+  bl_axis ux[3], uy[3], dx[3], dy[3];
+  dn_doub_axes<3>(ux, 3 * cx, owd, crs0.wd);
+  dn_doub_axes<3>(dx, 3 * cx, owd, crs1b.wd);
+  dn_doub_axes<3>(uy, 3 * cy, oht, crs0.ht);
+  dn_doub_axes<3>(dy, 3 * cy, oht, crs1b.ht);
+  int mx[3], my[3];
+#pragma unroll
+  for(int k = 0; k < 3; k++)
+  {
+    mx[k] = mirror(3 * cx + k + a.crop[0], in.wd);
+    my[k] = mirror(3 * cy + k + a.crop[1], in.ht);
+  }
+  float raw[9];
+#pragma unroll
+  for(int k = 0; k < 9; k++) raw[k] = ld_u16(in, mx[k % 3], my[k / 3]);
+  const bool odd = ((cx + cy) & 1) != 0;
+#pragma unroll
+  for(int j = 0; j < 3; j++)
+#pragma unroll
+    for(int i = 0; i < 3; i++)
+    {
+      const int k = 3 * j + i;
+      if(((i + j) & 1) == 0)
+      {
+        const float2 up = bilin_h4_chan<1, true>(crs0, ux[i], uy[j]);
+        const float dn = bilin_h4_chan<1, false>(crs1b, dx[i], dy[j]).x;
+        v[k] = dn_doub_tail(a, a.black[1], a.white[1], a.inv_range[1], up.x, dn, up.y, 0.5f * a.strength * up.y, a.luma, raw[k]);
+      }
+      else
+      { // xtrans_colour
+        const bool blue = odd ^ (j == 1);
+        const float2 up = bilin_h4_rb<true>(crs0, ux[i], uy[j], blue);
+        const float dn = bilin_h4_rb<false>(crs1b, dx[i], dy[j], blue).x;
+        v[k] = dn_doub_tail(a, blue ? a.black[2] : a.black[0], blue ? a.white[2] : a.white[0],
+                            blue ? a.inv_range[2] : a.inv_range[0], up.x, dn, up.y,
+                            0.5f * a.strength * up.y * frcp(fmaxf(1e-4f, up.y)), 1.0f, raw[k]);
+      }
+    }
 }
 
 // store the 2x2 block at even (x, y) of an f16 plane, v in row order: each
@@ -579,6 +629,17 @@ DEV void st_h1_quad(const dimg &o, int x, int y, const float v[4])
       st_h1(o, x, y + r, v[2 * r]);
       if(x + 1 < o.wd) st_h1(o, x + 1, y + r, v[2 * r + 1]);
     }
+  }
+}
+
+// store the 3x3 cell (cx, cy) of an f16 plane, v in row order
+DEV void st_h1_cell(const dimg &o, int cx, int cy, const float v[9])
+{
+#pragma unroll
+  for(int k = 0; k < 9; k++)
+  {
+    const int x = 3 * cx + k % 3, y = 3 * cy + k / 3;
+    if(x < o.wd && y < o.ht) st_h1(o, x, y, v[k]);
   }
 }
 
