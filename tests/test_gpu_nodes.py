@@ -118,3 +118,24 @@ def test_doub_blocks(hip, kind, W, H, cx, cy):
                   conn=["raw", "s0", "half", "dn"], wd=W, ht=H, dp=1, out=3)]
     host = parity.run_gpu_graph(hip, bufs, nodes, raw)
     parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))
+
+
+@pytest.mark.parametrize("W", [5, 67, 1030])
+@pytest.mark.parametrize("par", [(0.12, 1.0, 1.0, 0.2), (0.05, 1.6, 0.3, 1.0), (0.5, 0.2, 2.0, 0.0), (0.25, -0.5, -0.5, -0.3)])
+def test_llap_curve(hip, par, W):
+    """llap/curve over values on the gammas, at the joint of its two parts
+    (2 sigma from a gamma), far out and negative; few and many curves, odd
+    extents: against the oracle"""
+    import numpy as np
+    H, ng = 3, 10
+    rng = np.random.default_rng(W)
+    lum = rng.uniform(-0.2, 1.4, size=(H, W))
+    lum[0, ::2] = rng.integers(0, ng, lum[0, ::2].shape) / (ng - 1.0)
+    lum[1, ::2] = lum[0, 0] + 2.0 * par[0]
+    lum[2, 0], lum[2, 2] = 40.0, -3.0
+    raw = np.repeat(lum[:, :, None], 4, axis=2).astype(np.float16)
+    bufs = {"raw": (W, H, 4, gs.F16, 1), "pyr0": (W, H, 1, gs.F16, ng + 1)}
+    nodes = [dict(module="llap", kernel="curve", pc=gs.mixed_blob([("i", ng)]), params=gs.f32blob(list(par)),
+                  conn=["raw", "pyr0"], wd=W, ht=H, dp=1, out=1)]
+    host = parity.run_gpu_graph(hip, bufs, nodes, raw)
+    parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))
