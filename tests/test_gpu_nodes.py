@@ -139,3 +139,36 @@ def test_llap_curve(hip, par, W):
                   conn=["raw", "pyr0"], wd=W, ht=H, dp=1, out=1)]
     host = parity.run_gpu_graph(hip, bufs, nodes, raw)
     parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))
+
+
+@pytest.mark.parametrize("ng,step", [(2, 1), (10, 1), (10, 16), (32, 1)])
+def test_llap_assemble_planes(hip, ng, step):
+    """llap/assemble above the extent of the small kernel with tiles that
+    select a few of the planes, all of them and more than are held at once,
+    on every gamma (where the choice of the plane changes), partial tiles in
+    both directions, and both kinds of coarse level: against the oracle"""
+    import numpy as np
+    rng = np.random.default_rng(ng)
+    W, H = 1037, 531
+    lum = rng.uniform(-0.1, 1.2, size=(H // step + 1, W // step + 1)).repeat(step, 0).repeat(step, 1)[:H, :W]
+    lum[::3, ::5] = np.round(lum[::3, ::5] * (ng - 1)) / (ng - 1)
+    raw = np.repeat(lum[:, :, None], 4, axis=2).astype(np.float16)
+    w, h = [W], [H]
+    for l in range(2):
+        w.append((w[-1] - 1) // 2 + 1)
+        h.append((h[-1] - 1) // 2 + 1)
+    bufs = {"raw": (W, H, 4, gs.F16, 1)}
+    for l in range(3):
+        bufs[f"pyr{l}"] = (w[l], h[l], 1, gs.F16, ng + 1)
+    bufs.update(out0=(W, H, 1, gs.F16, 1), out1=(w[1], h[1], 1, gs.F16, 1), only=(W, H, 1, gs.F16, 1))
+    par = gs.f32blob([0.12, 1.2, 0.8, 0.3])
+    node = lambda k, pc, conn, wd, ht, dp=1: dict(module="llap", kernel=k, pc=pc, params=par, conn=conn, wd=wd, ht=ht, dp=dp,
+                                                  out=len(conn) - 1)
+    asm = lambda first: gs.mixed_blob([("i", ng), ("i", first)])
+    nodes = [node("curve", gs.mixed_blob([("i", ng)]), ["raw", "pyr0"], W, H),
+             node("reduce", None, ["pyr0", "pyr1"], w[1], h[1], ng + 1), node("reduce", None, ["pyr1", "pyr2"], w[2], h[2], ng + 1),
+             node("assemble", asm(1), ["pyr0", "pyr1", "pyr2", "out1"], w[1], h[1]),
+             node("assemble", asm(0), ["out1", "pyr0", "pyr1", "out0"], W, H),
+             node("assemble", asm(1), ["pyr0", "pyr0", "pyr1", "only"], W, H)]
+    host = parity.run_gpu_graph(hip, bufs, nodes, raw)
+    parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))

@@ -662,7 +662,7 @@ __global__ void __launch_bounds__(256) kb_asm(bt_launch L)
     }
     const int xc = min(x, fine.wd - 1);
     ll_assemble_tile<ASM_R>(coarse, l1, fine.wd, fine.ht, a, first, X0, Y0, tile, lims, v,
-                            [&](int k, int p) {
+                            [&](int k, int p, float) {
                               return ld_h1(fine, xc, min(Y0 + (int)threadIdx.y + BY * k, fine.ht - 1), p);
                             }, res);
 #pragma unroll
@@ -810,7 +810,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
       v[k] = r16(yl[k]);
     }
     ll_assemble_tile<ASM_R>(coarse, l1, f.wd, f.ht, a, first, X0, Y0, tile, lims, v,
-                            [&](int k, int p) { return r16(ll_curve(yl[k], a.gam[p], a)); }, res);
+                            [&](int k, int, float g) { return r16(ll_curve(yl[k], g, a)); }, res);
 #pragma unroll
     for(int k = 0; k < ASM_R; k++)
     {
@@ -1134,7 +1134,7 @@ static void build_launches(vkdt_batch_t *b)
     }
     if(L.njob) { b->seq.push_back(L); b->nctr += NUM_XCD; }
   };
-  const size_t asm_lds = sizeof(float) * (b->max_ng + 1) * AS_TN(ASM_R);
+  const size_t asm_lds = sizeof(float) * AS_TN(ASM_R);
   add(K_HALF, 0, 0);
   add(K_DOWNCOV, 0, 0);
   for(int l = 1; l < 4; l++) add(K_DOWN, l, 0);

@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(256) k_ll_reduce(dimg in, dimg out, int vec)
 
 __global__ void __launch_bounds__(256) k_ll_assemble(dimg coarse, dimg l0, dimg l1, dimg out, ll_args a)
 {
-  extern __shared__ float tile[];             // up to (num_gamma + 1) slots of AS_TN(AS_R)
+  extern __shared__ float tile[];             // AS_TN(AS_R)
   __shared__ int lims[2];
   const int2 t = xcd_block();
   const int X0 = t.x * BX, Y0 = t.y * (BY * AS_R);
@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(256) k_ll_assemble(dimg coarse, dimg l0, dimg 
   }
   const int xc = min(x, out.wd - 1);
   ll_assemble_tile<AS_R>(coarse, l1, out.wd, out.ht, a, a.first, X0, Y0, tile, lims, v,
-                         [&](int k, int p) { return ld_h1(l0, xc, min(Y0 + (int)threadIdx.y + 4 * k, out.ht - 1), p); },
+                         [&](int k, int p, float) { return ld_h1(l0, xc, min(Y0 + (int)threadIdx.y + 4 * k, out.ht - 1), p); },
                          res);
 #pragma unroll
   for(int k = 0; k < AS_R; k++)
@@ -253,7 +253,7 @@ int launch_llap_assemble(const node_call &c)
                        to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]), to_dimg(c.conn[3]), a);
     return launch_post("llap/assemble");
   }
-  const size_t lds = sizeof(float) * (a.num_gamma + 1) * AS_TN(AS_R);
+  const size_t lds = sizeof(float) * AS_TN(AS_R);
   const dim3 grid((c.wd + BX - 1) / BX, (c.ht + BY * AS_R - 1) / (BY * AS_R), 1);
   hipLaunchKernelGGL(k_ll_assemble, grid, dim3(BX, BY), lds, c.stream,
                      to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]), to_dimg(c.conn[3]), a);

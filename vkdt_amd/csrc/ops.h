@@ -1151,13 +1151,28 @@ DEV float ll_curve(float x, float g, const ll_args &a)
   return f32_value(__builtin_fmaf(a.clarity * c, fexp2(c * c * a.nc3), g + (pos ? v : -v)));
 }
 
-// llap.glsl:16-21: first curve index above v (1..num_gamma-1)
-DEV int gamma_hi_from_v(float v, const ll_args &a)
+// llap.glsl:16-21: the first curve index above v (1..num_gamma-1), that
+// curve's and the previous one's gamma, and v's place between them.  The
+// gammas are equidistant: the scaled value is the index or, rounded, its
+// neighbour, so two loads that depend on nothing take the place of a search
+// that waits for a gamma before it reads the next
+struct ll_pos { int hi; float g0, g1; };
+DEV ll_pos ll_pos_of(float v, const ll_args &a)
 {
-  int hi = 1;
-  for(; hi < a.num_gamma - 1 && a.gam[hi] <= v; hi++);
-  return hi;
+  const int last = a.num_gamma - 2;
+  int i = (int)fminf(fmaxf(v * (float)(a.num_gamma - 1), 0.0f), (float)last);
+  ll_pos q = { i + 1, a.gam[i], a.gam[i + 1] };
+  const bool dn = i > 0 && q.g0 > v, up = i < last && q.g1 <= v;
+  if(dn || up)
+  {
+    i += up ? 1 : -1;
+    q.hi = i + 1;
+    q.g0 = a.gam[i];
+    q.g1 = a.gam[i + 1];
+  }
+  return q;
 }
+DEV float ll_between(const ll_pos &q, float v) { return clampf((v - q.g0) / (q.g1 - q.g0), 0.0f, 1.0f); }
 
 // luminance of the clamped rgb (curve.comp:72)
 DEV float ll_lum(float4 t)
@@ -1262,20 +1277,29 @@ DEV void ll_reduce_px4(const dimg &in, const dimg &out, int planes, int x0, int 
 // owns the texels (X0+tx, Y0+ty+4k), k < R.  Every fine texel expands
 // (sample_soft at o/2+.5 = (1/2 1/2 1 1/2 1/2)/3 even, (1 1/2 1/2 1)/3 odd,
 // per axis) the coarse reconstruction and the two curve planes its
-// luminance selects.  The tile's coarse footprint is staged in LDS only for
+// luminance selects.  The tile's coarse rows are expanded along x once for
 // the planes some texel of the tile selects (the block's [min hi-1, max hi]
-// range), plus the coarse reconstruction in the last slot.
-//   first        the coarsest level: expand the luminance plane of l1
-//                instead of a coarse reconstruction
-//   v[k]         the fine luminance plane at the thread's texel k
-//   plane(k, p)  the fine curve plane p there; called for every k, also for
-//                texels outside (owd, oht), so it must clamp its address
+// range) and the coarse reconstruction, and held in LDS; a texel then expands
+// its three planes along y.  A texel that expanded both axes by itself read
+// 75 values from LDS and combined them in 72 operations; it reads 15 and
+// shares 3/4 of a row of each plane.  A lane loads one value of two rows and
+// takes its five taps from the wave's other lanes, so the rows need no
+// staging, and two rows of binary16 travel as one word.  kb_final of ten
+// stills (283 MP) 2492 -> 1842 us, kb_asm 693 -> 538, k_ll_assemble's large
+// levels at 24 MP 236 -> 186.
+//   first          the coarsest level: expand the luminance plane of l1
+//                  instead of a coarse reconstruction
+//   v[k]           the fine luminance plane at the thread's texel k
+//   plane(k, p, g) the fine curve plane p (gamma g) there; called for every k,
+//                  also for texels outside (owd, oht), so it must clamp its
+//                  address
 // Texels outside (owd, oht) get no result.  Loads are issued unconditionally
-// (clamped addresses) so that the rows' loads and the staging's are in
-// flight together instead of one memory latency each.
-#define AS_TX 36                       // coarse tile width for a 64 wide fine tile (+-2 halo)
-#define AS_TY(R) (2 * (R) + 4)         // coarse tile height for a 4R high fine tile
-#define AS_TN(R) (AS_TX * AS_TY(R))
+// (clamped addresses) so that the rows' loads and the texels' are in flight
+// together instead of one memory latency each.
+#define AS_TX 36                       // coarse columns of a 64 wide fine tile (+-2 halo)
+#define AS_TY(R) (2 * (R) + 4)         // coarse rows of a 4R high fine tile
+#define AS_SLOTS 6                     // planes held at once: 18 KB, so that LDS allows 8 waves a SIMD
+#define AS_TN(R) (AS_SLOTS * AS_TY(R) * BX)
 
 // The expand filter's five taps along one axis: weights 1/2 1/2 1 1/2 1/2 at
 // even texels and 0 1 1/2 1/2 1 at odd ones, summed from zero in tap order
@@ -1306,22 +1330,23 @@ template<int R, typename PlaneAt>
 DEV void ll_assemble_tile(const dimg &coarse, const dimg &l1, int owd, int oht, const ll_args &a, int first,
                           int X0, int Y0, float *tile, int *lims, const float v[R], PlaneAt plane, float res[R])
 {
-  constexpr int CN = AS_TN(R);
-  const int ng = a.num_gamma;
-  const int x = X0 + threadIdx.x;
+  constexpr int RY = AS_TY(R);
+  const int ng = a.num_gamma, lane = threadIdx.x, w = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int x = X0 + lane;
   if(threadIdx.x == 0 && threadIdx.y == 0) { lims[0] = LL_MAX_GAMMA; lims[1] = 0; }
   int hi[R];
-  float pv0[R], pv1[R];
+  float pv0[R], pv1[R], al[R];
   int lo_t = LL_MAX_GAMMA, hi_t = 0;
 #pragma unroll
   for(int k = 0; k < R; k++)
   {
-    const int y = Y0 + threadIdx.y + 4 * k;
-    hi[k] = gamma_hi_from_v(v[k], a);
-    // issued before the staging so their latency overlaps it
-    pv0[k] = plane(k, hi[k] - 1);
-    pv1[k] = plane(k, hi[k]);
-    if(x < owd && y < oht)
+    const ll_pos q = ll_pos_of(v[k], a);
+    hi[k] = q.hi;
+    al[k] = ll_between(q, v[k]);
+    // issued before the rows' loads so their latency overlaps those
+    pv0[k] = plane(k, q.hi - 1, q.g0);
+    pv1[k] = plane(k, q.hi, q.g1);
+    if(x < owd && Y0 + w + BY * k < oht)
     {
       lo_t = min(lo_t, hi[k] - 1);
       hi_t = max(hi_t, hi[k]);
@@ -1330,66 +1355,66 @@ DEV void ll_assemble_tile(const dimg &coarse, const dimg &l1, int owd, int oht, 
   lo_t = wave_min(lo_t);
   hi_t = wave_max(hi_t);
   __syncthreads();
-  if(threadIdx.x == 0) { atomicMin(&lims[0], lo_t); atomicMax(&lims[1], hi_t); }
+  if(lane == 0) { atomicMin(&lims[0], lo_t); atomicMax(&lims[1], hi_t); }
   __syncthreads();
-  const int p0 = lims[0], np = lims[1] - p0 + 1;
-  const int cx0 = X0 / 2 - 2, cy0 = Y0 / 2 - 2;
-  const int tid = threadIdx.y * BX + threadIdx.x;
-  // slots 0..np-1: planes p0.. of l1; slot np: the coarse reconstruction
-  // (l1's plane ng on the first assemble).  Four loads per thread and pass.
-  const int n = (np + 1) * CN;
-  constexpr int S = BX * BY, U = 4;
-  for(int i0 = tid; i0 < n; i0 += U * S)
+  // slot 0: the coarse reconstruction (l1's plane ng on the first assemble),
+  // slot s: plane p0 + s - 1 of l1
+  const int p0 = __builtin_amdgcn_readfirstlane(lims[0]), n = __builtin_amdgcn_readfirstlane(lims[1]) - p0 + 2;
+  const int gx = mirror(X0 / 2 - 2 + min(lane, AS_TX - 1), l1.wd), cy0 = Y0 / 2 - 2;
+  const int tap = 4 * (lane >> 1);   // the lane that holds the tap at offset -2, in bytes
+  const ll_expand_w wx = ll_expand_weights(lane & 1), wy = ll_expand_weights(w & 1);
+  for(int s0 = 0; s0 < n; s0 += AS_SLOTS)
   {
-    float c[U];
-#pragma unroll
-    for(int u = 0; u < U; u++)
+    const int m = min(AS_SLOTS, n - s0), pairs = m * (RY / 2);
+    if(s0) __syncthreads();   // the slots before these are read
+    constexpr int U = 2;      // row pairs in flight
+    for(int i0 = w; i0 < pairs; i0 += U * BY)
     {
-      const int idx = min(i0 + u * S, n - 1);
-      const int sl = idx / CN, r = idx - sl * CN;
-      const int ty = r / AS_TX, tx = r - ty * AS_TX;
-      const int gx = mirror(cx0 + tx, l1.wd), gy = mirror(cy0 + ty, l1.ht);
-      const bool fc = sl >= np && first <= 0;
-      const __half *src = fc ? (const __half *)coarse.p : (const __half *)l1.p;
-      const long off = fc ? (long)gy * coarse.pitch + gx
-                          : (long)(sl < np ? p0 + sl : ng) * l1.pstride + (long)gy * l1.pitch + gx;
-      c[u] = h2f(src[off]);
+      union pair { __half e[2]; int u; } c[U];
+#pragma unroll
+      for(int u = 0; u < U; u++)
+      {
+        const int i = min(i0 + u * BY, pairs - 1), sl = s0 + i / (RY / 2), y = cy0 + 2 * (i % (RY / 2));
+        const dimg &b = sl == 0 && first <= 0 ? coarse : l1;
+        const __half *src = (const __half *)b.p + (sl == 0 ? (first <= 0 ? 0 : ng) : p0 + sl - 1) * b.pstride;
+        c[u].e[0] = src[(long)mirror(y, l1.ht) * b.pitch + gx];
+        c[u].e[1] = src[(long)mirror(y + 1, l1.ht) * b.pitch + gx];
+      }
+#pragma unroll
+      for(int u = 0; u < U; u++)
+      {
+        if(i0 + u * BY >= pairs) break;
+        pair t[5];
+#pragma unroll
+        for(int q = 0; q < 5; q++) t[q].u = __builtin_amdgcn_ds_bpermute(tap + 4 * q, c[u].u);
+        // twice the horizontal sums
+#pragma unroll
+        for(int h = 0; h < 2; h++)
+          tile[(2 * (i0 + u * BY) + h) * BX + lane] =
+            ll_expand5(wx, h2f(t[0].e[h]), h2f(t[1].e[h]), h2f(t[2].e[h]), h2f(t[3].e[h]), h2f(t[4].e[h]));
+      }
     }
+    __syncthreads();
 #pragma unroll
-    for(int u = 0; u < U; u++)
-      if(i0 + u * S < n) tile[i0 + u * S] = c[u];
-  }
-  __syncthreads();
-  const ll_expand_w wx = ll_expand_weights(x & 1);
-  const int lx = x / 2 - cx0 - 2;   // tile column of offset -2
-#pragma unroll
-  for(int k = 0; k < R; k++)
-  {
-    const int y = Y0 + threadIdx.y + 4 * k;
-    if(x >= owd || y >= oht) continue;
-    const ll_expand_w wy = ll_expand_weights(y & 1);
-    const int ly = y / 2 - cy0 - 2;
-    const int h = hi[k];
-    const float al = clampf((v[k] - a.gam[h - 1]) / (a.gam[h] - a.gam[h - 1]), 0.0f, 1.0f);
-    const float *tc = tile + np * CN, *t0 = tile + (h - 1 - p0) * CN, *t1 = tile + (h - p0) * CN;
-    // rows: twice the horizontal sums; columns: twice again, so the
-    // reference's weighted sums are a quarter of these, exactly
-    float sc[5], s0[5], s1[5];
-#pragma unroll
-    for(int j = 0; j < 5; j++)
+    for(int k = 0; k < R; k++)
     {
-      const int o = (ly + j) * AS_TX + lx;
-      sc[j] = ll_expand5(wx, tc[o], tc[o + 1], tc[o + 2], tc[o + 3], tc[o + 4]);
-      s0[j] = ll_expand5(wx, t0[o], t0[o + 1], t0[o + 2], t0[o + 3], t0[o + 4]);
-      s1[j] = ll_expand5(wx, t1[o], t1[o + 1], t1[o + 2], t1[o + 3], t1[o + 4]);
+      // columns: twice again, so the reference's weighted sums are a quarter
+      // of these, exactly.  Slots not held now are read clamped and dropped
+      const float *c = tile + ((w + BY * k) >> 1) * BX + lane;
+      const auto expand = [&](int s) {
+        const float *q = c + s * (RY * BX);
+        return 0.25f * ll_expand5(wy, q[0], q[BX], q[2 * BX], q[3 * BX], q[4 * BX]);
+      };
+      const float s = 1.0f / 9.0f;
+      if(s0 == 0) res[k] = expand(0) * s;
+      const int q0 = hi[k] - p0 - s0, q1 = q0 + 1;
+      const float lv0 = pv0[k] - expand(min(max(q0, 0), m - 1)) * s;
+      const float r0 = res[k] + lv0 * (1.0f - al[k]);
+      res[k] = (unsigned)q0 < (unsigned)m ? r0 : res[k];
+      const float lv1 = pv1[k] - expand(min(max(q1, 0), m - 1)) * s;
+      const float r1 = res[k] + lv1 * al[k];
+      res[k] = (unsigned)q1 < (unsigned)m ? r1 : res[k];
     }
-    const float rs = 0.25f * ll_expand5(wy, sc[0], sc[1], sc[2], sc[3], sc[4]);
-    const float e0 = 0.25f * ll_expand5(wy, s0[0], s0[1], s0[2], s0[3], s0[4]);
-    const float e1 = 0.25f * ll_expand5(wy, s1[0], s1[1], s1[2], s1[3], s1[4]);
-    const float s = 1.0f / 9.0f;
-    const float lv0 = pv0[k] - e0 * s;
-    const float lv1 = pv1[k] - e1 * s;
-    res[k] = rs * s + lv0 * (1.0f - al) + lv1 * al;
   }
 }
 
@@ -1405,10 +1430,11 @@ template<typename Fine, typename Lo, typename Rec>
 DEV float ll_assemble_direct(const ll_args &a, int first, int cw, int ch, int x, int y, Fine fine, Lo lo, Rec rec)
 {
   const float v = fine(a.num_gamma);
-  const int h = gamma_hi_from_v(v, a);
+  const ll_pos q = ll_pos_of(v, a);
+  const int h = q.hi;
   const float pv0 = fine(h - 1), pv1 = fine(h);
   const ll_expand_w wx = ll_expand_weights(x & 1), wy = ll_expand_weights(y & 1);
-  const float al = clampf((v - a.gam[h - 1]) / (a.gam[h] - a.gam[h - 1]), 0.0f, 1.0f);
+  const float al = ll_between(q, v);
   float sc[5], s0[5], s1[5];
 #pragma unroll
   for(int j = 0; j < 5; j++)
