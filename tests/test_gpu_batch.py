@@ -94,6 +94,15 @@ def test_xtrans_tiles_equal_the_plain_graph(tmp_path, hip, W, Hh, kw):
     c[0].close()
 
 
+@pytest.mark.parametrize("W,Hh", [(16, 12), (126, 64), (128, 66), (250, 130), (382, 18)])
+def test_first_reduction_tiles_equal_the_plain_graph(tmp_path, hip, W, Hh):
+    """the pyramid's first level, made from the image by waves of 63 x 8
+    outputs: one, exactly full, one column and row over, partial ones"""
+    c = plain_and_planned(tmp_path, "bayer", W, Hh, 63, dict())
+    check_equal(batch.develop([c[0]], [c[1]]), [c], f"{W}x{Hh}")
+    c[0].close()
+
+
 def test_alone_equals_in_the_mix(cases):
     """each image developed in a batch of one equals its plain run too"""
     for i, c in enumerate(cases):

@@ -563,18 +563,21 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(XT ? 5
 
 // ---- llap ------------------------------------------------------------------
 
-// level-1 tile (64 x 4) of curve + reduce: the footprint (2X0-1 .. 2X0+128,
-// 2Y0-1 .. 2Y0+8, mirrored) of every level-0 plane is evaluated once into
-// LDS as binary16 -- the values the curve node stores -- and reduced from
-// there in reduce.comp's order
-#define P1_W (2 * BX + 2)
-#define P1_H (2 * BY + 1)
-#define P1_N (P1_W * P1_H)
+// curve + reduce, level 1 from filmcurv's output: a wave owns P1_W columns of
+// P1_R output rows and holds the luminance of their footprint, two columns a
+// lane (lane 0 those left of the tile), in registers.  Per plane every value
+// is evaluated once, rounded to binary16 as the curve node stores it, and
+// summed in reduce.comp's order; the third tap of a row is the previous lane's
+// and a row's sum is carried to the next output, so there is neither LDS nor a
+// barrier.  Bound by the curves' instructions: ten stills of 283 MP 2306 ->
+// 1705 us against a footprint staged in LDS (8 rows; 6 and 4 are 4 and 6 %
+// slower, with more footprint evaluated twice)
+#define P1_W (BX - 1)
+#define P1_R 8
 
 template<int P>
 __global__ void __launch_bounds__(256) kb_pyr1(bt_launch L)
 {
-  extern __shared__ __half pl[];   // (num_gamma + 1) x P1_N
   __shared__ ll_args a;
   dimg f, o;
   bt_tiles<P>(L, [&](const bt_job &jb) {
@@ -582,28 +585,49 @@ __global__ void __launch_bounds__(256) kb_pyr1(bt_launch L)
     lds_copy(a, im.ll);
     f = rfl(im.film); o = rfl(im.lp[1]);
   }, [&](const bt_job &jb, int lt) {
-    const int ng = a.num_gamma;
-    const int X0 = (lt % jb.tiles_x) * BX, Y0 = (lt / jb.tiles_x) * BY;
-    const int tid = threadIdx.y * BX + threadIdx.x;
-    for(int i = tid; i < P1_N; i += BX * BY)
+    const int ng = rfl(a.num_gamma), lane = threadIdx.x;
+    const int y = (lt / jb.tiles_x) * (BY * P1_R) + rfl((int)threadIdx.y) * P1_R;
+    const int x = (lt % jb.tiles_x) * P1_W - 1 + lane;
+    if(y >= o.ht) return;
+    const int rows = min(P1_R, o.ht - y);
+    const bool own = lane > 0 && x < o.wd;
+    const int xa = mirror(2 * x, f.wd), xb = mirror(2 * x + 1, f.wd);
+    const ll_curve_k k = ll_curve_load(a);
+    float la[2 * P1_R + 1], lb[2 * P1_R + 1];
+#pragma unroll
+    for(int j = 0; j < 2 * P1_R + 1; j++)
     {
-      const int ty = i / P1_W, tx = i - ty * P1_W;
-      const float yl = ll_lum(ld_h4(f, mirror(2 * X0 - 1 + tx, f.wd), mirror(2 * Y0 - 1 + ty, f.ht)));
-      for(int p = 0; p < ng; p++) pl[p * P1_N + i] = f2h(ll_curve(yl, a.gam[p], a));
-      pl[ng * P1_N + i] = f2h(yl);
+      const int fy = mirror(2 * y - 1 + j, f.ht);
+      la[j] = ll_lum(ld_h4(f, xa, fy));
+      lb[j] = ll_lum(ld_h4(f, xb, fy));
     }
-    __syncthreads();
-    const int x = X0 + threadIdx.x, y = Y0 + threadIdx.y;
-    if(x >= o.wd || y >= o.ht) return;
-    const int c = 2 * threadIdx.y * P1_W + 2 * threadIdx.x;   // local (2x-1, 2y-1)
-    for(int p = 0; p <= ng; p++)
+    __half *out = (__half *)o.p + (long)y * o.pitch + x;
+    const auto reduce = [&](auto value) {
+      // [1 2 1] of a row; doubling is exact, so the sums may be fused
+      const auto row = [&](int j) {
+        const __half ea = f2h(value(la[j])), eb = f2h(value(lb[j]));
+        const __half el = __builtin_bit_cast(__half, (short)__builtin_amdgcn_update_dpp(0, (int)__builtin_bit_cast(unsigned short, eb),
+                                                                                       0x138 /* wave_shr:1 */, 0xf, 0xf, false));
+        return __builtin_fmaf(2.0f, h2f(ea), h2f(el)) + h2f(eb);
+      };
+      float s0 = row(0);
+      __half *q = out;
+#pragma unroll
+      for(int r = 0; r < P1_R; r++)
+      {
+        const float s1 = row(2 * r + 1), s2 = row(2 * r + 2);
+        if(own && r < rows) *q = f2h((__builtin_fmaf(2.0f, s1, s0) + s2) * (1.0f / 16.0f));
+        q += o.pitch;
+        s0 = s2;
+      }
+      out += o.pstride;
+    };
+    for(int p = 0; p < ng; p++)
     {
-      const __half *q = pl + p * P1_N + c;
-      const float s0 = h2f(q[0]) + 2.0f * h2f(q[1]) + h2f(q[2]);
-      const float s1 = h2f(q[P1_W]) + 2.0f * h2f(q[P1_W + 1]) + h2f(q[P1_W + 2]);
-      const float s2 = h2f(q[2 * P1_W]) + 2.0f * h2f(q[2 * P1_W + 1]) + h2f(q[2 * P1_W + 2]);
-      st_h1(o, x, y, (s0 + 2.0f * s1 + s2) * (1.0f / 16.0f), p);
+      const float g = a.gam[p];
+      reduce([&](float l) { return ll_curve(l, g, k); });
     }
+    reduce([](float l) { return l; });
   });
 }
 
@@ -809,8 +833,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
       yl[k] = ll_lum(t[k]);
       v[k] = r16(yl[k]);
     }
+    const ll_curve_k ck = ll_curve_load(a);
     ll_assemble_tile<ASM_R>(coarse, l1, f.wd, f.ht, a, first, X0, Y0, tile, lims, v,
-                            [&](int k, int, float g) { return r16(ll_curve(yl[k], g, a)); }, res);
+                            [&](int k, int, float g) { return r16(ll_curve(yl[k], g, ck)); }, res);
 #pragma unroll
     for(int k = 0; k < ASM_R; k++)
     {
@@ -1094,7 +1119,7 @@ static int tiles_of(int kind, const dims_t &m, int level, int rows, int &tx)
     case K_GAUSS: w = m.cw; h = m.ch; th = BY * rows; break;
     case K_DEVELOP: w = m.W; h = m.H; tw = dev_tile<0>::W; th = dev_tile<0>::H; break;
     case K_DEVELOP_XT: w = m.W; h = m.H; tw = dev_tile<1>::W; th = dev_tile<1>::H; break;
-    case K_PYR1: w = m.lw[1]; h = m.lh[1]; break;
+    case K_PYR1: w = m.lw[1]; h = m.lh[1]; tw = P1_W; th = BY * P1_R; break;
     case K_REDUCE: case K_REDUCE_SPLIT: w = m.lw[level]; h = m.lh[level]; tw = 4 * BX; break;
     case K_TAIL: tx = 1; return 1;
     case K_ASM_SMALL: w = m.lw[level]; h = m.lh[level]; break;
@@ -1148,7 +1173,7 @@ static void build_launches(vkdt_batch_t *b)
   add(K_GAUSS, 0, 0);
   add(K_DEVELOP, 0, 0);
   add(K_DEVELOP_XT, 0, 0);
-  add(K_PYR1, 1, sizeof(__half) * (b->max_ng + 1) * P1_N);
+  add(K_PYR1, 1, 0);
   // a level's launch by the texels it has over all images
   auto texels = [&](int l) {
     size_t n = 0;

@@ -20,12 +20,13 @@ __global__ void __launch_bounds__(256) k_ll_curve(dimg in, dimg out, ll_args a, 
 {
   const int x0 = 4 * tid_x(), y = tid_y();
   if(x0 >= in.wd || y >= in.ht) return;
+  const ll_curve_k ck = ll_curve_load(a);
   if(!vec || x0 + 4 > in.wd)
   {
     for(int k = 0; k < 4 && x0 + k < in.wd; k++)
     {
       const float yl = ll_lum(ld_h4(in, x0 + k, y));
-      for(int i = 0; i < a.num_gamma; i++) st_h1(out, x0 + k, y, ll_curve(yl, a.gam[i], a), i);
+      for(int i = 0; i < a.num_gamma; i++) st_h1(out, x0 + k, y, ll_curve(yl, a.gam[i], ck), i);
       st_h1(out, x0 + k, y, yl, a.num_gamma);
     }
     return;
@@ -38,7 +39,7 @@ __global__ void __launch_bounds__(256) k_ll_curve(dimg in, dimg out, ll_args a, 
   for(int i = 0; i < a.num_gamma; i++)
   {
 #pragma unroll
-    for(int k = 0; k < 4; k++) w.e[k] = f2h(ll_curve(yl[k], a.gam[i], a));
+    for(int k = 0; k < 4; k++) w.e[k] = f2h(ll_curve(yl[k], a.gam[i], ck));
     *(uint2 *)(po + i * out.pstride) = w.u;
   }
 #pragma unroll
@@ -53,12 +54,13 @@ __global__ void __launch_bounds__(256) k_ll_curve8(dimg in, dimg out, ll_args a)
 {
   const int x0 = 8 * tid_x(), y = tid_y();
   if(x0 >= in.wd || y >= in.ht) return;
+  const ll_curve_k ck = ll_curve_load(a);
   if(x0 + 8 > in.wd)
   {
     for(int k = 0; k < 8 && x0 + k < in.wd; k++)
     {
       const float yl = ll_lum(ld_h4(in, x0 + k, y));
-      for(int i = 0; i < a.num_gamma; i++) st_h1(out, x0 + k, y, ll_curve(yl, a.gam[i], a), i);
+      for(int i = 0; i < a.num_gamma; i++) st_h1(out, x0 + k, y, ll_curve(yl, a.gam[i], ck), i);
       st_h1(out, x0 + k, y, yl, a.num_gamma);
     }
     return;
@@ -79,7 +81,7 @@ __global__ void __launch_bounds__(256) k_ll_curve8(dimg in, dimg out, ll_args a)
   for(int i = 0; i < a.num_gamma; i++)
   {
 #pragma unroll
-    for(int k = 0; k < 8; k++) w.e[k] = f2h(ll_curve(yl[k], a.gam[i], a));
+    for(int k = 0; k < 8; k++) w.e[k] = f2h(ll_curve(yl[k], a.gam[i], ck));
     *(uint4 *)(po + i * out.pstride) = w.u;
   }
 #pragma unroll

@@ -1139,12 +1139,20 @@ struct ll_args
 // fewer roundings (largest error against double over gammas and parameters
 // 2.3e-7, was 2.4e-7; kb_final of ten stills, 283 MP, 2996 -> 2492 us).  The value is a float before it is stored: fused with the
 // conversion the last product would round once in some kernels and twice in
-// others
-DEV float ll_curve(float x, float g, const ll_args &a)
+// others.  ll_curve_k: the parameters in registers -- from arguments held in
+// LDS or memory the selects would become selects of the address and a read a
+// curve (k_ll_curve8 at 24 MP 176 -> 147 us)
+struct ll_curve_k { float inv2s, sigma2, sh0, sh1, km0, km1, nc3, clarity; };
+DEV ll_curve_k ll_curve_load(const ll_args &a)
+{
+  return { f32_value(a.inv2s), f32_value(a.sigma2), f32_value(a.sh[0]), f32_value(a.sh[1]), f32_value(a.km[0]),
+           f32_value(a.km[1]), f32_value(a.nc3), f32_value(a.clarity) };
+}
+DEV float ll_curve(float x, float g, const ll_curve_k &a)
 {
   const float c = x - g, d = fabsf(c);
   const bool pos = c > 0.0f;
-  const float sh = pos ? a.sh[1] : a.sh[0], km = pos ? a.km[1] : a.km[0];
+  const float sh = pos ? a.sh1 : a.sh0, km = pos ? a.km1 : a.km0;
   const float t = clampf(d * a.inv2s, 0.0f, 1.0f);
   const float blend = t * __builtin_fmaf(t, km, a.sigma2), line = __builtin_fmaf(sh, d, -km);
   const float v = d > a.sigma2 ? line : blend;
