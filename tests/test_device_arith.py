@@ -52,6 +52,48 @@ def test_unorm16_corrected_product_equals_division(tmp_path):
     assert bare > 0
 
 
+RCP = r"""
+#include <math.h>
+#include <stdio.h>
+#include <stdint.h>
+#include <string.h>
+static float f(uint32_t u) { float v; memcpy(&v, &u, 4); return v; }
+int main(void)
+{
+  long div = 0, n = 0;
+  uint64_t s = 1;
+  for(uint32_t m = 0; m < 1u << 23; m++)
+  {
+    const float x = f(127u << 23 | m), want = 1.0f / x;
+    for(int k = 0; k < 8; k++, n++)
+    {
+      s = s * 6364136223846793005ull + 1442695040888963407ull;
+      const float a = f(127u << 23 | (uint32_t)(s >> 41)), q = a * want;
+      div += fmaf(fmaf(-x, q, a), want, q) != a / x;
+    }
+  }
+  printf("%ld %ld\n", div, n);
+  return 0;
+}
+"""
+
+
+def test_corrected_quotient_equals_division(tmp_path):
+    """common.h div_rn: with the correctly rounded reciprocal of the
+    denominator one residual step gives the correctly rounded quotient (random
+    numerators for every mantissa of the denominator)"""
+    c = tmp_path / "rcp.c"
+    c.write_text(RCP)
+    exe = tmp_path / "rcp"
+    try:
+        subprocess.run(["gcc", "-O2", "-mfma", "-ffp-contract=off", "-o", str(exe), str(c), "-lm"], check=True,
+                       capture_output=True)
+    except (OSError, subprocess.CalledProcessError) as e:
+        pytest.skip(f"no C compiler: {e}")
+    div, n = map(int, subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split())
+    assert div == 0 and n == 8 << 23
+
+
 # llap expand (ops.h ll_expand5): the reference's weighted 5x5 sum against
 # the kernels' form, bit for bit in binary32 on random f16-valued taps
 

@@ -986,7 +986,8 @@ struct vkdt_batch_t
 
 // the device tables at the end of the scratch: image records, job lists
 // (at most one job per image and launch) and the tile counters
-#define BT_MAX_LAUNCH (12 + 2 * BT_LEVELS + 2 * HL_LEVELS)
+// 8 wavelet and doub, 2 + 2 (HL_LEVELS - 1) hilite, 4 to pyr1, 2 (BT_LEVELS - 2) + 1 pyramid, 1 final
+#define BT_MAX_LAUNCH (16 + 2 * (HL_LEVELS - 1) + 2 * (BT_LEVELS - 2))
 static size_t table_bytes(int n)
 {
   return align256(sizeof(bt_img) * n) + align256(sizeof(bt_job) * (size_t)BT_MAX_LAUNCH * n)
