@@ -172,3 +172,32 @@ def test_llap_assemble_planes(hip, ng, step):
              node("assemble", asm(1), ["pyr0", "pyr0", "pyr1", "only"], W, H)]
     host = parity.run_gpu_graph(hip, bufs, nodes, raw)
     parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))
+
+
+@pytest.mark.parametrize("W,H", [(96 * 30, 24 * 18 + 6), (96 * 46 + 3, 24 * 46)])
+def test_xtrans_tiles_in_parts(hip, W, H):
+    """splat and fix above the tile counts at which a tile is cut into nine
+    parts, three and none (540 and 2162 tiles; the smaller extents of
+    test_xtrans_tiles have nine): the general path's values, which a graph cut
+    to a part of the image gives, away from the cut"""
+    import numpy as np
+    rng = np.random.default_rng(W)
+    mos = rng.uniform(0.05, 1, size=(H, W)).astype(np.float16)
+    p = gs.DevelopParams(kind="xtrans")
+    pc = gs.mixed_blob([("f", 1.0)] * 4 + [("i", p.filters)])
+    par = gs.mixed_blob([("i", 0), ("i", 0)])
+
+    def run(m):
+        h, w = m.shape
+        bufs = {"raw": (w, h, 1, gs.F16, 1), "cov": (w // 3, h // 3, 4, gs.F16, 1), "green": (w, h, 1, gs.F16, 1),
+                "out": (w, h, 4, gs.F16, 1)}
+        nodes = [dict(module="demosaic", kernel="gauss", pc=pc, params=par, conn=["raw", "raw", "cov"], wd=w // 3, ht=h // 3, dp=1, out=2),
+                 dict(module="demosaic", kernel="splat", pc=pc, params=par, conn=["raw", "cov", "green"], wd=w, ht=h, dp=1, out=2),
+                 dict(module="demosaic", kernel="fix", pc=pc, params=par, conn=["raw", "green", "cov", "out"], wd=w, ht=h, dp=1, out=3)]
+        return parity.run_gpu_graph(hip, bufs, nodes, np.ascontiguousarray(m))
+
+    host = run(mos)
+    for y0, x0 in ((0, 0), (6 * (H // 12), 6 * (W // 12)), (H - 132 - H % 6, W - 132 - W % 6)):
+        part = run(mos[y0:y0 + 132, x0:x0 + 132])
+        for k in ("green", "out"):
+            assert np.array_equal(host[k][y0 + 12:y0 + 120, x0 + 12:x0 + 120], part[k][12:120, 12:120]), (k, y0, x0)

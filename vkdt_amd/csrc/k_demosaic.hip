@@ -106,7 +106,10 @@ __global__ void __launch_bounds__(256) k_dm_fix(dimg in, dimg gr, dimg cv, dimg 
 
 // X-Trans by phase (dm_splat_xt, dm_fix_xt): a tile of 32x8 cells with its
 // halo staged in LDS, each wave two rows of cells, one phase of them at a
-// time; tiles whose taps leave the image take the general path per site
+// time; tiles whose taps leave the image take the general path per site.
+// gridDim.z parts share a tile's phases (or sites): a tile alone takes about
+// 40 us, which images of few tiles wait for instead of filling the chip (see
+// xt_parts)
 template<int U16>
 __global__ void __launch_bounds__(256) k_dm_splat_xt(dimg in, dimg ga, dimg out)
 {
@@ -123,19 +126,22 @@ __global__ void __launch_bounds__(256) k_dm_splat_xt(dimg in, dimg ga, dimg out)
     auto mos = [&](int px, int py) { return mt[(py - Y0 + 2) * mw + (px - X0 + 2)]; };
     const int sx = l % 32, sy = 2 * wv + l / 32;
 #pragma unroll 1
-    for(int ph = 0; ph < 9; ph++)
+    for(int ph = blockIdx.z; ph < 9; ph += gridDim.z)
       xt_phase(ph, [&](auto px, auto py) {
         constexpr int PX = decltype(px)::value, PY = decltype(py)::value;
-        o[(3 * sy + PY) * XT_TW + 3 * sx + PX] = f2h(dm_splat_xt<PX, PY>(mos, ga, X0 / 3 + sx, Y0 / 3 + sy));
+        const __half g = f2h(dm_splat_xt<PX, PY>(mos, ga, X0 / 3 + sx, Y0 / 3 + sy));
+        if(gridDim.z == 1) o[(3 * sy + PY) * XT_TW + 3 * sx + PX] = g;
+        else ((__half *)out.p)[(long)(Y0 + 3 * sy + PY) * out.pitch + X0 + 3 * sx + PX] = g;
       });
+    if(gridDim.z > 1) return;
     __syncthreads();
     tile_walk ws(tid, 256, XT_TW);
     for(int i = tid; i < XT_TW * XT_TH; i += 256, ws.next())
       ((__half *)out.p)[(long)(Y0 + ws.ty) * out.pitch + X0 + ws.tx] = o[i];
     return;
   }
-  tile_walk ws(tid, 256, XT_TW);
-  for(int i = tid; i < XT_TW * XT_TH; i += 256, ws.next())
+  tile_walk ws(tid + 256 * blockIdx.z, 256 * gridDim.z, XT_TW);
+  for(int i = tid + 256 * blockIdx.z; i < XT_TW * XT_TH; i += 256 * gridDim.z, ws.next())
   {
     const int x = X0 + ws.tx, y = Y0 + ws.ty;
     if(x < out.wd && y < out.ht) st_h1(out, x, y, dm_splat_px<1, U16>(in, ga, x, y));
@@ -164,15 +170,15 @@ __global__ void __launch_bounds__(256) k_dm_fix_xt(dimg in, dimg gr, dimg cv, di
     auto green = [&](int px, int py) { return gt[(py - Y0 + 2) * mw + (px - X0 + 2)]; };
     const int cx = X0 / 3 + l % 32, cy = Y0 / 3 + 2 * wv + l / 32;
 #pragma unroll 1
-    for(int ph = 0; ph < 9; ph++)
+    for(int ph = blockIdx.z; ph < 9; ph += gridDim.z)
       xt_phase(ph, [&](auto px, auto py) {
         constexpr int PX = decltype(px)::value, PY = decltype(py)::value;
         st_h4(out, 3 * cx + PX, 3 * cy + PY, dm_fix_xt<PX, PY>(mos, cv, cx, cy, green));
       });
     return;
   }
-  tile_walk ws(tid, 256, XT_TW);
-  for(int i = tid; i < XT_TW * XT_TH; i += 256, ws.next())
+  tile_walk ws(tid + 256 * blockIdx.z, 256 * gridDim.z, XT_TW);
+  for(int i = tid + 256 * blockIdx.z; i < XT_TW * XT_TH; i += 256 * gridDim.z, ws.next())
   {
     const int x = X0 + ws.tx, y = Y0 + ws.ty;
     if(x < out.wd && y < out.ht)
@@ -217,7 +223,16 @@ __global__ void __launch_bounds__(256) k_dm_halfsize(dimg in, dimg out)
 #define DM_PICK(kern, xt, u16) \
   ((xt) ? ((u16) ? kern<1, 1> : kern<1, 0>) : ((u16) ? kern<0, 1> : kern<0, 0>))
 
-static dim3 xt_grid(const node_call &c) { return dim3((c.wd + XT_TW - 1) / XT_TW, (c.ht + XT_TH - 1) / XT_TH, 1); }
+// the parts a tile is cut into: 9 below 512 tiles, 3 below 2048, so that there
+// are several work groups a CU where the tiles alone are not; more parts stage
+// the tile more often, which larger images pay for.  A node graph with hilite
+// off took 327 us at 780x520 and 457 us at 2100x1400 with whole tiles, 247 and
+// 418 us with parts
+static dim3 xt_grid(const node_call &c)
+{
+  const int tx = (c.wd + XT_TW - 1) / XT_TW, ty = (c.ht + XT_TH - 1) / XT_TH, n = tx * ty;
+  return dim3(tx, ty, n < 512 ? 9 : n < 2048 ? 3 : 1);
+}
 
 static int decode(dm_args &a, const node_call &c, const char *what)
 {
