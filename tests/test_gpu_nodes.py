@@ -21,6 +21,8 @@ pytestmark = pytest.mark.gpu
 CASES = [("bayer", 256, 192, 7, False, 0.5), ("xtrans", 258, 198, 11, False, 0.5),
          ("bayer", 256, 192, 17, True, 0.5), ("xtrans", 258, 198, 19, True, 0.5),
          ("bayer", 256, 192, 23, False, 0.0), ("xtrans", 258, 198, 29, False, 0.0)]
+# downcov of hashed inputs (test_downcov_rounding): extent, digest of the output
+DOWNCOV = [(67, 35, "1a9a005727e35180"), (258, 130, "c313927aa9e01344")]
 IDS = [c[0] + ("-hilite" if c[4] else "") + ("-noop" if c[5] <= 0 else "") for c in CASES]
 
 
@@ -139,6 +141,39 @@ def test_llap_curve(hip, par, W):
                   conn=["raw", "pyr0"], wd=W, ht=H, dp=1, out=1)]
     host = parity.run_gpu_graph(hip, bufs, nodes, raw)
     parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))
+
+
+def _hashed(n, seed):
+    """n values of 0..1 from an integer hash: the same wherever they are made"""
+    import numpy as np
+    u = np.arange(n, dtype=np.uint64) * np.uint64(2654435761) + np.uint64(seed) * np.uint64(40503)
+    u = ((u ^ (u >> np.uint64(15))) * np.uint64(2246822519)) & np.uint64(0xffffffff)
+    u = ((u ^ (u >> np.uint64(13))) * np.uint64(3266489917)) & np.uint64(0xffffffff)
+    return ((u ^ (u >> np.uint64(16))) & np.uint64(0xffff)).astype(np.float64) / 65535
+
+
+@pytest.mark.parametrize("W,H,digest", DOWNCOV, ids=[f"{w}x{h}" for w, h, _ in DOWNCOV])
+def test_downcov_rounding(hip, W, H, digest):
+    """denoise/downcov's bytes as recorded on a gfx950.  Its weighted sums
+    feed the wavelet's base level, and a binary16 step there can reach gauss's
+    choice between two nearly equal covariances, which changes a pixel visibly:
+    a rounding in another place is a change of the developed image"""
+    import hashlib
+    import numpy as np
+    v = _hashed(W * H * 3, 7).reshape(H, W, 3)
+    base = 0.02 + 0.5 * (((np.arange(W) // 5)[None, :] + (np.arange(H) // 3)[:, None]) % 4)   # edges of several heights
+    raw = np.ones((H, W, 4), np.float16)
+    raw[..., :3] = (base[:, :, None] * (0.9 + 0.2 * v)).astype(np.float16)
+    lv = [("f", 1.0)] * 4 + [("f", np.float32(512 / 65535.0))] * 4 + [("f", np.float32(16383 / 65535.0))] * 4 + [("i", 0)] * 4
+    par = gs.mixed_blob([("f", 0.6), ("f", 0.3), ("f", 0.7), ("f", 0.0)] + [("f", 1.0)] * 4 + [("i", 1)])
+    bufs = {"raw": (W, H, 4, gs.F16, 1), "s0": (W, H, 4, gs.F16, 1)}
+    nodes = [dict(module="denoise", kernel="downcov", pc=gs.mixed_blob(lv + [("f", 1e-4), ("f", 1e-6), ("i", 0), ("i", 2)]),
+                  params=par, conn=["raw", "s0"], wd=W, ht=H, dp=1, out=1)]
+    host = parity.run_gpu_graph(hip, bufs, nodes, raw)
+    parity.check_nodes(bufs, nodes, host, log=lambda s: print(s, flush=True))
+    got = hashlib.sha256(np.ascontiguousarray(host["s0"]).tobytes()).hexdigest()[:16]
+    print(f"[downcov] {W}x{H} {got}", flush=True)
+    assert got == digest
 
 
 @pytest.mark.parametrize("ng,step", [(2, 1), (10, 1), (10, 16), (32, 1)])

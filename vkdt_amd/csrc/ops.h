@@ -189,8 +189,12 @@ struct dn_cov_smem { float4 tile[DN_TN(R)]; float lum[DN_TN(R)], rlum[DN_TN(R)],
 DEV float add_times(float s, int k, float v) { return k == 0 ? s : __builtin_fmaf((float)k, v, s); }
 
 // Bound by instructions.  With the divisions in four instructions (rcp_rn,
-// div_rn) and these products left out or fused, and FMAs in the weighted sums:
-// downcov of ten stills (283 MP) 1888 -> 1609 us, at 24 MP 196 -> 167 us.
+// div_rn) and these products left out or fused: downcov of ten stills (283 MP)
+// 1888 -> 1653 us, at 24 MP 196 -> 172 us, the same values.  The weighted sums
+// and their exponents keep every rounding: with FMAs in them (1621 and 168 us)
+// the base level of the wavelet moves by a binary16 step here and there, and
+// where gauss's two covariances are nearly equal that flips its choice, a
+// visible change of the pixel.
 // The structure tensors of the 5x5 window at tile index c0 (offset (-2,-2)),
 // the choice between them and its eigen decomposition; mean_b is the
 // window's mean luminance.
@@ -271,10 +275,8 @@ DEV void dn_downcov_tile(const dimg &in, const dimg &out, const dimg &cov, const
     ev[0] = clampf(ev[0], 0.01f, 25.0f);
     ev[1] = clampf(ev[1], 0.01f, 25.0f);
     if(cov.p) st_h4(cov, x + a.crop[0], y + a.crop[1], make_float4(ev[0], ev[1], e0[0], e0[1]));
-    const float ri0 = -0.72134752f * frcp(ev[0]), ri1 = -0.72134752f * frcp(ev[1]);   // -log2(e) / 2
-    // the sums are continuous in their inputs (but for the hot pixel test,
-    // which they do not feed), so they use FMAs: fewer roundings.
-    // The anisotropic weight of offset o = (i-2, j-2) equals that of -o bit
+    const float ri0 = -0.5f * frcp(ev[0]), ri1 = -0.5f * frcp(ev[1]);
+    // the anisotropic weight of offset o = (i-2, j-2) equals that of -o bit
     // for bit (negating both offsets negates each rounded product and their
     // rounded sum exactly, and the sums are squared), so the exponentials
     // are taken for the half plane j > 2 or (j = 2, i >= 2) and mirrored
@@ -285,9 +287,9 @@ DEV void dn_downcov_tile(const dimg &in, const dimg &out, const dimg &cov, const
       for(int i = 0; i < 5; i++)
       {
         if(j == 2 && i < 2) continue;
-        const float x0 = __builtin_fmaf((float)(i - 2), e0[0], (float)(j - 2) * e0[1]);
-        const float x1 = __builtin_fmaf((float)(i - 2), e1[0], (float)(j - 2) * e1[1]);
-        const float w = fmaxf(1e-9f, fexp2(__builtin_fmaf(x1 * x1, ri1, x0 * x0 * ri0)));
+        const float x0 = (float)(i - 2) * e0[0] + (float)(j - 2) * e0[1];
+        const float x1 = (float)(i - 2) * e1[0] + (float)(j - 2) * e1[1];
+        const float w = fmaxf(1e-9f, fexp(x0 * x0 * ri0 + x1 * x1 * ri1));
         wgt[j][i] = w;
         wgt[4 - j][4 - i] = w;
       }
@@ -301,7 +303,7 @@ DEV void dn_downcov_tile(const dimg &in, const dimg &out, const dimg &cov, const
         const float4 v = s.tile[c0 + j * TW + i];
         if(v.x > hot) continue;   // hot pixel
         const float w = wgt[j][i];
-        r0 = __builtin_fmaf(w, v.x, r0); r1 = __builtin_fmaf(w, v.y, r1); r2 = __builtin_fmaf(w, v.z, r2);
+        r0 += w * v.x; r1 += w * v.y; r2 += w * v.z;
         wt += w;
       }
     const float d = frcp(fmaxf(wt, 1e-8f));
