@@ -152,6 +152,38 @@ def _hashed(n, seed):
     return ((u ^ (u >> np.uint64(16))) & np.uint64(0xffff)).astype(np.float64) / 65535
 
 
+@pytest.mark.parametrize("W", [67, 1030], ids=["scalar", "vector"])
+@pytest.mark.parametrize("par", [(0.12, 1.2, 0.8), (0.05, 1.6, 0.3), (0.25, -0.5, -0.5)])
+def test_llap_curve_rounding(hip, par, W):
+    """llap/curve without clarity uses no transcendental: it equals the
+    reference's formula (curve.comp:39-63) in float32, each operation rounded
+    once in the order written there, bit for bit"""
+    import numpy as np
+    f = np.float32
+    H, ng = 96, 10
+    lum = _hashed(W * H, 5).reshape(H, W) * 1.5 - 0.2
+    raw = np.repeat(lum[:, :, None], 4, axis=2).astype(np.float16)
+    bufs = {"raw": (W, H, 4, gs.F16, 1), "pyr0": (W, H, 1, gs.F16, ng + 1)}
+    nodes = [dict(module="llap", kernel="curve", pc=gs.mixed_blob([("i", ng)]), params=gs.f32blob(list(par) + [0.0]),
+                  conn=["raw", "pyr0"], wd=W, ht=H, dp=1, out=1)]
+    got = parity.run_gpu_graph(hip, bufs, nodes, raw)["pyr0"].reshape(ng + 1, H, W)
+    x, k = raw[..., 0].astype(f), [f(2.62700212e-01), f(6.77998072e-01), f(5.93017165e-02)]
+    x = (k[0] * x + k[1] * x) + k[2] * x                      # the luminance of a grey pixel
+    sigma, shadows, highlights = (f(v) for v in par)
+    for i in range(ng):
+        g = f(i) / f(ng - 1)
+        c = x - g
+        s = np.where(c > 0, sigma, -sigma)
+        sh = np.where(c > 0, shadows, highlights)
+        far = g + s + sh * (c - s)
+        t = np.clip(c * np.where(c > 0, f(1) / (f(2) * sigma), -(f(1) / (f(2) * sigma))), f(0), f(1))
+        near = g + s * f(2) * (f(1) - t) * t + t * t * (s + s * sh)
+        want = np.where(np.abs(c) > f(2) * sigma, far, near)
+        assert want.dtype == np.float32
+        nd = int(np.count_nonzero(want.astype(np.float16) != got[i]))
+        assert nd == 0, (i, nd)
+
+
 @pytest.mark.parametrize("W,H,digest", DOWNCOV, ids=[f"{w}x{h}" for w, h, _ in DOWNCOV])
 def test_downcov_rounding(hip, W, H, digest):
     """denoise/downcov's bytes as recorded on a gfx950.  Its weighted sums

@@ -1143,38 +1143,48 @@ struct ll_args
 {
   float sigma, clarity;
   float inv2s, sigma2;       // 1/(2 sigma), 2 sigma
-  float sh[2], km[2];        // highlights, shadows; sigma (sh - 1)
-  float nc3;                 // -3/(2 sigma^2) log2(e)
+  float sh[2], k[2];         // highlights, shadows; sigma + sigma sh
+  float c3;                  // 3/(2 sigma^2)
   int   num_gamma;
   int   first;
   float gam[LL_MAX_GAMMA];   // gamma_from_i(i) = i/(num_gamma-1), correctly rounded
 };
 
-// curve.comp:39-63, on d = |c| with the sign put back at the end: the linear
-// part is +-(sh d - km) from g, the blend t (2 sigma + t km), t = d / (2 sigma).
-// The eleven curves of a pixel are most of what the kernels that call it
-// issue: 17 instructions a curve against 30 as the reference writes it, with
-// fewer roundings (largest error against double over gammas and parameters
-// 2.3e-7, was 2.4e-7; kb_final of ten stills, 283 MP, 2996 -> 2492 us).  The value is a float before it is stored: fused with the
-// conversion the last product would round once in some kernels and twice in
-// others.  ll_curve_k: the parameters in registers -- from arguments held in
-// LDS or memory the selects would become selects of the address and a read a
-// curve (k_ll_curve8 at 24 MP 176 -> 147 us)
-struct ll_curve_k { float inv2s, sigma2, sh0, sh1, km0, km1, nc3, clarity; };
+// curve.comp:39-63 on d = |c|: the reference's two parts, the line beyond 2
+// sigma and the blend below it, change sign with c and no rounding does, so
+// each is formed once for d and joins g by an FMA with +-1 (exactly the sum):
+// the same values bit for bit in fewer instructions.  The eleven curves of a
+// pixel are most of what the kernels that call it issue; with ten stills
+// (283 MP) kb_final takes 1906 us (1843 with FMAs in other places, which
+// round differently).  The parts stay a branch: a wave's pixels mostly take
+// the same one, and with selects kb_pyr1 took 1992 us instead of 1688.
+// ll_curve_k: the parameters in registers -- from arguments held in LDS or
+// memory the selects would become selects of the address and a read a curve
+// (k_ll_curve8 at 24 MP 176 -> 147 us)
+struct ll_curve_k { float sigma, inv2s, sigma2, sh0, sh1, k0, k1, c3, clarity; };
 DEV ll_curve_k ll_curve_load(const ll_args &a)
 {
-  return { f32_value(a.inv2s), f32_value(a.sigma2), f32_value(a.sh[0]), f32_value(a.sh[1]), f32_value(a.km[0]),
-           f32_value(a.km[1]), f32_value(a.nc3), f32_value(a.clarity) };
+  return { f32_value(a.sigma), f32_value(a.inv2s), f32_value(a.sigma2), f32_value(a.sh[0]), f32_value(a.sh[1]),
+           f32_value(a.k[0]), f32_value(a.k[1]), f32_value(a.c3), f32_value(a.clarity) };
 }
 DEV float ll_curve(float x, float g, const ll_curve_k &a)
 {
   const float c = x - g, d = fabsf(c);
   const bool pos = c > 0.0f;
-  const float sh = pos ? a.sh1 : a.sh0, km = pos ? a.km1 : a.km0;
-  const float t = clampf(d * a.inv2s, 0.0f, 1.0f);
-  const float blend = t * __builtin_fmaf(t, km, a.sigma2), line = __builtin_fmaf(sh, d, -km);
-  const float v = d > a.sigma2 ? line : blend;
-  return f32_value(__builtin_fmaf(a.clarity * c, fexp2(c * c * a.nc3), g + (pos ? v : -v)));
+  const float sign = pos ? 1.0f : -1.0f;
+  float p, q;
+  if(d > a.sigma2)
+  {
+    p = a.sigma;
+    q = (pos ? a.sh1 : a.sh0) * (d - a.sigma);
+  }
+  else
+  {
+    const float t = clampf(d * a.inv2s, 0.0f, 1.0f);
+    p = a.sigma2 * (1.0f - t) * t;
+    q = t * t * (pos ? a.k1 : a.k0);
+  }
+  return __builtin_fmaf(sign, q, __builtin_fmaf(sign, p, g)) + a.clarity * c * fexp(-c * c * a.c3);
 }
 
 // llap.glsl:16-21: the first curve index above v (1..num_gamma-1), that
@@ -1506,8 +1516,8 @@ static inline void ll_args_init(ll_args &a, const float *p, int ng)
   a.clarity = p[3];
   a.inv2s = 1.0f / (2.0f * a.sigma);
   a.sigma2 = 2.0f * a.sigma;
-  for(int k = 0; k < 2; k++) a.km[k] = (float)((double)a.sigma * ((double)a.sh[k] - 1.0));
-  a.nc3 = (float)(-1.5 * 1.4426950408889634 / ((double)a.sigma * a.sigma));
+  for(int k = 0; k < 2; k++) a.k[k] = a.sigma + a.sigma * a.sh[k];
+  a.c3 = 1.0f / (2.0f * a.sigma * a.sigma / 3.0f);
   a.num_gamma = ng;
   a.first = 0;
   for(int i = 0; i < LL_MAX_GAMMA; i++) a.gam[i] = i < ng ? (float)i / ((float)ng - 1.0f) : 2.0f;
