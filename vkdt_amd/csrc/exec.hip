@@ -6,8 +6,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 #include <string.h>
-#include <mutex>
-#include <vector>
+#include <new>
 
 static thread_local char g_err[512] = "";
 
@@ -37,90 +36,27 @@ int launch_post(const char *what) { return hip_fail(hipGetLastError(), what); }
 // 3.8 -> 1.3 ms, lossless JPEG 24 MP 2.4 -> 1.64 ms, a 6 MP 14-bit unpack 680 ->
 // 355 us (its upload takes 340).
 
-struct scratch_pool
+namespace {
+struct hip_memory
 {
-  std::mutex mx;
-  std::vector<scratch_t> idle;   // oldest first
-  size_t kept = 0;
+  static int device(int *d) { return (int)hipGetDevice(d); }
+  static int dev_alloc(void **p, size_t n) { return (int)hipMalloc(p, n); }
+  static int pin_alloc(void **p, size_t n) { return (int)hipHostMalloc(p, n, hipHostMallocDefault); }
+  static void dev_free(void *p) { (void)hipFree(p); }
+  static void pin_free(void *p) { (void)hipHostFree(p); }
+  static bool oom(int e) { return e == (int)hipErrorOutOfMemory; }
 };
+}
 
-static scratch_pool &pool()
+static scratch_pool<hip_memory> &pool()
 { // never destroyed: the runtime may be gone when static objects are
-  static scratch_pool *p = new scratch_pool;
+  alignas(scratch_pool<hip_memory>) static unsigned char mem[sizeof(scratch_pool<hip_memory>)];
+  static scratch_pool<hip_memory> *p = new(mem) scratch_pool<hip_memory>;
   return *p;
 }
 
-static void scratch_free(const scratch_t &s)
-{
-  (void)hipFree(s.dev);
-  (void)hipHostFree(s.pin);
-}
-
-// gives the idle blocks back to the driver; false if there were none
-static bool scratch_trim()
-{
-  std::vector<scratch_t> out;
-  {
-    std::lock_guard<std::mutex> lk(pool().mx);
-    out.swap(pool().idle);
-    pool().kept = 0;
-  }
-  for(const scratch_t &s : out) scratch_free(s);
-  return !out.empty();
-}
-
-int scratch_get(scratch_t &s, size_t bytes, const char *what)
-{
-  s = scratch_t{};
-  if(int e = hip_fail(hipGetDevice(&s.device), what)) return e;
-  // whole megabytes, so that images of about one size share blocks
-  s.size = (bytes + ((size_t)1 << 20)) & ~(((size_t)1 << 20) - 1);
-  {
-    std::lock_guard<std::mutex> lk(pool().mx);
-    std::vector<scratch_t> &v = pool().idle;
-    int best = -1;
-    for(int k = 0; k < (int)v.size(); k++)
-      if(v[k].device == s.device && v[k].size >= s.size && v[k].size <= 2 * s.size && (best < 0 || v[k].size < v[best].size))
-        best = k;
-    if(best >= 0)
-    {
-      s = v[best];
-      v.erase(v.begin() + best);
-      pool().kept -= s.size;
-      return VKDT_HIP_OK;
-    }
-  }
-  hipError_t e = hipMalloc((void **)&s.dev, s.size);
-  if(e == hipErrorOutOfMemory && scratch_trim()) e = hipMalloc((void **)&s.dev, s.size);
-  if(e == hipSuccess)
-  {
-    e = hipHostMalloc((void **)&s.pin, SCRATCH_PINNED, hipHostMallocDefault);
-    if(e != hipSuccess) (void)hipFree(s.dev);
-  }
-  return hip_fail(e, what);
-}
-
-void scratch_put(scratch_t &s, bool ok)
-{
-  if(!s.dev) return;
-  std::vector<scratch_t> out;
-  if(!ok || s.size > SCRATCH_KEEP) out.push_back(s);
-  else
-  {
-    std::lock_guard<std::mutex> lk(pool().mx);
-    scratch_pool &p = pool();
-    p.idle.push_back(s);
-    p.kept += s.size;
-    while(p.kept > SCRATCH_KEEP)
-    {
-      p.kept -= p.idle.front().size;
-      out.push_back(p.idle.front());
-      p.idle.erase(p.idle.begin());
-    }
-  }
-  for(const scratch_t &o : out) scratch_free(o);
-  s = scratch_t{};
-}
+int scratch_get(scratch_t &s, size_t bytes, const char *what) { return hip_fail((hipError_t)pool().get(s, bytes), what); }
+void scratch_put(scratch_t &s, bool ok) { pool().put(s, ok); }
 
 int check_blob(const node_call &c, size_t pc_min, size_t params_min, const char *what)
 {
@@ -251,9 +187,7 @@ int vkdt_hip_node_launch(uint64_t module, uint64_t kernel, const void *pc, size_
 
 int vkdt_hip_alloc(void **ptr, size_t bytes)
 {
-  hipError_t e = hipMalloc(ptr, bytes ? bytes : 16);
-  if(e == hipErrorOutOfMemory && scratch_trim()) e = hipMalloc(ptr, bytes ? bytes : 16);
-  return hip_fail(e, "hipMalloc");
+  return hip_fail((hipError_t)pool().alloc(hip_memory::dev_alloc, ptr, bytes ? bytes : 16), "hipMalloc");
 }
 int vkdt_hip_free(void *ptr) { return hip_fail(hipFree(ptr), "hipFree"); }
 int vkdt_hip_host_alloc(void **ptr, size_t bytes) { return hip_fail(hipHostMalloc(ptr, bytes ? bytes : 16, hipHostMallocDefault), "hipHostMalloc"); }

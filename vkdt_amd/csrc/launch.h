@@ -7,6 +7,7 @@
 
 #include "../../include/vkdt_hip.h"
 #include "common.h"
+#include "scratch_pool.h"
 
 struct node_call
 {
@@ -70,18 +71,9 @@ int hip_fail(hipError_t e, const char *what);
 // Device scratch and pinned staging of one call of a codec entry point
 // (JPEG encode, lossless-JPEG decode, unpack).  Blocks return to a pool that
 // all threads and streams share: a call drains its stream before it puts its
-// block back, so the next user of any stream may take it at once.  The pool
-// keeps at most SCRATCH_KEEP bytes of idle device memory and gives all of it
-// back when an allocation of this library fails.
-#define SCRATCH_KEEP ((size_t)512 << 20)
-#define SCRATCH_PINNED ((size_t)64 << 10)
-struct scratch_t
-{
-  uint8_t *dev;      // device memory of at least the bytes asked for
-  uint8_t *pin;      // SCRATCH_PINNED bytes of pinned host memory
-  size_t   size;
-  int      device;
-};
+// block back, so the next user of any stream may take it at once.  The pool is
+// bounded and gives all its idle blocks back when an allocation of this
+// library fails (scratch_pool.h).
 int scratch_get(scratch_t &s, size_t bytes, const char *what);
 // ok: the stream has drained; else the block is freed (which waits for it)
 void scratch_put(scratch_t &s, bool ok);
