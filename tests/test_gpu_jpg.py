@@ -146,6 +146,24 @@ def test_threads_and_sizes_share_the_scratch(hip):
     assert not errs, errs
 
 
+def test_allocation_failure_is_reported_once(hip):
+    """an allocation that cannot be had (32 TB) is an error of that call alone,
+    also where idle scratch was given back and it was tried again: the launches
+    after it find no error of it"""
+    import ctypes as C
+    img = next(images())[1]
+    want = oracle_jpg(img, 95, 1, 1)
+    assert gpu_jpg(hip, img, 95, 1, 1) == want          # leaves idle scratch
+    p = C.c_void_p()
+    for _ in range(2):
+        assert H.lib().vkdt_hip_alloc(C.byref(p), 1 << 45) == H.OOM
+        assert gpu_jpg(hip, img, 95, 1, 1) == want
+    assert H.lib().vkdt_hip_alloc(C.byref(p), 1 << 45) == H.OOM
+    buf = hip.DeviceBuffer(16, 16, 1, H.FMT_F16)
+    buf.clear()
+    buf.free()
+
+
 def test_24mp_timing(hip):
     rng = np.random.default_rng(5)
     W, Hh = 6000, 4000

@@ -65,6 +65,31 @@ static int pinned_failure()
   return 0;
 }
 
+// an allocation that succeeds at the second try, without the idle blocks, and
+// one that fails altogether leave no error for a later check to find
+static int last_error_is_cleared()
+{
+  pool_t p;
+  scratch_t s;
+  limit = 10 * MB;
+  CHECK(p.get(s, 6 * MB) == 0);
+  p.put(s, true);
+  CHECK(p.get(s, 1 * MB) == 0);          // too small for the idle block
+  CHECK(last_error == 0);
+  p.put(s, true);
+  void *q = nullptr;
+  CHECK(p.alloc(mem::dev_alloc, &q, 8 * MB) == 0 && q && last_error == 0);
+  CHECK(dev_live.size() == 1);           // the idle blocks went
+  CHECK(p.get(s, 6 * MB) == OOM && !s.dev && last_error == 0);
+  mem::dev_free(q);
+  fail_dev = OTHER;                      // no lack of memory: nothing is given back for it
+  CHECK(p.get(s, 6 * MB) == OTHER && last_error == 0);
+  fail_dev = 0;
+  fail_pin = 1;
+  CHECK(p.get(s, 6 * MB) == OOM && last_error == 0 && dev_live.empty() && bad_frees == 0);
+  return 0;
+}
+
 // a block that failed comes back to the driver, a good one to the next caller
 static int reuse()
 {
@@ -130,7 +155,7 @@ int main(int, char **v)
   return 2;
 }
 """
-NAMES = ["pinned_failure", "reuse", "devices", "bounded"]
+NAMES = ["pinned_failure", "last_error_is_cleared", "reuse", "devices", "bounded"]
 
 
 @pytest.fixture(scope="module")

@@ -22,6 +22,7 @@ int vkdt_set_error(int code, const char *fmt, ...)
 int hip_fail(hipError_t e, const char *what)
 {
   if(e == hipSuccess) return VKDT_HIP_OK;
+  (void)hipGetLastError();   // told here, not once more by the check of the next launch
   return vkdt_set_error(e == hipErrorOutOfMemory ? VKDT_HIP_OOM : VKDT_HIP_DEVICE,
                         "%s: %s", what, hipGetErrorString(e));
 }
@@ -45,6 +46,7 @@ struct hip_memory
   static void dev_free(void *p) { (void)hipFree(p); }
   static void pin_free(void *p) { (void)hipHostFree(p); }
   static bool oom(int e) { return e == (int)hipErrorOutOfMemory; }
+  static void forget() { (void)hipGetLastError(); }
 };
 }
 

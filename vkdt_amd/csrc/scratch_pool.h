@@ -5,6 +5,7 @@
 //   int dev_alloc(void **, size_t), void dev_free(void *)
 //   int pin_alloc(void **, size_t), void pin_free(void *)
 //   bool oom(int)                whether that error is a lack of memory
+//   void forget()                clears the error that the thread last had
 // Errors are M's, 0 is success.  Nothing here throws: the callers are C entry
 // points, and the idle blocks lie in arrays of fixed size.
 #pragma once
@@ -52,6 +53,7 @@ public:
     if(!b.pin)
       if(int e = M::pin_alloc((void **)&b.pin, SCRATCH_PINNED))
       {
+        M::forget();
         M::dev_free(b.dev);
         return e;
       }
@@ -91,12 +93,20 @@ public:
     return no > 0;
   }
 
-  // an allocation, tried again without the idle blocks where memory lacks
+  // an allocation, tried again without the idle blocks where memory lacks.  Its
+  // error is forgotten, whether the second try succeeds or the caller is told:
+  // the runtime keeps it through later successful calls, and the check of the
+  // next launch would read it
   template<typename F>
   int alloc(F f, void **p, size_t bytes)
   {
     int e = f(p, bytes);
-    if(e && M::oom(e) && trim()) e = f(p, bytes);
+    if(e) M::forget();
+    if(e && M::oom(e) && trim())
+    {
+      e = f(p, bytes);
+      if(e) M::forget();
+    }
     return e;
   }
 
