@@ -90,6 +90,21 @@ static int last_error_is_cleared()
   return 0;
 }
 
+// pinned memory that is short comes from the idle blocks too
+static int pinned_from_idle()
+{
+  pool_t p;
+  scratch_t a, b;
+  CHECK(p.get(a, 2 * MB) == 0);
+  p.put(a, true);
+  fail_pin = 2;                          // one pinned buffer at a time
+  CHECK(p.get(b, 20 * MB) == 0 && b.pin && dev_live.size() == 1 && pin_live.size() == 1 && last_error == 0);
+  p.put(b, true);
+  void *q = nullptr;
+  CHECK(p.alloc(mem::pin_alloc, &q, MB) == 0 && q && dev_live.empty() && bad_frees == 0);
+  return 0;
+}
+
 // a block that failed comes back to the driver, a good one to the next caller
 static int reuse()
 {
@@ -155,7 +170,7 @@ int main(int, char **v)
   return 2;
 }
 """
-NAMES = ["pinned_failure", "last_error_is_cleared", "reuse", "devices", "bounded"]
+NAMES = ["pinned_failure", "last_error_is_cleared", "pinned_from_idle", "reuse", "devices", "bounded"]
 
 
 @pytest.fixture(scope="module")

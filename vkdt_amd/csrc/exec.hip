@@ -192,7 +192,10 @@ int vkdt_hip_alloc(void **ptr, size_t bytes)
   return hip_fail((hipError_t)pool().alloc(hip_memory::dev_alloc, ptr, bytes ? bytes : 16), "hipMalloc");
 }
 int vkdt_hip_free(void *ptr) { return hip_fail(hipFree(ptr), "hipFree"); }
-int vkdt_hip_host_alloc(void **ptr, size_t bytes) { return hip_fail(hipHostMalloc(ptr, bytes ? bytes : 16, hipHostMallocDefault), "hipHostMalloc"); }
+int vkdt_hip_host_alloc(void **ptr, size_t bytes)
+{
+  return hip_fail((hipError_t)pool().alloc(hip_memory::pin_alloc, ptr, bytes ? bytes : 16), "hipHostMalloc");
+}
 int vkdt_hip_host_free(void *ptr) { return hip_fail(hipHostFree(ptr), "hipHostFree"); }
 
 int vkdt_hip_upload(void *dst_dev, const void *src_host, size_t bytes, void *stream)

@@ -51,9 +51,8 @@ public:
     if(!b.dev)
       if(int e = alloc(M::dev_alloc, (void **)&b.dev, b.size)) return e;
     if(!b.pin)
-      if(int e = M::pin_alloc((void **)&b.pin, SCRATCH_PINNED))
+      if(int e = alloc(M::pin_alloc, (void **)&b.pin, SCRATCH_PINNED))
       {
-        M::forget();
         M::dev_free(b.dev);
         return e;
       }
