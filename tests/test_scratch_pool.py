@@ -57,7 +57,7 @@ static int pinned_failure()
   pool_t p;
   scratch_t s;
   fail_pin = 1;
-  CHECK(p.get(s, 3 * MB) == OOM);
+  CHECK(p.get(s, 3 * MB, true) == OOM);
   CHECK(!s.dev && !s.pin && dev_live.empty());
   p.put(s, false);
   p.put(s, true);
@@ -72,21 +72,21 @@ static int last_error_is_cleared()
   pool_t p;
   scratch_t s;
   limit = 10 * MB;
-  CHECK(p.get(s, 6 * MB) == 0);
+  CHECK(p.get(s, 6 * MB, false) == 0);
   p.put(s, true);
-  CHECK(p.get(s, 1 * MB) == 0);          // too small for the idle block
+  CHECK(p.get(s, 1 * MB, false) == 0);          // too small for the idle block
   CHECK(last_error == 0);
   p.put(s, true);
   void *q = nullptr;
   CHECK(p.alloc(mem::dev_alloc, &q, 8 * MB) == 0 && q && last_error == 0);
   CHECK(dev_live.size() == 1);           // the idle blocks went
-  CHECK(p.get(s, 6 * MB) == OOM && !s.dev && last_error == 0);
+  CHECK(p.get(s, 6 * MB, false) == OOM && !s.dev && last_error == 0);
   mem::dev_free(q);
   fail_dev = OTHER;                      // no lack of memory: nothing is given back for it
-  CHECK(p.get(s, 6 * MB) == OTHER && last_error == 0);
+  CHECK(p.get(s, 6 * MB, false) == OTHER && last_error == 0);
   fail_dev = 0;
   fail_pin = 1;
-  CHECK(p.get(s, 6 * MB) == OOM && last_error == 0 && dev_live.empty() && bad_frees == 0);
+  CHECK(p.get(s, 6 * MB, true) == OOM && last_error == 0 && dev_live.empty() && bad_frees == 0);
   return 0;
 }
 
@@ -95,13 +95,29 @@ static int pinned_from_idle()
 {
   pool_t p;
   scratch_t a, b;
-  CHECK(p.get(a, 2 * MB) == 0);
+  CHECK(p.get(a, 2 * MB, true) == 0);
   p.put(a, true);
   fail_pin = 2;                          // one pinned buffer at a time
-  CHECK(p.get(b, 20 * MB) == 0 && b.pin && dev_live.size() == 1 && pin_live.size() == 1 && last_error == 0);
+  CHECK(p.get(b, 20 * MB, true) == 0 && b.pin && dev_live.size() == 1 && pin_live.size() == 1 && last_error == 0);
   p.put(b, true);
   void *q = nullptr;
   CHECK(p.alloc(mem::pin_alloc, &q, MB) == 0 && q && dev_live.empty() && bad_frees == 0);
+  return 0;
+}
+
+// a pinned buffer is made where one is asked for, and stays with its block
+static int pinned_where_used()
+{
+  pool_t p;
+  scratch_t s;
+  CHECK(p.get(s, 5 * MB, false) == 0 && !s.pin && pin_allocs == 0);
+  uint8_t *first = s.dev;
+  p.put(s, true);
+  CHECK(p.get(s, 5 * MB, true) == 0 && s.dev == first && s.pin && pin_allocs == 1);
+  p.put(s, true);
+  CHECK(p.get(s, 5 * MB, true) == 0 && pin_allocs == 1);
+  p.put(s, false);
+  CHECK(dev_live.empty() && pin_live.empty() && bad_frees == 0);
   return 0;
 }
 
@@ -110,19 +126,19 @@ static int reuse()
 {
   pool_t p;
   scratch_t a, b;
-  CHECK(p.get(a, 5 * MB) == 0 && a.size >= 5 * MB);
+  CHECK(p.get(a, 5 * MB, false) == 0 && a.size >= 5 * MB);
   uint8_t *first = a.dev;
   p.put(a, true);
   CHECK(!a.dev && dev_live.size() == 1);
-  CHECK(p.get(b, 4 * MB) == 0 && b.dev == first && dev_allocs == 1);
+  CHECK(p.get(b, 4 * MB, false) == 0 && b.dev == first && dev_allocs == 1);
   p.put(b, false);
   CHECK(dev_live.empty() && bad_frees == 0);
   // not a block of more than twice the size, nor a smaller one
-  CHECK(p.get(a, 20 * MB) == 0);
+  CHECK(p.get(a, 20 * MB, false) == 0);
   p.put(a, true);
-  CHECK(p.get(b, 4 * MB) == 0 && b.size < 10 * MB);
+  CHECK(p.get(b, 4 * MB, false) == 0 && b.size < 10 * MB);
   p.put(b, true);
-  CHECK(p.get(b, 8 * MB) == 0 && dev_allocs == 4);
+  CHECK(p.get(b, 8 * MB, false) == 0 && dev_allocs == 4);
   p.put(b, true);
   CHECK(p.trim() && dev_live.empty() && pin_live.empty() && !p.trim() && bad_frees == 0);
   return 0;
@@ -132,14 +148,14 @@ static int devices()
 {
   pool_t p;
   scratch_t a, b;
-  CHECK(p.get(a, 5 * MB) == 0);
+  CHECK(p.get(a, 5 * MB, false) == 0);
   uint8_t *first = a.dev;
   p.put(a, true);
   cur_device = 1;
-  CHECK(p.get(b, 5 * MB) == 0 && b.dev != first && b.device == 1);
+  CHECK(p.get(b, 5 * MB, false) == 0 && b.dev != first && b.device == 1);
   p.put(b, true);
   cur_device = 0;
-  CHECK(p.get(a, 5 * MB) == 0 && a.dev == first);
+  CHECK(p.get(a, 5 * MB, false) == 0 && a.dev == first);
   p.put(a, true);
   return 0;
 }
@@ -149,15 +165,15 @@ static int bounded()
 {
   pool_t p;
   scratch_t s[4], t[SCRATCH_SLOTS + 3];
-  for(int k = 0; k < 4; k++) CHECK(p.get(s[k], SCRATCH_KEEP / 3 - 2 * MB) == 0);
+  for(int k = 0; k < 4; k++) CHECK(p.get(s[k], SCRATCH_KEEP / 3 - 2 * MB, false) == 0);
   uint8_t *first = s[0].dev, *second = s[1].dev;
   for(int k = 0; k < 4; k++) p.put(s[k], true);
   CHECK(mem::used() <= SCRATCH_KEEP && dev_live.size() == 3 && !dev_live.count(first) && dev_live.count(second));
-  CHECK(p.get(s[0], SCRATCH_KEEP + MB) == 0);
+  CHECK(p.get(s[0], SCRATCH_KEEP + MB, false) == 0);
   p.put(s[0], true);
   CHECK(mem::used() <= SCRATCH_KEEP && dev_live.size() == 3);
   p.trim();
-  for(auto &b : t) CHECK(p.get(b, 1) == 0);
+  for(auto &b : t) CHECK(p.get(b, 1, false) == 0);
   for(auto &b : t) p.put(b, true);
   CHECK(dev_live.size() == SCRATCH_SLOTS && bad_frees == 0);
   return 0;
@@ -170,7 +186,7 @@ int main(int, char **v)
   return 2;
 }
 """
-NAMES = ["pinned_failure", "last_error_is_cleared", "pinned_from_idle", "reuse", "devices", "bounded"]
+NAMES = ["pinned_failure", "last_error_is_cleared", "pinned_from_idle", "pinned_where_used", "reuse", "devices", "bounded"]
 
 
 @pytest.fixture(scope="module")

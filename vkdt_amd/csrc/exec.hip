@@ -57,7 +57,10 @@ static scratch_pool<hip_memory> &pool()
   return *p;
 }
 
-int scratch_get(scratch_t &s, size_t bytes, const char *what) { return hip_fail((hipError_t)pool().get(s, bytes), what); }
+int scratch_get(scratch_t &s, size_t bytes, const char *what, bool pinned)
+{
+  return hip_fail((hipError_t)pool().get(s, bytes, pinned), what);
+}
 void scratch_put(scratch_t &s, bool ok) { pool().put(s, ok); }
 
 int check_blob(const node_call &c, size_t pc_min, size_t params_min, const char *what)

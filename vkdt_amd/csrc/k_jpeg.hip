@@ -1035,7 +1035,7 @@ extern "C" int vkdt_hip_jpg_encode_ex(const void *rgba, uint32_t wd, uint32_t ht
   const size_t o_blen = o_bits + (size_t)(ngroups + 1) * 8;
   const size_t total = o_blen + (size_t)nbl * 2;
   scratch_t sc, st = {};
-  if(int e = scratch_get(sc, total, "jpg scratch")) return e;
+  if(int e = scratch_get(sc, total, "jpg scratch", true)) return e;
   uint8_t *dev = sc.dev;
   hipStream_t s = (hipStream_t)stream;
   int16_t *coef = (int16_t *)(dev + o_coef);

@@ -74,7 +74,8 @@ int hip_fail(hipError_t e, const char *what);
 // block back, so the next user of any stream may take it at once.  The pool is
 // bounded and gives all its idle blocks back when an allocation of this
 // library fails (scratch_pool.h).
-int scratch_get(scratch_t &s, size_t bytes, const char *what);
+// pinned: with SCRATCH_PINNED bytes of pinned staging
+int scratch_get(scratch_t &s, size_t bytes, const char *what, bool pinned = false);
 // ok: the stream has drained; else the block is freed (which waits for it)
 void scratch_put(scratch_t &s, bool ok);
 

@@ -30,9 +30,9 @@ template<typename M>
 class scratch_pool
 {
 public:
-  // a block of at least `bytes`.  A failure leaves s empty: putting it back is
-  // no harm
-  int get(scratch_t &s, size_t bytes)
+  // a block of at least `bytes`, with a pinned buffer where asked for.  A
+  // failure leaves s empty: putting it back is no harm
+  int get(scratch_t &s, size_t bytes, bool pinned)
   {
     s = scratch_t{};
     scratch_t b = {};
@@ -50,7 +50,7 @@ public:
     }
     if(!b.dev)
       if(int e = alloc(M::dev_alloc, (void **)&b.dev, b.size)) return e;
-    if(!b.pin)
+    if(pinned && !b.pin)
       if(int e = alloc(M::pin_alloc, (void **)&b.pin, SCRATCH_PINNED))
       {
         M::dev_free(b.dev);
