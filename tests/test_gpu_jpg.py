@@ -164,6 +164,30 @@ def test_allocation_failure_is_reported_once(hip):
     buf.free()
 
 
+def test_large_export_takes_memory_for_its_stream(hip):
+    """36 MP 4:4:4, above the extent whose stream is given room unseen: the
+    blocks' scratch (130 bytes each) and the stream's own length are taken, not
+    another 96 bytes a block; the file is the oracle's"""
+    import ctypes as C
+    import torch
+    W = Hh = 6016
+    blocks = 3 * (W // 8) * (Hh // 8)
+    img = np.zeros((Hh, W, 3), np.uint8)
+    img[1000:1016, :, 1] = (np.arange(W) // 3) % 256
+    rgba = np.dstack([img, np.full((Hh, W), 255, np.uint8)])
+    buf = hip.DeviceBuffer(W, Hh, 4, H.FMT_UI8)
+    buf.upload(rgba)
+    p = C.c_void_p()
+    assert H.lib().vkdt_hip_alloc(C.byref(p), 1 << 45) == H.OOM      # gives the idle scratch back
+    free = torch.cuda.mem_get_info()[0]
+    out = H.jpg_encode(buf.ptr, W, Hh, W, 90, 1, 1)
+    held = free - torch.cuda.mem_get_info()[0]
+    buf.free()
+    print(f"[gpu_jpg] 36 MP: {len(out)} bytes, {held / blocks:.0f} bytes of scratch a block", flush=True)
+    assert held < 150 * blocks
+    assert out == oracle_jpg(img, 90, 1, 1)
+
+
 def test_24mp_timing(hip):
     rng = np.random.default_rng(5)
     W, Hh = 6000, 4000

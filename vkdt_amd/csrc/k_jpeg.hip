@@ -881,6 +881,9 @@ __global__ void __launch_bounds__(256) k_jpg_zero_words(uint4 *w, const uint64_t
 
 // ---- host ------------------------------------------------------------------
 
+// the stream's room that is taken without knowing its length: 30 MP in 4:4:4
+#define JPG_ROOM ((size_t)128 << 20)
+
 // optimal code lengths (T.81 K.2: the two smallest frequencies merged, ties to
 // the larger symbol, a reserved symbol 256; K.3: lengths limited to 16)
 void jpg_huff(const uint32_t *freq_in, uint8_t bits[17], uint8_t val[256], int *nval)
@@ -1108,16 +1111,33 @@ extern "C" int vkdt_hip_jpg_encode_ex(const void *rgba, uint32_t wd, uint32_t ht
   }
   // The stream is written into room for 4 bits a coefficient, so that its
   // length need not come back first; the kernels leave a longer one alone, and
-  // it is written again into room for its length
+  // it is written again into room for its length.  Above JPG_ROOM bytes, where
+  // the round trip (20 us) is little against the kernels, and where there is no
+  // memory for that room, the length is asked for first
   const uint64_t *tot = bits + ngroups;
   uint64_t nbits = 0, nff = 0;
   uint8_t *stuffed = nullptr;
   size_t cap = (size_t)nbl * 32;
-  for(int pass = 0; pass < 2 && !err; pass++)
+  bool known = false;   // cap is the length
+  const auto length = [&]() {
+    int e = hip_fail(hipMemcpyAsync(sizes, tot, 8, hipMemcpyDeviceToHost, s), "jpg total");
+    if(!e) e = hip_fail(hipStreamSynchronize(s), "jpg sync");
+    if(e) return e;
+    cap = (size_t)((sizes[0] + 7) / 8);
+    known = true;
+    return e;
+  };
+  if(!err && 3 * cap > JPG_ROOM) err = length();
+  while(!err)
   { // words | 0xFF bytes before each chunk, their total | stuffed bytes (at most twice)
     const long nwords = (long)((cap + 15) / 16 * 4), nchunks = (long)((cap + JS_BYTES - 1) / JS_BYTES);
     const size_t wbytes = ((size_t)nwords * 4 + 255) & ~(size_t)255, cbytes = ((size_t)(nchunks + 1) * 8 + 255) & ~(size_t)255;
     err = scratch_get(st, wbytes + cbytes + 2 * cap + 16, "jpg stream");
+    if(err == VKDT_HIP_OOM && !known)
+    {
+      err = length();
+      continue;
+    }
     if(err) break;
     uint32_t *words = (uint32_t *)st.dev;
     uint64_t *cnt = (uint64_t *)(st.dev + wbytes);
@@ -1137,9 +1157,10 @@ extern "C" int vkdt_hip_jpg_encode_ex(const void *rgba, uint32_t wd, uint32_t ht
     if(err) break;
     nbits = sizes[0];
     nff = sizes[1];
-    if(nbits <= (uint64_t)cap * 8) break;
+    if(known || nbits <= (uint64_t)cap * 8) break;
     scratch_put(st, true);
     cap = (size_t)((nbits + 7) / 8);
+    known = true;
   }
   const size_t nbytes = (size_t)((nbits + 7) / 8);
   out_t o;
