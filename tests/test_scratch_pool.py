@@ -144,6 +144,23 @@ static int reuse()
   return 0;
 }
 
+// the blocks of a 9504x6336 export in 4:4:4 (130 bytes a block of coefficients,
+// three times a stream of 4 bits a coefficient) serve the next one
+static int large_export()
+{
+  const size_t blocks = (size_t)3 * (9504 / 8) * (6336 / 8);
+  pool_t p;
+  for(int k = 0; k < 3; k++)
+  {
+    scratch_t a, b;
+    CHECK(p.get(a, 130 * blocks, true) == 0 && p.get(b, 96 * blocks, false) == 0);
+    p.put(a, true);
+    p.put(b, true);
+  }
+  CHECK(dev_allocs == 2 && pin_allocs == 1);
+  return 0;
+}
+
 static int devices()
 {
   pool_t p;
@@ -186,7 +203,7 @@ int main(int, char **v)
   return 2;
 }
 """
-NAMES = ["pinned_failure", "last_error_is_cleared", "pinned_from_idle", "pinned_where_used", "reuse", "devices", "bounded"]
+NAMES = ["pinned_failure", "last_error_is_cleared", "pinned_from_idle", "pinned_where_used", "reuse", "large_export", "devices", "bounded"]
 
 
 @pytest.fixture(scope="module")
