@@ -428,15 +428,20 @@ __global__ void __launch_bounds__(256) kb_gauss(bt_launch L)
 // mosaic through the bounds-checked global path.  Both see the same values.
 #define DEV_M 5   // r + rs <= 3 + 2
 
-// tile of the develop stage: 64x16 texels, X-Trans 96x24 (whole 3x3 cells and
-// whole waves of each phase)
-template<int XT> struct dev_tile { static constexpr int W = XT ? XT_TW : BX, H = XT ? XT_TH : BY * DEV_R; };
+// tile of the develop stage: 64x16 texels, X-Trans by phase 96x24 (whole 3x3
+// cells and whole waves of each phase).  F: DEV_BAYER, DEV_XT by phase, or
+// DEV_XT_SITE, X-Trans a site a thread with taps of any colour, for launches
+// of few tiles: a phase tile has nine phases of splat and of fix one after
+// the other for more than twice the texels, which a launch that does not fill
+// the chip waits for (see dev_xt_sites)
+enum { DEV_BAYER, DEV_XT, DEV_XT_SITE };
+template<int F> struct dev_tile { static constexpr int W = F == DEV_XT ? XT_TW : BX, H = F == DEV_XT ? XT_TH : BY * DEV_R; };
 
-template<int XT>
+template<int F>
 DEV void develop_tile(const dimg &mos, const dimg &cov, const dimg &film, const co_args &co, const fc_args &fc,
                       int r, int X0, int Y0, float *gt, float *mt)
 {
-  constexpr int rs = XT ? 2 : 1, DW = dev_tile<XT>::W, DH = dev_tile<XT>::H;
+  constexpr int XT = F != DEV_BAYER, rs = XT ? 2 : 1, DW = dev_tile<F>::W, DH = dev_tile<F>::H;
   const int gw = DW + 2 * r, gh = DH + 2 * r;
   const int W = film.wd, H = film.ht;
   const int m = r + rs, mw = DW + 2 * m, mh = DH + 2 * m;
@@ -450,7 +455,7 @@ DEV void develop_tile(const dimg &mos, const dimg &cov, const dimg &film, const 
       mt[i] = ld_h1(mos, X0 - m + wm.tx, Y0 - m + wm.ty);
     __syncthreads();
     auto mosl = [&](int px, int py) { return mt[(py - Y0 + m) * mw + (px - X0 + m)]; };
-    if(XT && r == 2)
+    if(F == DEV_XT && r == 2)
     { // each wave one phase of the CFA cells at a time (dm_splat_xt): the tile
       // starts on a cell, and its halo of 2 holds 33 or 34 by 9 or 10 sites of a
       // phase, dealt to the waves 64 at a time
@@ -513,7 +518,8 @@ DEV void develop_tile(const dimg &mos, const dimg &cov, const dimg &film, const 
       tile_walk wt(tid, BX * BY, DW);
 #pragma unroll 1
       for(int i = tid; i < DW * DH; i += BX * BY, wt.next())
-        finish(dm_fix_loop<1>(mosl, cov, r, X0 + wt.tx, Y0 + wt.ty, green), X0 + wt.tx, Y0 + wt.ty);
+        finish(F == DEV_XT_SITE ? dm_fix_r<1>(mosl, cov, r, X0 + wt.tx, Y0 + wt.ty, green)
+                                : dm_fix_loop<1>(mosl, cov, r, X0 + wt.tx, Y0 + wt.ty, green), X0 + wt.tx, Y0 + wt.ty);
       return;
     }
 #pragma unroll 1
@@ -538,12 +544,13 @@ DEV void develop_tile(const dimg &mos, const dimg &cov, const dimg &film, const 
   }
 }
 
-// Bayer: at most 80 VGPRs, 6 waves per SIMD: the staging and splat phases'
-// memory latency is hidden by the extra waves.  X-Trans: 5, what its LDS holds
-template<int XT, int P>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(XT ? 5 : 6))) kb_develop(bt_launch L)
+// Bayer and X-Trans by site: at most 80 VGPRs, 6 waves per SIMD: the staging
+// and splat phases' memory latency is hidden by the extra waves.  X-Trans by
+// phase: 5, what its LDS holds
+template<int F, int P>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(F == DEV_XT ? 5 : 6))) kb_develop(bt_launch L)
 {
-  constexpr int DW = dev_tile<XT>::W, DH = dev_tile<XT>::H;
+  constexpr int DW = dev_tile<F>::W, DH = dev_tile<F>::H;
   __shared__ float gt[(DW + 6) * (DH + 6)];                       // green, halo r <= 3
   __shared__ float mt[(DW + 2 * DEV_M) * (DH + 2 * DEV_M)];       // mosaic, halo r + rs
   __shared__ co_args co;
@@ -557,7 +564,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(XT ? 5
     mos = rfl(im.mos); cov = rfl(im.cov); film = rfl(im.film); r = rfl(im.dm_r);
   }, [&](const bt_job &jb, int lt) {
     const int X0 = (lt % jb.tiles_x) * DW, Y0 = (lt / jb.tiles_x) * DH;
-    develop_tile<XT>(mos, cov, film, co, fc, r, X0, Y0, gt, mt);
+    develop_tile<F>(mos, cov, film, co, fc, r, X0, Y0, gt, mt);
   });
 }
 
@@ -850,8 +857,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 namespace {
 
 enum kind_t { K_HALF, K_DOWNCOV, K_DOWN, K_DNASM, K_DOUB, K_DOUB_XT, K_HL_HALF, K_HL_REDUCE, K_HL_ASM, K_HL_DOUB, K_GAUSS,
-              K_DEVELOP, K_DEVELOP_XT, K_PYR1, K_REDUCE, K_REDUCE_SPLIT, K_TAIL, K_ASM_SMALL, K_ASM, K_FINAL };
-const int kind_group[] = { 0, 1, 1, 2, 3, 3, 4, 4, 4, 4, 5, 6, 6, 7, 8, 8, 8, 8, 8, 9 };
+              K_DEVELOP, K_DEVELOP_XT, K_DEVELOP_XS, K_PYR1, K_REDUCE, K_REDUCE_SPLIT, K_TAIL, K_ASM_SMALL, K_ASM, K_FINAL };
+const int kind_group[] = { 0, 1, 1, 2, 3, 3, 4, 4, 4, 4, 5, 6, 6, 6, 7, 8, 8, 8, 8, 8, 9 };
 const char *group_name[VKDT_BATCH_STAGES] = { "half", "wavelet", "dnasm", "doub", "hilite", "gauss", "develop",
                                               "pyr1", "pyramid", "final" };
 
@@ -1118,8 +1125,8 @@ static int tiles_of(int kind, const dims_t &m, int level, int rows, int &tx)
     case K_HL_ASM: w = m.hw[level]; h = m.hh[level]; th = BY * rows; break;
     case K_HL_DOUB: w = std::min((m.qw + 7) / 8 * 8, m.W); h = std::min((m.qh + 7) / 8 * 8, m.H); th = BY * rows; break;
     case K_GAUSS: w = m.cw; h = m.ch; th = BY * rows; break;
-    case K_DEVELOP: w = m.W; h = m.H; tw = dev_tile<0>::W; th = dev_tile<0>::H; break;
-    case K_DEVELOP_XT: w = m.W; h = m.H; tw = dev_tile<1>::W; th = dev_tile<1>::H; break;
+    case K_DEVELOP: case K_DEVELOP_XS: w = m.W; h = m.H; tw = dev_tile<DEV_BAYER>::W; th = dev_tile<DEV_BAYER>::H; break;
+    case K_DEVELOP_XT: w = m.W; h = m.H; tw = dev_tile<DEV_XT>::W; th = dev_tile<DEV_XT>::H; break;
     case K_PYR1: w = m.lw[1]; h = m.lh[1]; tw = P1_W; th = BY * P1_R; break;
     case K_REDUCE: case K_REDUCE_SPLIT: w = m.lw[level]; h = m.lh[level]; tw = 4 * BX; break;
     case K_TAIL: tx = 1; return 1;
@@ -1132,6 +1139,23 @@ static int tiles_of(int kind, const dims_t &m, int level, int rows, int &tx)
 }
 
 // launch sequence and job tables for the current tune
+// X-Trans images develop by site where their phase tiles are fewer than the
+// chip holds at once (5 work groups on each of 256 CUs): the stage then takes
+// as long as one tile, 105 us by phase against 53 by site.  780x520 alone 107 ->
+// 55 us, 1500x1000 128 -> 86; equal at 1300 to 1700 tiles, and above by phase is
+// faster (2688 tiles 216 us against 227, 5250 305 against 410)
+#define DEV_XT_TILES 1280
+static int dev_xt_sites(const std::vector<dims_t> &dm)
+{
+  long n = 0;
+  for(const dims_t &m : dm)
+  {
+    int tx;
+    if(m.block == 3) n += tiles_of(K_DEVELOP_XT, m, 0, 1, tx);
+  }
+  return n < DEV_XT_TILES;
+}
+
 static void build_launches(vkdt_batch_t *b)
 {
   b->seq.clear();
@@ -1147,7 +1171,7 @@ static void build_launches(vkdt_batch_t *b)
       if((kind == K_ASM || kind == K_ASM_SMALL) && level > std::min(m.nl - 2, m.tail - 1)) continue;
       if(kind == K_TAIL && m.tail >= m.nl) continue;
       if((kind == K_DEVELOP || kind == K_DOUB) && m.block == 3) continue;      // Bayer and X-Trans
-      if((kind == K_DEVELOP_XT || kind == K_DOUB_XT) && m.block != 3) continue;   // run as two launches
+      if((kind == K_DEVELOP_XT || kind == K_DEVELOP_XS || kind == K_DOUB_XT) && m.block != 3) continue;   // run as two launches
       if(kind >= K_HL_HALF && kind <= K_HL_DOUB && !m.hl) continue;
       if(kind == K_HL_REDUCE && level > m.hn) continue;
       if(kind == K_HL_ASM && level >= m.hn) continue;
@@ -1173,7 +1197,7 @@ static void build_launches(vkdt_batch_t *b)
   add(K_HL_DOUB, 0, 0);
   add(K_GAUSS, 0, 0);
   add(K_DEVELOP, 0, 0);
-  add(K_DEVELOP_XT, 0, 0);
+  add(dev_xt_sites(b->dm) ? K_DEVELOP_XS : K_DEVELOP_XT, 0, 0);
   add(K_PYR1, 1, 0);
   // a level's launch by the texels it has over all images
   auto texels = [&](int l) {
@@ -1287,8 +1311,9 @@ static int enqueue(vkdt_batch_t *b, hipStream_t s, int timed)
         case K_HL_ASM:  hipLaunchKernelGGL(kb_hl_asm<P>, grid, blk, 0, s, a); break;
         case K_HL_DOUB: hipLaunchKernelGGL(kb_hl_doub<P>, grid, blk, 0, s, a); break;
         case K_GAUSS:   hipLaunchKernelGGL(kb_gauss<P>, grid, blk, 0, s, a); break;
-        case K_DEVELOP: hipLaunchKernelGGL((kb_develop<0, P>), grid, blk, 0, s, a); break;
-        case K_DEVELOP_XT: hipLaunchKernelGGL((kb_develop<1, P>), grid, blk, 0, s, a); break;
+        case K_DEVELOP: hipLaunchKernelGGL((kb_develop<DEV_BAYER, P>), grid, blk, 0, s, a); break;
+        case K_DEVELOP_XT: hipLaunchKernelGGL((kb_develop<DEV_XT, P>), grid, blk, 0, s, a); break;
+        case K_DEVELOP_XS: hipLaunchKernelGGL((kb_develop<DEV_XT_SITE, P>), grid, blk, 0, s, a); break;
         case K_PYR1:    hipLaunchKernelGGL(kb_pyr1<P>, grid, blk, L.lds, s, a); break;
         case K_REDUCE:  hipLaunchKernelGGL((kb_reduce<0, P>), grid, blk, 0, s, a); break;
         case K_REDUCE_SPLIT: hipLaunchKernelGGL((kb_reduce<1, P>), grid, blk, 0, s, a); break;
