@@ -115,6 +115,20 @@ def test_first_reduction_tiles_equal_the_plain_graph(tmp_path, hip, W, Hh):
     c[0].close()
 
 
+def test_first_reduction_of_many_tiles_equals_the_plain_graph(tmp_path, hip):
+    """the same extents by waves of 63 x 4 outputs, which a launch takes from
+    1280 work groups of them on, and of 63 x 8, from 8192 on (a still of 24 x
+    57 work groups beside them, and twelve times the same; fewer, the tests
+    above, by waves of 63 x 2)"""
+    cs = [plain_and_planned(tmp_path, "bayer", W, Hh, 70 + n, dict())
+          for n, (W, Hh) in enumerate([(16, 12), (126, 64), (128, 66), (250, 130), (382, 18), (3000, 1810)])]
+    for n in (1, 12):
+        mix = cs + [cs[-1]] * (n - 1)
+        check_equal(batch.develop([c[0] for c in mix], [c[1] for c in mix]), mix, f"many tiles, {n}")
+    for c in cs:
+        c[0].close()
+
+
 def test_alone_equals_in_the_mix(cases):
     """each image developed in a batch of one equals its plain run too"""
     for i, c in enumerate(cases):

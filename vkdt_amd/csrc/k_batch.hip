@@ -433,7 +433,7 @@ __global__ void __launch_bounds__(256) kb_gauss(bt_launch L)
 // DEV_XT_SITE, X-Trans a site a thread with taps of any colour, for launches
 // of few tiles: a phase tile has nine phases of splat and of fix one after
 // the other for more than twice the texels, which a launch that does not fill
-// the chip waits for (see dev_xt_sites)
+// the chip waits for (see DEV_XT_TILES)
 enum { DEV_BAYER, DEV_XT, DEV_XT_SITE };
 template<int F> struct dev_tile { static constexpr int W = F == DEV_XT ? XT_TW : BX, H = F == DEV_XT ? XT_TH : BY * DEV_R; };
 
@@ -571,18 +571,24 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(F == D
 // ---- llap ------------------------------------------------------------------
 
 // curve + reduce, level 1 from filmcurv's output: a wave owns P1_W columns of
-// P1_R output rows and holds the luminance of their footprint, two columns a
+// R output rows and holds the luminance of their footprint, two columns a
 // lane (lane 0 those left of the tile), in registers.  Per plane every value
 // is evaluated once, rounded to binary16 as the curve node stores it, and
 // summed in reduce.comp's order; the third tap of a row is the previous lane's
 // and a row's sum is carried to the next output, so there is neither LDS nor a
 // barrier.  Bound by the curves' instructions: ten stills of 283 MP 2306 ->
-// 1705 us against a footprint staged in LDS (8 rows; 6 and 4 are 4 and 6 %
-// slower, with more footprint evaluated twice)
+// 1690 us against a footprint staged in LDS.  More rows evaluate fewer of them
+// twice, fewer rows leave less of the chip idle: eight from 8192 work groups of
+// them on (65 MP; ten stills 1690 us against 1790 with four), else four (a
+// 4096x2160 frame 72 us against 83 with eight; 24 MP 166 both), and two where
+// there are fewer work groups of four than the chip holds at once (5 a CU): the
+// launch then takes as long as one wave, 14 us against 20 at 640x480, 21
+// against 25 at 1500x1000
 #define P1_W (BX - 1)
-#define P1_R 8
+#define P1_MANY 8192
+#define P1_FEW 1280
 
-template<int P>
+template<int R, int P>
 __global__ void __launch_bounds__(256) kb_pyr1(bt_launch L)
 {
   __shared__ ll_args a;
@@ -593,16 +599,16 @@ __global__ void __launch_bounds__(256) kb_pyr1(bt_launch L)
     f = rfl(im.film); o = rfl(im.lp[1]);
   }, [&](const bt_job &jb, int lt) {
     const int ng = rfl(a.num_gamma), lane = threadIdx.x;
-    const int y = (lt / jb.tiles_x) * (BY * P1_R) + rfl((int)threadIdx.y) * P1_R;
+    const int y = (lt / jb.tiles_x) * (BY * R) + rfl((int)threadIdx.y) * R;
     const int x = (lt % jb.tiles_x) * P1_W - 1 + lane;
     if(y >= o.ht) return;
-    const int rows = min(P1_R, o.ht - y);
+    const int rows = min(R, o.ht - y);
     const bool own = lane > 0 && x < o.wd;
     const int xa = mirror(2 * x, f.wd), xb = mirror(2 * x + 1, f.wd);
     const ll_curve_k k = ll_curve_load(a);
-    float la[2 * P1_R + 1], lb[2 * P1_R + 1];
+    float la[2 * R + 1], lb[2 * R + 1];
 #pragma unroll
-    for(int j = 0; j < 2 * P1_R + 1; j++)
+    for(int j = 0; j < 2 * R + 1; j++)
     {
       const int fy = mirror(2 * y - 1 + j, f.ht);
       la[j] = ll_lum(ld_h4(f, xa, fy));
@@ -620,7 +626,7 @@ __global__ void __launch_bounds__(256) kb_pyr1(bt_launch L)
       float s0 = row(0);
       __half *q = out;
 #pragma unroll
-      for(int r = 0; r < P1_R; r++)
+      for(int r = 0; r < R; r++)
       {
         const float s1 = row(2 * r + 1), s2 = row(2 * r + 2);
         if(own && r < rows) *q = f2h((__builtin_fmaf(2.0f, s1, s0) + s2) * (1.0f / 16.0f));
@@ -857,8 +863,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 namespace {
 
 enum kind_t { K_HALF, K_DOWNCOV, K_DOWN, K_DNASM, K_DOUB, K_DOUB_XT, K_HL_HALF, K_HL_REDUCE, K_HL_ASM, K_HL_DOUB, K_GAUSS,
-              K_DEVELOP, K_DEVELOP_XT, K_DEVELOP_XS, K_PYR1, K_REDUCE, K_REDUCE_SPLIT, K_TAIL, K_ASM_SMALL, K_ASM, K_FINAL };
-const int kind_group[] = { 0, 1, 1, 2, 3, 3, 4, 4, 4, 4, 5, 6, 6, 6, 7, 8, 8, 8, 8, 8, 9 };
+              K_DEVELOP, K_DEVELOP_XT, K_DEVELOP_XS, K_PYR1_8, K_PYR1_4, K_PYR1_2, K_REDUCE, K_REDUCE_SPLIT, K_TAIL, K_ASM_SMALL, K_ASM, K_FINAL };
+const int kind_group[] = { 0, 1, 1, 2, 3, 3, 4, 4, 4, 4, 5, 6, 6, 6, 7, 7, 7, 8, 8, 8, 8, 8, 9 };
 const char *group_name[VKDT_BATCH_STAGES] = { "half", "wavelet", "dnasm", "doub", "hilite", "gauss", "develop",
                                               "pyr1", "pyramid", "final" };
 
@@ -1127,7 +1133,8 @@ static int tiles_of(int kind, const dims_t &m, int level, int rows, int &tx)
     case K_GAUSS: w = m.cw; h = m.ch; th = BY * rows; break;
     case K_DEVELOP: case K_DEVELOP_XS: w = m.W; h = m.H; tw = dev_tile<DEV_BAYER>::W; th = dev_tile<DEV_BAYER>::H; break;
     case K_DEVELOP_XT: w = m.W; h = m.H; tw = dev_tile<DEV_XT>::W; th = dev_tile<DEV_XT>::H; break;
-    case K_PYR1: w = m.lw[1]; h = m.lh[1]; tw = P1_W; th = BY * P1_R; break;
+    case K_PYR1_8: case K_PYR1_4: case K_PYR1_2:
+      w = m.lw[1]; h = m.lh[1]; tw = P1_W; th = BY * (8 >> (kind - K_PYR1_8)); break;
     case K_REDUCE: case K_REDUCE_SPLIT: w = m.lw[level]; h = m.lh[level]; tw = 4 * BX; break;
     case K_TAIL: tx = 1; return 1;
     case K_ASM_SMALL: w = m.lw[level]; h = m.lh[level]; break;
@@ -1145,15 +1152,16 @@ static int tiles_of(int kind, const dims_t &m, int level, int rows, int &tx)
 // 55 us, 1500x1000 128 -> 86; equal at 1300 to 1700 tiles, and above by phase is
 // faster (2688 tiles 216 us against 227, 5250 305 against 410)
 #define DEV_XT_TILES 1280
-static int dev_xt_sites(const std::vector<dims_t> &dm)
+// the tiles of a stage over the images of a CFA (block 2 or 3, 0 for all)
+static long tiles_all(const std::vector<dims_t> &dm, int kind, int level, int block)
 {
   long n = 0;
   for(const dims_t &m : dm)
   {
     int tx;
-    if(m.block == 3) n += tiles_of(K_DEVELOP_XT, m, 0, 1, tx);
+    if(!block || m.block == block) n += tiles_of(kind, m, level, 1, tx);
   }
-  return n < DEV_XT_TILES;
+  return n;
 }
 
 static void build_launches(vkdt_batch_t *b)
@@ -1197,8 +1205,8 @@ static void build_launches(vkdt_batch_t *b)
   add(K_HL_DOUB, 0, 0);
   add(K_GAUSS, 0, 0);
   add(K_DEVELOP, 0, 0);
-  add(dev_xt_sites(b->dm) ? K_DEVELOP_XS : K_DEVELOP_XT, 0, 0);
-  add(K_PYR1, 1, 0);
+  add(tiles_all(b->dm, K_DEVELOP_XT, 0, 3) < DEV_XT_TILES ? K_DEVELOP_XS : K_DEVELOP_XT, 0, 0);
+  add(tiles_all(b->dm, K_PYR1_8, 1, 0) >= P1_MANY ? K_PYR1_8 : tiles_all(b->dm, K_PYR1_4, 1, 0) >= P1_FEW ? K_PYR1_4 : K_PYR1_2, 1, 0);
   // a level's launch by the texels it has over all images
   auto texels = [&](int l) {
     size_t n = 0;
@@ -1314,7 +1322,9 @@ static int enqueue(vkdt_batch_t *b, hipStream_t s, int timed)
         case K_DEVELOP: hipLaunchKernelGGL((kb_develop<DEV_BAYER, P>), grid, blk, 0, s, a); break;
         case K_DEVELOP_XT: hipLaunchKernelGGL((kb_develop<DEV_XT, P>), grid, blk, 0, s, a); break;
         case K_DEVELOP_XS: hipLaunchKernelGGL((kb_develop<DEV_XT_SITE, P>), grid, blk, 0, s, a); break;
-        case K_PYR1:    hipLaunchKernelGGL(kb_pyr1<P>, grid, blk, L.lds, s, a); break;
+        case K_PYR1_8:  hipLaunchKernelGGL((kb_pyr1<8, P>), grid, blk, 0, s, a); break;
+        case K_PYR1_4:  hipLaunchKernelGGL((kb_pyr1<4, P>), grid, blk, 0, s, a); break;
+        case K_PYR1_2:  hipLaunchKernelGGL((kb_pyr1<2, P>), grid, blk, 0, s, a); break;
         case K_REDUCE:  hipLaunchKernelGGL((kb_reduce<0, P>), grid, blk, 0, s, a); break;
         case K_REDUCE_SPLIT: hipLaunchKernelGGL((kb_reduce<1, P>), grid, blk, 0, s, a); break;
         case K_TAIL:    hipLaunchKernelGGL(kb_tail, grid, dim3(BX, LL_TAIL_Y), L.lds, s, a); break;
