@@ -96,12 +96,13 @@ def test_xtrans_tiles_equal_the_plain_graph(tmp_path, hip, W, Hh, kw):
 
 def test_xtrans_phases_equal_the_plain_graph(tmp_path, hip):
     """the fused X-Trans develop by phase, which a launch takes from 1280 tiles
-    on (below, the tests above, by site): the tile cases above, each in a batch
-    with a still of 25 x 58 tiles"""
+    on (below, the tests above, by site), and doub by cells, from 700000 on
+    (below, by their rows): the tile cases above, each in a batch with two
+    stills of 25 x 58 tiles and 770 x 462 cells"""
     big = plain_and_planned(tmp_path, "xtrans", 2310, 1386, 64, dict())
     for n, (W, Hh, kw) in enumerate(((96, 24, dict()), (294, 81, dict()), (390, 123, dict(extra=["param:demosaic:01:colour:1"])))):
         c = plain_and_planned(tmp_path, "xtrans", W, Hh, 65 + n, kw)
-        check_equal(batch.develop([c[0], big[0]], [c[1], big[1]]), [c, big], f"{W}x{Hh} and 2310x1386")
+        check_equal(batch.develop([c[0], big[0], big[0]], [c[1], big[1], big[1]]), [c, big, big], f"{W}x{Hh} and 2310x1386")
         c[0].close()
     big[0].close()
 

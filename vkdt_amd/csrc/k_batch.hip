@@ -272,10 +272,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) k
 // cells.  Instructions bound both.  Two kernels: in one, X-Trans took a texel
 // per thread with the registers of the Bayer branch (four waves per SIMD);
 // doub of ten stills, 283 MP of both kinds, went from 3240 to 1559 us
-template<int XT, int P>
+// B: 0 Bayer, 3 X-Trans cells, 1 their rows, three times the threads, for launches
+// of fewer than DOUB_CELLS cells: nine texels a thread are 26 us however small
+// the image, three 13 (1500x1000 28 -> 17 us, 3000x2000 44 -> 40; above, cells
+// share more: 984k cells 54 us against 56, 24 MP 129 against 133)
+#define DOUB_CELLS 700000
+template<int B, int P>
 __global__ void __launch_bounds__(256) kb_doub(bt_launch L)
 {
-  constexpr int B = XT ? 3 : 2;
   __shared__ dn_args a;
   dimg cfa, crs0, crs1, o;
   bt_tiles<P>(L, [&](const bt_job &jb) {
@@ -283,22 +287,23 @@ __global__ void __launch_bounds__(256) kb_doub(bt_launch L)
     lds_copy(a, im.dn_doub);
     cfa = rfl(im.cfa); crs0 = rfl(im.qa); crs1 = rfl(im.qh); o = rfl(im.dmos);
   }, [&](const bt_job &jb, int lt) {
-    const int cx = (lt % jb.tiles_x) * BX + threadIdx.x, Y0 = (lt / jb.tiles_x) * (BY * L.rows);
+    const int cx = (lt % jb.tiles_x) * BX + threadIdx.x, Y0 = (lt / jb.tiles_x) * (BY * L.rows) + rfl((int)threadIdx.y);
 #pragma unroll 1
     for(int k = 0; k < L.rows; k++)
     {
-      const int cy = Y0 + threadIdx.y + BY * k;
-      if(B * cx >= o.wd || B * cy >= o.ht) continue;
-      float v[B * B];
-      if(XT)
+      const int y = (B ? B : 2) * (Y0 + BY * k);
+      if((B ? 3 : 2) * cx >= o.wd || y >= o.ht) continue;
+      if constexpr(B != 0)
       {
-        dn_doub_cell(cfa, crs0, crs1, o.wd, o.ht, a, cx, cy, v);
-        st_h1_cell(o, cx, cy, v);
+        float v[3 * B];
+        dn_doub_cell<B>(cfa, crs0, crs1, o.wd, o.ht, a, cx, y, v);
+        st_h1_cell<B>(o, cx, y, v);
       }
       else
       {
-        dn_doub_quad(cfa, crs0, crs1, o.wd, o.ht, a, 2 * cx, 2 * cy, v);
-        st_h1_quad(o, 2 * cx, 2 * cy, v);
+        float v[4];
+        dn_doub_quad(cfa, crs0, crs1, o.wd, o.ht, a, 2 * cx, y, v);
+        st_h1_quad(o, 2 * cx, y, v);
       }
     }
   });
@@ -862,9 +867,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) k
 
 namespace {
 
-enum kind_t { K_HALF, K_DOWNCOV, K_DOWN, K_DNASM, K_DOUB, K_DOUB_XT, K_HL_HALF, K_HL_REDUCE, K_HL_ASM, K_HL_DOUB, K_GAUSS,
+enum kind_t { K_HALF, K_DOWNCOV, K_DOWN, K_DNASM, K_DOUB, K_DOUB_XT, K_DOUB_XR, K_HL_HALF, K_HL_REDUCE, K_HL_ASM, K_HL_DOUB, K_GAUSS,
               K_DEVELOP, K_DEVELOP_XT, K_DEVELOP_XS, K_PYR1_8, K_PYR1_4, K_PYR1_2, K_REDUCE, K_REDUCE_SPLIT, K_TAIL, K_ASM_SMALL, K_ASM, K_FINAL };
-const int kind_group[] = { 0, 1, 1, 2, 3, 3, 4, 4, 4, 4, 5, 6, 6, 6, 7, 7, 7, 8, 8, 8, 8, 8, 9 };
+const int kind_group[] = { 0, 1, 1, 2, 3, 3, 3, 4, 4, 4, 4, 5, 6, 6, 6, 7, 7, 7, 8, 8, 8, 8, 8, 9 };
 const char *group_name[VKDT_BATCH_STAGES] = { "half", "wavelet", "dnasm", "doub", "hilite", "gauss", "develop",
                                               "pyr1", "pyramid", "final" };
 
@@ -1108,7 +1113,7 @@ static int build_image(bt_img &b, const vkdt_develop_image_t &d, const dims_t &m
 
 static int is_pixel_stage(int kind)
 {
-  return kind == K_HALF || kind == K_DNASM || kind == K_DOUB || kind == K_DOUB_XT || kind == K_GAUSS || kind == K_HL_HALF ||
+  return kind == K_HALF || kind == K_DNASM || kind == K_DOUB || kind == K_DOUB_XT || kind == K_DOUB_XR || kind == K_GAUSS || kind == K_HL_HALF ||
          kind == K_HL_ASM || kind == K_HL_DOUB;
 }
 
@@ -1126,6 +1131,7 @@ static int tiles_of(int kind, const dims_t &m, int level, int rows, int &tx)
     case K_DOWNCOV: w = m.qw; h = m.qh; th = BY * COV_R; break;
     case K_DOWN: w = m.qw; h = m.qh; th = BY * DOWN_R; break;
     case K_DOUB: case K_DOUB_XT: w = (m.W + m.block - 1) / m.block; h = (m.H + m.block - 1) / m.block; th = BY * rows; break;
+    case K_DOUB_XR: w = (m.W + 2) / 3; h = m.H; th = BY * rows; break;
     case K_HL_HALF: w = m.qw; h = m.qh; th = BY * rows; break;
     case K_HL_REDUCE: w = m.hw[level]; h = m.hh[level]; break;
     case K_HL_ASM: w = m.hw[level]; h = m.hh[level]; th = BY * rows; break;
@@ -1179,7 +1185,7 @@ static void build_launches(vkdt_batch_t *b)
       if((kind == K_ASM || kind == K_ASM_SMALL) && level > std::min(m.nl - 2, m.tail - 1)) continue;
       if(kind == K_TAIL && m.tail >= m.nl) continue;
       if((kind == K_DEVELOP || kind == K_DOUB) && m.block == 3) continue;      // Bayer and X-Trans
-      if((kind == K_DEVELOP_XT || kind == K_DEVELOP_XS || kind == K_DOUB_XT) && m.block != 3) continue;   // run as two launches
+      if((kind == K_DEVELOP_XT || kind == K_DEVELOP_XS || kind == K_DOUB_XT || kind == K_DOUB_XR) && m.block != 3) continue;   // run as two launches
       if(kind >= K_HL_HALF && kind <= K_HL_DOUB && !m.hl) continue;
       if(kind == K_HL_REDUCE && level > m.hn) continue;
       if(kind == K_HL_ASM && level >= m.hn) continue;
@@ -1198,7 +1204,9 @@ static void build_launches(vkdt_batch_t *b)
   for(int l = 1; l < 4; l++) add(K_DOWN, l, 0);
   add(K_DNASM, 0, 0);
   add(K_DOUB, 0, 0);
-  add(K_DOUB_XT, 0, 0);
+  size_t cells = 0;
+  for(const dims_t &m : b->dm) if(m.block == 3) cells += (size_t)((m.W + 2) / 3) * ((m.H + 2) / 3);
+  add(cells < DOUB_CELLS ? K_DOUB_XR : K_DOUB_XT, 0, 0);
   add(K_HL_HALF, 0, 0);
   for(int l = 1; l <= b->max_hn; l++) add(K_HL_REDUCE, l, 0);
   for(int l = b->max_hn - 1; l >= 0; l--) add(K_HL_ASM, l, 0);
@@ -1313,7 +1321,8 @@ static int enqueue(vkdt_batch_t *b, hipStream_t s, int timed)
         case K_DOWN:    hipLaunchKernelGGL(kb_down<P>, grid, blk, 0, s, a); break;
         case K_DNASM:   hipLaunchKernelGGL(kb_dnasm<P>, grid, blk, 0, s, a, b->mats); break;
         case K_DOUB:    hipLaunchKernelGGL((kb_doub<0, P>), grid, blk, 0, s, a); break;
-        case K_DOUB_XT: hipLaunchKernelGGL((kb_doub<1, P>), grid, blk, 0, s, a); break;
+        case K_DOUB_XT: hipLaunchKernelGGL((kb_doub<3, P>), grid, blk, 0, s, a); break;
+        case K_DOUB_XR: hipLaunchKernelGGL((kb_doub<1, P>), grid, blk, 0, s, a); break;
         case K_HL_HALF: hipLaunchKernelGGL(kb_hl_half<P>, grid, blk, 0, s, a); break;
         case K_HL_REDUCE: hipLaunchKernelGGL(kb_hl_reduce<P>, grid, blk, 0, s, a); break;
         case K_HL_ASM:  hipLaunchKernelGGL(kb_hl_asm<P>, grid, blk, 0, s, a); break;

@@ -86,16 +86,17 @@ __global__ void __launch_bounds__(256) k_dn_assemble(dimg s0, dimg s1, dimg s2, 
   st_h4(out, x, y, dn_assemble_px(s0, s1, s2, s3, s4, a, m, x, y));
 }
 
-// X-Trans mosaics: one 3x3 cell per thread (dn_doub_cell); the gain map is
-// Bayer's alone.  Bound by instructions; a texel per thread took 161 us at
-// 26 MP, the cell 131
+// X-Trans mosaics: one row of a 3x3 cell per thread (dn_doub_cell); the gain map
+// is Bayer's alone.  Bound by instructions; a texel per thread took 161 us at
+// 26 MP, a cell 131, which on small images waited for its nine texels (26 us
+// however small, a row 13)
 __global__ void __launch_bounds__(256) k_dn_doub_xtrans(dimg in, dimg crs0, dimg crs1b, dimg out, dn_args a)
 {
-  const int cx = tid_x(), cy = tid_y();
-  if(3 * cx >= out.wd || 3 * cy >= out.ht) return;
-  float v[9];
-  dn_doub_cell(in, crs0, crs1b, out.wd, out.ht, a, cx, cy, v);
-  st_h1_cell(out, cx, cy, v);
+  const int cx = tid_x(), y = __builtin_amdgcn_readfirstlane(tid_y());
+  if(3 * cx >= out.wd || y >= out.ht) return;
+  float v[3];
+  dn_doub_cell<1>(in, crs0, crs1b, out.wd, out.ht, a, cx, y, v);
+  st_h1_cell<1>(out, cx, y, v);
 }
 
 // Bayer mosaics: one 2x2 block per thread (dn_doub_quad)
@@ -248,7 +249,7 @@ int launch_denoise_doub(const node_call &c)
   read_params(a, c);
   if(int e = read_gainmap(a, c, 4, pi[19], pf + 20, "denoise/doub gainmap")) return e;
   if(a.filters == 9)
-    hipLaunchKernelGGL(k_dn_doub_xtrans, grid2d((c.wd + 2) / 3, (c.ht + 2) / 3, 1), dim3(BX, BY), 0, c.stream,
+    hipLaunchKernelGGL(k_dn_doub_xtrans, grid2d((c.wd + 2) / 3, c.ht, 1), dim3(BX, BY), 0, c.stream,
                        to_dimg(c.conn[0]), to_dimg(c.conn[1]), to_dimg(c.conn[2]), to_dimg(c.conn[3]), a);
   else
     hipLaunchKernelGGL(k_dn_doub_bayer, grid2d((c.wd + 1) / 2, (c.ht + 1) / 2, 1), dim3(BX, BY), 0, c.stream,

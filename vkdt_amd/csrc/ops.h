@@ -591,51 +591,59 @@ DEV float2 bilin_h4_rb(const dimg &b, const bl_axis &ax, const bl_axis &ay, bool
   return r;
 }
 
-// the same on X-Trans mosaics for the 3x3 cell (cx, cy), v in row order: five
-// green texels, and two each of red and blue that swap with the cell's
-// parity.  A texel per thread formed its own axes (four divisions, eight
-// mirrored taps) and interpolated eight channels of which it used three
-DEV void dn_doub_cell(const dimg &in, const dimg &crs0, const dimg &crs1b, int owd, int oht, const dn_args &a,
-                      int cx, int cy, float v[9])
+// the same on X-Trans mosaics for a row of a 3x3 cell of parity `odd`, MID the
+// middle one: green texels, and red and blue ones that swap with the parity and
+// the middle row (xtrans_colour)
+template<bool MID>
+DEV void dn_doub_xrow(const dimg &crs0, const dimg &crs1b, const dn_args &a, const bl_axis ux[3], const bl_axis &uy,
+                      const bl_axis dx[3], const bl_axis &dy, bool odd, const float raw[3], float v[3])
 {
-  bl_axis ux[3], uy[3], dx[3], dy[3];
+  const bool blue = odd ^ MID;
+#pragma unroll
+  for(int i = 0; i < 3; i++)
+    if((i == 1) == MID)
+    {
+      const float2 up = bilin_h4_chan<1, true>(crs0, ux[i], uy);
+      const float dn = bilin_h4_chan<1, false>(crs1b, dx[i], dy).x;
+      v[i] = dn_doub_tail(a, a.black[1], a.white[1], a.inv_range[1], up.x, dn, up.y, 0.5f * a.strength * up.y, a.luma, raw[i]);
+    }
+    else
+    {
+      const float2 up = bilin_h4_rb<true>(crs0, ux[i], uy, blue);
+      const float dn = bilin_h4_rb<false>(crs1b, dx[i], dy, blue).x;
+      v[i] = dn_doub_tail(a, blue ? a.black[2] : a.black[0], blue ? a.white[2] : a.white[0],
+                          blue ? a.inv_range[2] : a.inv_range[0], up.x, dn, up.y,
+                          0.5f * a.strength * up.y * frcp(fmaxf(1e-4f, up.y)), 1.0f, raw[i]);
+    }
+}
+
+// ROWS 3: the 3x3 cell at column 3 cx, row y = 3 cy.  ROWS 1: one row of it, at
+// row y, the same for a whole wave.  v in row order.  A texel per thread formed
+// its own axes (four divisions, eight mirrored taps) and interpolated eight
+// channels of which it used three
+template<int ROWS>
+DEV void dn_doub_cell(const dimg &in, const dimg &crs0, const dimg &crs1b, int owd, int oht, const dn_args &a,
+                      int cx, int y, float v[3 * ROWS])
+{
+  bl_axis ux[3], uy[ROWS], dx[3], dy[ROWS];
   dn_doub_axes<3>(ux, 3 * cx, owd, crs0.wd);
   dn_doub_axes<3>(dx, 3 * cx, owd, crs1b.wd);
-  dn_doub_axes<3>(uy, 3 * cy, oht, crs0.ht);
-  dn_doub_axes<3>(dy, 3 * cy, oht, crs1b.ht);
-  int mx[3], my[3];
+  dn_doub_axes<ROWS>(uy, y, oht, crs0.ht);
+  dn_doub_axes<ROWS>(dy, y, oht, crs1b.ht);
+  int mx[3], my[ROWS];
 #pragma unroll
-  for(int k = 0; k < 3; k++)
-  {
-    mx[k] = mirror(3 * cx + k + a.crop[0], in.wd);
-    my[k] = mirror(3 * cy + k + a.crop[1], in.ht);
-  }
-  float raw[9];
+  for(int k = 0; k < 3; k++) mx[k] = mirror(3 * cx + k + a.crop[0], in.wd);
 #pragma unroll
-  for(int k = 0; k < 9; k++) raw[k] = ld_u16(in, mx[k % 3], my[k / 3]);
+  for(int k = 0; k < ROWS; k++) my[k] = mirror(y + k + a.crop[1], in.ht);
+  float raw[3 * ROWS];
+#pragma unroll
+  for(int k = 0; k < 3 * ROWS; k++) raw[k] = ld_u16(in, mx[k % 3], my[k / 3]);
+  const int cy = y / 3;
   const bool odd = ((cx + cy) & 1) != 0;
 #pragma unroll
-  for(int j = 0; j < 3; j++)
-#pragma unroll
-    for(int i = 0; i < 3; i++)
-    {
-      const int k = 3 * j + i;
-      if(((i + j) & 1) == 0)
-      {
-        const float2 up = bilin_h4_chan<1, true>(crs0, ux[i], uy[j]);
-        const float dn = bilin_h4_chan<1, false>(crs1b, dx[i], dy[j]).x;
-        v[k] = dn_doub_tail(a, a.black[1], a.white[1], a.inv_range[1], up.x, dn, up.y, 0.5f * a.strength * up.y, a.luma, raw[k]);
-      }
-      else
-      { // xtrans_colour
-        const bool blue = odd ^ (j == 1);
-        const float2 up = bilin_h4_rb<true>(crs0, ux[i], uy[j], blue);
-        const float dn = bilin_h4_rb<false>(crs1b, dx[i], dy[j], blue).x;
-        v[k] = dn_doub_tail(a, blue ? a.black[2] : a.black[0], blue ? a.white[2] : a.white[0],
-                            blue ? a.inv_range[2] : a.inv_range[0], up.x, dn, up.y,
-                            0.5f * a.strength * up.y * frcp(fmaxf(1e-4f, up.y)), 1.0f, raw[k]);
-      }
-    }
+  for(int j = 0; j < ROWS; j++)
+    if(ROWS == 3 ? j == 1 : y - 3 * cy == 1) dn_doub_xrow<true>(crs0, crs1b, a, ux, uy[j], dx, dy[j], odd, raw + 3 * j, v + 3 * j);
+    else dn_doub_xrow<false>(crs0, crs1b, a, ux, uy[j], dx, dy[j], odd, raw + 3 * j, v + 3 * j);
 }
 
 // store the 2x2 block at even (x, y) of an f16 plane, v in row order: each
@@ -657,13 +665,14 @@ DEV void st_h1_quad(const dimg &o, int x, int y, const float v[4])
   }
 }
 
-// store the 3x3 cell (cx, cy) of an f16 plane, v in row order
-DEV void st_h1_cell(const dimg &o, int cx, int cy, const float v[9])
+// store dn_doub_cell's texels of an f16 plane
+template<int ROWS>
+DEV void st_h1_cell(const dimg &o, int cx, int y0, const float v[3 * ROWS])
 {
 #pragma unroll
-  for(int k = 0; k < 9; k++)
+  for(int k = 0; k < 3 * ROWS; k++)
   {
-    const int x = 3 * cx + k % 3, y = 3 * cy + k / 3;
+    const int x = 3 * cx + k % 3, y = y0 + k / 3;
     if(x < o.wd && y < o.ht) st_h1(o, x, y, v[k]);
   }
 }
