@@ -15,6 +15,7 @@
 // of the scan at (i mod tile_wd, i div tile_wd)); sites outside the image
 // are decoded and dropped.
 #include "launch.h"
+#include "lj92_pos.h"
 
 #include <map>
 #include <string.h>
@@ -911,7 +912,7 @@ __global__ void __launch_bounds__(256) k_lj92_write(const lj92_pst *ps, int np, 
     // a tail runs on into the zeros after the data, which reach past the staged words
     const uint32_t x = lj92_window(l, min(pos - kb * LJ92_SUB, 32u * (LJ92_LW - 2))), e = lj92_sym(l, x);
     if((e & 31) == 31) { atomicAdd(status, 1); return; }      // a sample of the scan with no valid code
-    pos += e >> 10;
+    pos = lj92_next(pos, e >> 10, B);
     const uint32_t len = e & 31, cat = (e >> 5) & 31;
     // the category's bits; a leading zero marks a negative difference
     int d = cat == 16 ? 32768 : (int)(((x << len) >> 1) >> (31 - cat));
