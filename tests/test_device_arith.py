@@ -135,3 +135,48 @@ def test_llap_expand_sum_form():
             rows = np.stack([_expand5(ox, t[j]) for j in range(5)])
             got = (np.float32(0.25) * _expand5(oy, rows)).astype(np.float32)
             assert np.array_equal(got, ref), (ox, oy, int((got != ref).sum()))
+
+
+@pytest.mark.gpu
+def test_device_division(hip):
+    """common.h rcp_rn and div_rn as the kernels have them, on the GPU: equal to
+    IEEE division for every mantissa at exponents over the ranges they are for
+    (2^-125 to 2^125 and 2^-40 to 2^32, both ends), of both signs, and for
+    zeros, infinities and NaN"""
+    import ctypes as C
+    import os
+    from vkdt_amd import hip as H
+    L = C.CDLL(os.path.join(os.path.dirname(os.path.abspath(H.__file__)), "lib", "libvkdt_calib.so"))
+    L.vkdt_calib_div.argtypes = [C.c_void_p] * 4 + [C.c_long, C.c_void_p]
+
+    def run(a, b):
+        a, b = np.ascontiguousarray(a, np.float32), np.ascontiguousarray(b, np.float32)
+        bufs = [H.DeviceBuffer(a.size, 1, 1, H.FMT_F32) for _ in range(4)]
+        bufs[0].upload(a.reshape(1, -1))
+        bufs[1].upload(b.reshape(1, -1))
+        H.check(L.vkdt_calib_div(*[x.ptr for x in bufs], a.size, None), "division")
+        H.sync()
+        out = [x.download().reshape(-1) for x in bufs[2:]]
+        for x in bufs:
+            x.free()
+        return out
+
+    def same(got, want):
+        return (got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))
+
+    rng = np.random.default_rng(11)
+    mant = np.arange(1 << 23, dtype=np.uint32)
+    for e in (-125, -60, -40, -24, -1, 0, 1, 16, 31, 90, 124):
+        b = (mant | np.uint32((e + 127) << 23) | (mant & 1) << 31).view(np.float32)
+        ea = rng.integers(-40, 32, b.size)
+        a = (rng.integers(0, 1 << 23, b.size).astype(np.uint32) | ((ea + 127).astype(np.uint32) << 23)).view(np.float32)
+        r, q = run(a, b)
+        bad_r = int((~same(r, np.float32(1) / b)).sum())
+        bad_q = int((~same(q, a / b)).sum()) if -40 <= e < 32 else 0      # the range div_rn is for
+        print(f"[arith] 2^{e}: reciprocals {bad_r}, quotients {bad_q} differ of {b.size}", flush=True)
+        assert bad_r == 0 and bad_q == 0, e
+    v = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1.0, -3.0, 65504.0, 6e-8], np.float32)
+    a, b = (x.reshape(-1) for x in np.meshgrid(v, v))
+    with np.errstate(all="ignore"):
+        r, q = run(a, b)
+        assert same(r, np.float32(1) / b).all() and same(q, a / b).all(), list(zip(a, b, r, q))

@@ -1,7 +1,7 @@
 """Build the native parts in-tree.
 
   vkdt_amd/lib/libvkdt_hip.so    HIP kernels + C ABI (hipcc, gfx950)
-  vkdt_amd/lib/libvkdt_calib.so  instruction-rate calibration kernels (bench.py)
+  vkdt_amd/lib/libvkdt_calib.so  instruction-rate calibration kernels (bench.py), the division test's kernel
   vkdt_amd/lib/libvkdt_pipe.so   host graph runtime (C, gcc)
   vkdt_amd/modules/<m>/lib<m>.so module DSOs (C, gcc)
   vkdt_amd/bin/vkdt-cli          command line front end
@@ -56,10 +56,12 @@ def build_hip():
 
 
 def build_calib():
-    """the instruction-rate calibration kernels bench.py --calibrate-valu times"""
+    """the instruction-rate calibration kernels bench.py --calibrate-valu times,
+    and the kernels' division over arrays for its test"""
     os.makedirs(LIB, exist_ok=True)
     out = os.path.join(LIB, "libvkdt_calib.so")
-    run([HIPCC] + HIP_FLAGS + ["-shared", "-o", out + ".tmp", os.path.join(CSRC, "calib", "calib.hip")])
+    run([HIPCC] + HIP_FLAGS + ["-shared", "-o", out + ".tmp"]
+        + [os.path.join(CSRC, "calib", s) for s in ("calib.hip", "arith.hip")])
     os.replace(out + ".tmp", out)
     return out
 

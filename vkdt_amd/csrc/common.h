@@ -63,10 +63,12 @@ DEV float fpow(float x, float y) { return __builtin_amdgcn_exp2f(y * __builtin_a
 // IEEE 1/x and a/b (given y = rcp_rn(b)) in 4 instructions each for the compiler's 11,
 // which scales operands that need it: an approximation within an ulp, one exact
 // residual and one rounding, with zeros, infinities and nan put right by
-// v_div_fixup.  rcp_rn equals 1/x for every x of magnitude 2^-125 to 2^125 and
-// the special values (compared over all of them on a gfx950); div_rn had no
-// differing bit over 6.9e10 random pairs of magnitudes 2^-40 to 2^32.  Results
-// or residuals below 2^-126 may be a last place off.
+// v_div_fixup.  rcp_rn equals 1/x for every x of magnitude 2^-125 to 2^125, 0,
+// infinity and nan (compared over all of them on a gfx950); div_rn had no
+// differing bit over 6.9e10 random pairs of magnitudes 2^-40 to 2^32, and takes
+// the same special values.  Outside, they are not for use: a denormal x has an
+// infinite approximation and nan for a reciprocal, one above 2^126 has 0, and
+// a quotient or residual below 2^-126 may be a last place off
 DEV float rcp_rn(float x)
 {
   const float y = __builtin_amdgcn_rcpf(x);
