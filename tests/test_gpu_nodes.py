@@ -244,7 +244,7 @@ def test_llap_assemble_planes(hip, ng, step):
 @pytest.mark.parametrize("W,H", [(96 * 30, 24 * 18 + 6), (96 * 46 + 3, 24 * 46)])
 def test_xtrans_tiles_in_parts(hip, W, H):
     """splat and fix above the tile counts at which a tile is cut into nine
-    parts, three and none (540 and 2162 tiles; the smaller extents of
+    parts, three and none (570 and 2162 tiles; the smaller extents of
     test_xtrans_tiles have nine): the general path's values, which a graph cut
     to a part of the image gives, away from the cut"""
     import numpy as np

@@ -983,7 +983,7 @@ dimg mk(void *p, int wd, int ht, int pitch, int chan, long pstride, int fmt = DI
 
 struct vkdt_batch_t
 {
-  int n = 0, ncu = 256, max_nl = 0, max_ng = 0, max_hn = 0;
+  int n = 0, ncu = 256, max_nl = 0, max_hn = 0;
   std::vector<dims_t> dm;
   std::vector<bt_img> img;         // host copies of the device tables
   std::vector<bt_job> job;
@@ -1239,14 +1239,13 @@ int vkdt_hip_batch_create(vkdt_batch_t **out, const vkdt_develop_image_t *img, i
   *out = nullptr;
   std::vector<dims_t> dm(n);
   size_t need = 0;
-  int max_nl = 0, max_ng = 0, max_hn = 0;
+  int max_nl = 0, max_hn = 0;
   for(int i = 0; i < n; i++)
   {
     if(int e = image_dims(img[i], dm[i], i)) return e;
     if(!img[i].cfa || !img[i].out) return vkdt_set_error(VKDT_HIP_INCOMPLETE, "batch image %d: no mosaic or output", i);
     need += image_scratch(dm[i]);
     max_nl = std::max(max_nl, dm[i].nl);
-    max_ng = std::max(max_ng, dm[i].ng);
     max_hn = std::max(max_hn, dm[i].hn);
   }
   const size_t tables = need;
@@ -1264,7 +1263,6 @@ int vkdt_hip_batch_create(vkdt_batch_t **out, const vkdt_develop_image_t *img, i
   b->dm = dm;
   b->img = h;
   b->max_nl = max_nl;
-  b->max_ng = max_ng;
   b->max_hn = max_hn;
   for(int s = 0; s < VKDT_BATCH_STAGES; s++) b->tune[s] = tune ? tune[s] : (4 << 8);
   asm_mats_init(b->mats);

@@ -109,7 +109,7 @@ __global__ void __launch_bounds__(256) k_dm_fix(dimg in, dimg gr, dimg cv, dimg 
 // time; tiles whose taps leave the image take the general path per site.
 // gridDim.z parts share a tile's phases (or sites): a tile alone takes about
 // 40 us, which images of few tiles wait for instead of filling the chip (see
-// xt_parts)
+// xt_grid)
 template<int U16>
 __global__ void __launch_bounds__(256) k_dm_splat_xt(dimg in, dimg ga, dimg out)
 {
