@@ -35,7 +35,8 @@ int launch_post(const char *what) { return hip_fail(hipGetLastError(), what); }
 // of a small image.  With pooled blocks, no further look at sizes and no copy
 // of the caller's or the result's bytes: JPEG 1620x1080 266 -> 198 us, 24 MP
 // 3.8 -> 1.3 ms, lossless JPEG 24 MP 2.4 -> 1.64 ms, a 6 MP 14-bit unpack 680 ->
-// 355 us (its upload takes 340).
+// 355 us (its upload takes 340; the last two where pageable uploads run at 30
+// GB/s, and where they are slower those decide).
 
 namespace {
 struct hip_memory

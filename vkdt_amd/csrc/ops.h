@@ -185,7 +185,7 @@ struct dn_cov_smem { float4 tile[DN_TN(R)]; float lum[DN_TN(R)], rlum[DN_TN(R)],
 // s + k v for an offset |k| <= 2: the product is exact, so fusing it changes
 // nothing, and a zero is left out.  That leaves a NaN out where v is infinite
 // or NaN; the tensor's sums are NaN there with or without it (their weights
-// v v are infinite or NaN, and divided by their own sum)
+// v v are infinite or NaN, and divided by their own sum), if of another sign
 DEV float add_times(float s, int k, float v) { return k == 0 ? s : __builtin_fmaf((float)k, v, s); }
 
 // Bound by instructions.  With the divisions in four instructions (rcp_rn,
@@ -1330,8 +1330,8 @@ DEV void ll_reduce_px4(const dimg &in, const dimg &out, int planes, int x0, int 
 // shares 3/4 of a row of each plane.  A lane loads one value of two rows and
 // takes its five taps from the wave's other lanes, so the rows need no
 // staging, and two rows of binary16 travel as one word.  kb_final of ten
-// stills (283 MP) 2492 -> 1842 us, kb_asm 693 -> 538, k_ll_assemble's large
-// levels at 24 MP 236 -> 186.
+// stills (283 MP) 2492 -> 1842 us (now 1906: see ll_curve), kb_asm 693 -> 552,
+// k_ll_assemble's large levels at 24 MP 236 -> 188.
 //   first          the coarsest level: expand the luminance plane of l1
 //                  instead of a coarse reconstruction
 //   v[k]           the fine luminance plane at the thread's texel k
