@@ -88,7 +88,8 @@ def test_coarse_levels_equal_the_plain_graph(tmp_path, hip, W, Hh, kw):
 @pytest.mark.parametrize("W,Hh,kw", [(96, 24, dict()), (294, 81, dict()), (390, 123, dict(extra=["param:demosaic:01:colour:1"]))],
                          ids=["one-tile", "inner-tile", "radius-3"])
 def test_xtrans_tiles_equal_the_plain_graph(tmp_path, hip, W, Hh, kw):
-    """the fused X-Trans develop tiles of 96x24: none, one and several inside"""
+    """the fused X-Trans develop of few tiles, by site (by phase in tiles of
+    96x24: the next test): extents with none, one and several of them inside"""
     c = plain_and_planned(tmp_path, "xtrans", W, Hh, 62, kw)
     check_equal(batch.develop([c[0]], [c[1]]), [c], f"{W}x{Hh} {kw}")
     c[0].close()
@@ -109,8 +110,9 @@ def test_xtrans_phases_equal_the_plain_graph(tmp_path, hip):
 
 @pytest.mark.parametrize("W,Hh", [(16, 12), (126, 64), (128, 66), (250, 130), (382, 18)])
 def test_first_reduction_tiles_equal_the_plain_graph(tmp_path, hip, W, Hh):
-    """the pyramid's first level, made from the image by waves of 63 x 8
-    outputs: one, exactly full, one column and row over, partial ones"""
+    """the pyramid's first level, made from the image by waves of 63 x 2
+    outputs (of more rows in larger launches: the next test): one, exactly
+    full, one column and row over, partial ones"""
     c = plain_and_planned(tmp_path, "bayer", W, Hh, 63, dict())
     check_equal(batch.develop([c[0]], [c[1]]), [c], f"{W}x{Hh}")
     c[0].close()

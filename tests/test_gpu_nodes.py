@@ -96,7 +96,7 @@ def test_xtrans_tiles(hip, fmt, W, H):
                                             ("xtrans", 3, 3, 0, 0), ("xtrans", 97, 26, 0, 0), ("xtrans", 100, 25, 6, 3),
                                             ("xtrans", 195, 51, 1, 2)])
 def test_doub_blocks(hip, kind, W, H, cx, cy):
-    """denoise/doub, a block or cell per thread, where the last ones are cut
+    """denoise/doub, a block or a cell's row per thread, where the last ones are cut
     (one and two columns and rows left), the output is one block, and the crop
     moves it over the mosaic's mirrored edge: against the oracle on the same
     inputs"""
