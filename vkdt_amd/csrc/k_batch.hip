@@ -71,7 +71,6 @@ struct bt_launch
   const bt_job *job;
   int njob, total;
   int *ctr;          // NUM_XCD tile counters (persistent launches)
-  int persist;       // 0: one tile per work group, k: k persistent work groups per CU
   int rows;          // per-pixel stages: rows per thread (tile 64 x 4 rows)
 };
 
@@ -1306,9 +1305,9 @@ static int enqueue(vkdt_batch_t *b, hipStream_t s, int timed)
         if(int e = hip_fail(hipEventRecord(b->ev[k], s), "batch timing")) return e;
       group = g;
     }
-    const int persist = tune_persist(b->tune[g]);
+    const int persist = tune_persist(b->tune[g]);   // work groups per CU, 0: one tile per work group
     const int rows = is_pixel_stage(L.kind) ? tune_rows(b->tune[g]) : 1;
-    bt_launch a = { b->d_img, b->d_job + L.job0, L.njob, L.total, b->d_ctr + L.ctr0, persist, rows };
+    bt_launch a = { b->d_img, b->d_job + L.job0, L.njob, L.total, b->d_ctr + L.ctr0, rows };
     const dim3 grid(persist && L.kind != K_TAIL ? b->ncu * persist : L.total), blk(BX, BY);
     const auto run = [&](auto persistent) {
       constexpr int P = decltype(persistent)::value;
